@@ -21,7 +21,9 @@
 #include <cstdlib>
 
 #include "epm_physics.hpp"
+#include "row_ops.hpp"
 #include "solver.hpp"
+#include "wave_ops.hpp"
 
 namespace uepm {
 
@@ -260,6 +262,187 @@ __global__ __launch_bounds__(256) void apply_q_kernel(const VT* __restrict__ V, 
             }
         }
     }
+}
+
+// ---------------------------------------------------------------------------
+// x = Q z for real reflectors, one wave per k-point and 16 bands.  Lane (g, b),
+// b = lane % 16, holds band b at rows 64 q + 16 g + r in registers x[q][r].  A
+// reflector is one coalesced load of 64 values per q: lane (g, r) then has v at
+// row 64 q + 16 g + r, just where the bands of its 16-lane row need it, so both
+// passes over it (s = v^T x, x -= tau s v) are multiply-adds with a DPP row
+// operand (row_ops.hpp) and only s crosses the four rows of the wave.  No LDS and
+// no barriers; the next reflector's loads are in flight during the current one.
+// Against the per-reflector kernel above (its rows spread over 16 lanes, bands
+// over rows) there is one row sum per reflector and 16 bands instead of one per
+// band group.  Real output (T = double) for the refinement, or the eigenvectors
+// themselves (T = double2) with the gradients: the FP64 form's last stage.
+// waves per SIMD that the registers of a lane allow: x, two reflectors and 44 more
+template <typename R, int NQ>
+constexpr int apply_q_real_waves() {
+    return 512 / ((int)sizeof(R) / 4 * 18 * NQ + 44);
+}
+template <typename R, int NQ, typename T>
+__global__ __launch_bounds__(64, (apply_q_real_waves<R, NQ>())) void apply_q_real_kernel(const R* __restrict__ V, int n, const R* __restrict__ tauall,
+                                                          const double* __restrict__ Z, int nb, T* __restrict__ X,
+                                                          double* __restrict__ grads, DevParams P,
+                                                          const double* __restrict__ kpts,
+                                                          const int32_t* __restrict__ G, const int* __restrict__ kstat,
+                                                          unsigned long long* __restrict__ status, int64_t k0) {
+    const int64_t kk = blockIdx.x;
+    const int lane = threadIdx.x, l16 = lane & 15, g16 = lane & 48;
+    if (status && blockIdx.y == 0 && lane == 0 && kstat[kk]) {
+        atomicAdd(&status[0], 1ull);
+        atomicMin(&status[1], (unsigned long long)(k0 + kk));
+    }
+    const int b = 16 * blockIdx.y + l16;
+    const bool live = b < nb;
+    const R* Vk = V + kk * (int64_t)n * n;
+    const R* tau = tauall + kk * n;
+    const double* z = Z + (kk * nb + (live ? b : nb - 1)) * (int64_t)n;
+
+    R x[NQ][16];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int i = 64 * q + g16 + r;
+            x[q][r] = (R)z[i < n ? i : n - 1] * (live && i < n ? R(1) : R(0));
+        }
+        __builtin_amdgcn_sched_barrier(0);  // a block's loads at a time: more in flight would spill
+    }
+    // v_j at row 64 q + lane: 1 at row j + 1, the stored reflector below, zero above
+    auto vload = [&](int j, int q) -> R { return Vk[min(64 * q + lane, n - 1) + (int64_t)j * n]; };
+    R v[NQ], vn[NQ];
+    R t = 0, tn = 0;
+    if (n >= 2) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) vn[q] = vload(n - 2, q);
+        tn = tau[n - 2];
+    }
+    for (int j = n - 2; j >= 0; --j) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) v[q] = vn[q];
+        t = tn;
+        {
+            const int jn = j > 0 ? j - 1 : 0, qn = (jn + 1) >> 6;  // first block with a row of v_jn
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+                if (q >= qn) vn[q] = vload(jn, q);
+            tn = tau[jn];
+        }
+        const int q0 = (j + 1) >> 6;
+        R acc[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+            if (q >= q0) {
+                const int i = 64 * q + lane;
+                v[q] = i > j + 1 && i < n ? v[q] : i == j + 1 ? R(1) : R(0);
+                rowop::dot16(acc, v[q], x[q]);
+            }
+        // sum over the four rows of the wave: every lane of a band gets it
+        R s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        wave::Words<R> w0(s), w1(s);
+#pragma unroll
+        for (int i = 0; i < wave::Words<R>::n; ++i) wave::swap16(w0.w[i], w1.w[i]);
+        s = w0.value() + w1.value();
+        wave::Words<R> w2(s), w3(s);
+#pragma unroll
+        for (int i = 0; i < wave::Words<R>::n; ++i) wave::swap32(w2.w[i], w3.w[i]);
+        s = w2.value() + w3.value();
+        const R c = -t * s;
+        // opaque, or the compiler threads the first pass's branches into this one:
+        // a copy of the code, and of the registers, per q0
+        int q1 = q0;
+        asm volatile("" : "+s"(q1));
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+            if (q >= q1) rowop::axpy16(x[q], v[q], c);
+    }
+    T* xo = X ? X + (kk * nb + (live ? b : 0)) * (int64_t)n : nullptr;
+    const double* k = kpts + 3 * kk;
+    double sx = 0.0, sy = 0.0, sz = 0.0;
+    // the same values, opaque to the compiler: it would otherwise keep every row's
+    // index and range test from the load above, in registers the reflectors need
+    int ge = g16, ne = n;
+    asm volatile("" : "+v"(ge), "+s"(ne));
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int i = 64 * q + ge + r;
+            if (i < ne) {
+                const double a = (double)x[q][r];
+                if (xo && live) {
+                    if constexpr (sizeof(T) == sizeof(double)) xo[i] = a;
+                    else xo[i] = make_double2(a, a - a);  // imaginary part zero, NaN with a NaN real part
+                }
+                if (grads) {
+                    const double w = a * a;  // Hellmann-Feynman on the kinetic term
+                    sx += (k[0] + (double)G[3 * i]) * w;
+                    sy += (k[1] + (double)G[3 * i + 1]) * w;
+                    sz += (k[2] + (double)G[3 * i + 2]) * w;
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (grads) {
+        for (int o = 16; o < 64; o <<= 1) {
+            sx += __shfl_xor(sx, o, 64);
+            sy += __shfl_xor(sy, o, 64);
+            sz += __shfl_xor(sz, o, 64);
+        }
+        if (live && g16 == 0) {
+            double* gg = grads + 3 * (kk * nb + b);
+            gg[0] = sx * P.grad_pref * P.frac_to_phys;
+            gg[1] = sy * P.grad_pref * P.frac_to_phys;
+            gg[2] = sz * P.grad_pref * P.frac_to_phys;
+        }
+    }
+}
+
+namespace {
+template <typename R, typename T>
+hipError_t apply_q_real(const R* dV, int n, const R* dtau, const double* dZ, int nb, T* dX, double* dgrads,
+                        const DevParams& P, const double* dk, const int32_t* dG, int64_t nk, const int* kstat,
+                        unsigned long long* status, int64_t k0, hipStream_t s) {
+    const dim3 grid((unsigned)nk, (unsigned)((nb + 15) / 16));
+#define UEPM_NQ(q)                                                                                                   \
+    case q:                                                                                                          \
+        hipLaunchKernelGGL((apply_q_real_kernel<R, q, T>), grid, dim3(64), 0, s, dV, n, dtau, dZ, nb, dX, dgrads, P, dk, \
+                           dG, kstat, status, k0);                                                                   \
+        break
+    switch ((n + 63) / 64) {
+        UEPM_NQ(1);
+        UEPM_NQ(2);
+        UEPM_NQ(3);
+        UEPM_NQ(4);
+        UEPM_NQ(5);
+        default:
+            if constexpr (sizeof(R) == sizeof(float)) {
+                switch ((n + 63) / 64) {
+                    UEPM_NQ(6);
+                    UEPM_NQ(7);
+                    default: return hipErrorInvalidValue;
+                }
+                break;
+            }
+            return hipErrorInvalidValue;
+    }
+#undef UEPM_NQ
+    return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_apply_q_real_f32(const float* dV, int n, const float* dtau, const double* dZ, int nb, double* dX,
+                                   int64_t nk, hipStream_t s) {
+    return apply_q_real<float, double>(dV, n, dtau, dZ, nb, dX, nullptr, DevParams{}, nullptr, nullptr, nk, nullptr, nullptr,
+                                       0, s);
+}
+hipError_t launch_apply_q_real_f64(const double* dV, int n, const double* dtau, const double* dZ, int nb, double2* dX,
+                                   double* dgrads, const DevParams& P, const double* dk, const int32_t* dG, int64_t nk,
+                                   const int* kstat, unsigned long long* status, int64_t k0, hipStream_t s) {
+    return apply_q_real<double, double2>(dV, n, dtau, dZ, nb, dX, dgrads, P, dk, dG, nk, kstat, status, k0, s);
 }
 
 // ---------------------------------------------------------------------------

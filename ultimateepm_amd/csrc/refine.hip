@@ -690,6 +690,390 @@ __global__ __launch_bounds__(BS, 2) void refine_mfma2_kernel(const double2* __re
                        reinterpret_cast<double*>(Mm));
 }
 
+// ---------------------------------------------------------------------------
+// The same refinement for a real H(k) (and so real X0, Ritz vectors and small
+// problem): a quarter of the MFMAs, half the bytes.
+
+// The small real symmetric problem on nbr <= LDM Ritz vectors, in one wave, as
+// small_rayleigh_ritz does it: Cholesky S = L L^T, M' = L^-1 M L^-T, round-robin
+// Jacobi M' = Z Theta Z^T, C = L^-T Z (in Wt), Ritz values th and the order perm.
+template <int LDM>
+__device__ bool small_rayleigh_ritz_real(int nbr, double* __restrict__ Ss, double* __restrict__ Mm,
+                                         double* __restrict__ Zm, double* __restrict__ Wt, double* __restrict__ th,
+                                         int* __restrict__ perm, double2* __restrict__ rot, int lane) {
+    const int i = lane;
+    for (int j = 0; j < nbr; ++j) {
+        const double ljj = sqrt(Ss[j * LDM + j]);
+        const double rl = 1.0 / ljj;
+        wsync();
+        if (i > j && i < nbr) Ss[i * LDM + j] *= rl;
+        if (i == 0) Ss[j * LDM + j] = ljj;
+        wsync();
+        for (int e = i; e < LDM * LDM; e += 64) {
+            const int r = e / LDM, c = e % LDM;
+            if (c > j && r >= c && r < nbr) Ss[r * LDM + c] -= Ss[r * LDM + j] * Ss[c * LDM + j];
+        }
+        wsync();
+    }
+    // Wt = L^-1 M (lane = column of M), then U = L^-1 Wt^T (lane = row of Wt): M' = U^T.
+    // Columns stay in registers; a row's terms are subtracted in ascending order.
+    auto lower = [&](double (&v)[LDM]) {
+#pragma unroll
+        for (int r = 0; r < LDM; ++r)
+            if (r < nbr) {
+                double s = v[r];
+#pragma unroll
+                for (int k = 0; k < r; ++k) s = fma(-Ss[r * LDM + k], v[k], s);
+                v[r] = s * (1.0 / Ss[r * LDM + r]);
+            }
+    };
+    if (i < nbr) {
+        double v[LDM];
+#pragma unroll
+        for (int r = 0; r < LDM; ++r) v[r] = r < nbr ? Mm[r * LDM + i] : 0.0;
+        lower(v);
+#pragma unroll
+        for (int r = 0; r < LDM; ++r)
+            if (r < nbr) Wt[r * LDM + i] = v[r];
+    }
+    wsync();
+    if (i < nbr) {
+        double v[LDM];
+#pragma unroll
+        for (int r = 0; r < LDM; ++r) v[r] = r < nbr ? Wt[i * LDM + r] : 0.0;
+        lower(v);
+#pragma unroll
+        for (int c = 0; c < LDM; ++c)
+            if (c < nbr) {
+                Mm[i * LDM + c] = v[c];
+                Zm[i * LDM + c] = i == c ? 1.0 : 0.0;
+            }
+    }
+    wsync();
+    if (i < nbr)
+        for (int c = i + 1; c < nbr; ++c) {  // symmetrise
+            const double h = 0.5 * (Mm[i * LDM + c] + Mm[c * LDM + i]);
+            Mm[i * LDM + c] = h;
+            Mm[c * LDM + i] = h;
+        }
+    wsync();
+    // the rotation test, the rounds and the stopping rules of small_rayleigh_ritz
+    const int m = (nbr + 1) & ~1, half = m >> 1;
+    auto negligible = [&](int p, int q) {
+        const double ac = fabs(Mm[p * LDM + q]);
+        const double a = Mm[p * LDM + p], b = Mm[q * LDM + q];
+        const double scale = fabs(a) + fabs(b) + 1e-300;
+        return ac <= 1e-15 * scale || ac * ac <= 1e-13 * scale * fabs(b - a);
+    };
+    auto all_negligible = [&]() {
+        bool big = false;
+        for (int pq = i; pq < LDM * LDM; pq += 64) {
+            const int p = pq / LDM, q = pq % LDM;
+            if (p < q && q < nbr && !negligible(p, q)) big = true;
+        }
+        return !__any(big);
+    };
+    bool converged = false;
+    for (int sweep = 0; sweep < 20; ++sweep) {
+        if (all_negligible()) {
+            converged = true;
+            break;
+        }
+        bool rotated = false;
+        for (int round = 0; round < m - 1; ++round) {
+            auto elem = [&](int pos) {
+                if (pos == 0) return 0;
+                const int v = pos - 1 + round;  // < 2 (m - 1)
+                return (v >= m - 1 ? v - (m - 1) : v) + 1;
+            };
+            bool did = false;
+            if (i < half) {
+                int p = elem(i), q = elem(m - 1 - i);
+                if (p > q) { const int t = p; p = q; q = t; }
+                double2 g = make_double2(1.0, 0.0);  // cs, sn with the element's sign
+                if (q < nbr && !negligible(p, q)) {
+                    did = true;
+                    const double c = Mm[p * LDM + q];
+                    const double tau_ = (Mm[q * LDM + q] - Mm[p * LDM + p]) / (2.0 * c);
+                    const double t = (tau_ >= 0 ? 1.0 : -1.0) / (fabs(tau_) + sqrt(1.0 + tau_ * tau_));
+                    const double cs = 1.0 / sqrt(1.0 + t * t);
+                    g = make_double2(cs, t * cs);
+                }
+                rot[i] = g;
+            }
+            wsync();
+            if (__any(did)) {
+                rotated = true;
+                // columns: M <- M G, Z <- Z G with G = [[cs, sn], [-sn, cs]] on (p, q)
+                for (int task = i; task < half * LDM; task += 64) {
+                    const int k = task / LDM, row = task % LDM;
+                    if (row >= nbr) continue;
+                    int p = elem(k), q = elem(m - 1 - k);
+                    if (p > q) { const int t = p; p = q; q = t; }
+                    if (q >= nbr) continue;
+                    const double2 g = rot[k];
+                    const double mp = Mm[row * LDM + p], mq = Mm[row * LDM + q];
+                    Mm[row * LDM + p] = mp * g.x - mq * g.y;
+                    Mm[row * LDM + q] = mp * g.y + mq * g.x;
+                    const double zp = Zm[row * LDM + p], zq = Zm[row * LDM + q];
+                    Zm[row * LDM + p] = zp * g.x - zq * g.y;
+                    Zm[row * LDM + q] = zp * g.y + zq * g.x;
+                }
+                wsync();
+                // rows: M <- G^T M
+                for (int task = i; task < half * LDM; task += 64) {
+                    const int k = task / LDM, col = task % LDM;
+                    if (col >= nbr) continue;
+                    int p = elem(k), q = elem(m - 1 - k);
+                    if (p > q) { const int t = p; p = q; q = t; }
+                    if (q >= nbr) continue;
+                    const double2 g = rot[k];
+                    const double rp = Mm[p * LDM + col], rq = Mm[q * LDM + col];
+                    // the rotated pair's own off-diagonal element is zero by construction
+                    const bool own = g.y != 0.0 && (col == p || col == q);
+                    const double np = rp * g.x - rq * g.y, nq = rp * g.y + rq * g.x;
+                    Mm[p * LDM + col] = own && col == q ? 0.0 : np;
+                    Mm[q * LDM + col] = own && col == p ? 0.0 : nq;
+                }
+                wsync();
+            }
+        }
+        if (!rotated) {
+            converged = true;
+            break;
+        }
+    }
+    if (!converged) converged = all_negligible();
+    wsync();
+    // C = L^-T Z (back substitution, lane = column of Z)
+    if (i < nbr) {
+        double v[LDM];
+#pragma unroll
+        for (int r = 0; r < LDM; ++r) v[r] = r < nbr ? Zm[r * LDM + i] : 0.0;
+#pragma unroll
+        for (int r = LDM - 1; r >= 0; --r)
+            if (r < nbr) {
+                double s = v[r];
+#pragma unroll
+                for (int k = r + 1; k < LDM; ++k)
+                    if (k < nbr) s = fma(-Ss[k * LDM + r], v[k], s);
+                v[r] = s * (1.0 / Ss[r * LDM + r]);
+            }
+#pragma unroll
+        for (int r = 0; r < LDM; ++r)
+            if (r < nbr) Wt[r * LDM + i] = v[r];
+        th[i] = Mm[i * LDM + i];
+        perm[i] = i;
+    }
+    wsync();
+    if (i < nbr) {
+        const double ti = th[i];
+        int rank = 0;
+        for (int c = 0; c < nbr; ++c) {
+            const double tc = th[c];
+            rank += (tc < ti || (tc == ti && c < i)) ? 1 : 0;
+        }
+        perm[rank] = i;
+    }
+    wsync();
+    return converged;
+}
+
+// NT = 1: nbr <= 16, per-wave partials of S and M; NT = 2: nbr <= 32 on two 16-band
+// tiles, the waves adding into one slot in turn.  Element layout and phases as in
+// refine_mfma_kernel / refine_mfma2_kernel.
+template <int BS, int NT>
+__global__ __launch_bounds__(BS, NT == 1 ? 4 : 3) void refine_real_kernel(
+    const double* __restrict__ H, int n, const double* __restrict__ Xall, int nbr, int nb, double* __restrict__ evals,
+    double2* __restrict__ evecs, double* __restrict__ grads, DevParams P, const double* __restrict__ kpts,
+    const int32_t* __restrict__ G, const int* __restrict__ kstat, unsigned long long* __restrict__ status, int64_t k0) {
+    constexpr int NW = BS / 64, LDM = 16 * NT, NQ = NT * NT;
+    constexpr int KU = NT == 1 ? 16 : 8;  // column quads loaded ahead of their MFMAs
+    __shared__ __align__(16) double part[NT == 1 ? NW : NQ][2][16][16];
+    __shared__ double Mm[LDM * LDM], Ss[LDM * LDM];
+    static_assert(sizeof(part) >= 2 * LDM * LDM * sizeof(double), "Z and W fit in the partial slots");
+    double* Zm = &part[0][0][0][0];
+    double* Wt = Zm + LDM * LDM;
+    __shared__ double th[LDM];
+    __shared__ int perm[LDM];
+    __shared__ double2 rot[LDM / 2 + 1];
+    __shared__ double red[3 * 8 * NW];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int l16 = lane & 15, l4 = lane >> 4;
+    const int64_t kk = blockIdx.x;
+    const double* A = H + kk * (int64_t)n * n;
+    const double* X = Xall + kk * (int64_t)nbr * n;  // X[b * n + r]
+    double bm[NT];  // 1 for a live band, 0 past nbr
+    const double* Xb[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const bool live = 16 * t + l16 < nbr;
+        bm[t] = live ? 1.0 : 0.0;
+        Xb[t] = X + (live ? 16 * t + l16 : 0) * (int64_t)n;
+    }
+    dbl4 sa[NQ], ma[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) sa[q] = ma[q] = dbl4{0, 0, 0, 0};
+    const int ntile = (n + 15) >> 4;
+    for (int t = wv; t < ntile; t += NW) {
+        const int row = 16 * t + l16;
+        const double* Ar = A + (row < n ? row : n - 1);
+        const double mrow = row < n ? 1.0 : 0.0;
+        dbl4 y[NT];
+#pragma unroll
+        for (int bt = 0; bt < NT; ++bt) y[bt] = dbl4{0, 0, 0, 0};
+        for (int c0 = 0; c0 < n; c0 += 4 * KU) {
+            double h[KU], x[KU][NT];
+#pragma unroll
+            for (int u = 0; u < KU; ++u) {
+                const int col = c0 + 4 * u + l4, cc = col < n ? col : n - 1;
+                const double mc = col < n ? 1.0 : 0.0;
+                h[u] = Ar[(int64_t)cc * n] * (mrow * mc);
+#pragma unroll
+                for (int bt = 0; bt < NT; ++bt) x[u][bt] = Xb[bt][cc] * (bm[bt] * mc);
+            }
+#pragma unroll
+            for (int u = 0; u < KU; ++u)
+#pragma unroll
+                for (int bt = 0; bt < NT; ++bt) y[bt] = mfma64(h[u], x[u][bt], y[bt]);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = 16 * t + 4 * v + l4;
+            double x[NT];
+#pragma unroll
+            for (int bt = 0; bt < NT; ++bt) x[bt] = Xb[bt][r < n ? r : n - 1] * (r < n ? bm[bt] : 0.0);
+#pragma unroll
+            for (int at = 0; at < NT; ++at)
+#pragma unroll
+                for (int bt = 0; bt < NT; ++bt) {
+                    sa[NT * at + bt] = mfma64(x[at], x[bt], sa[NT * at + bt]);
+                    ma[NT * at + bt] = mfma64(x[at], y[bt][v], ma[NT * at + bt]);
+                }
+        }
+    }
+    if constexpr (NT == 1) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            part[wv][0][4 * v + l4][l16] = sa[0][v];
+            part[wv][1][4 * v + l4][l16] = ma[0][v];
+        }
+        __syncthreads();
+        static_assert(BS == 256, "one (a, b) entry of S and M per thread");
+        const int a = tid >> 4, b = tid & 15;
+        double s = 0, m = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            s += part[w][0][a][b];
+            m += part[w][1][a][b];
+        }
+        if (a < nbr && b < nbr) {
+            Ss[a * LDM + b] = s;
+            Mm[a * LDM + b] = m;
+        }
+    } else {
+        for (int rd = 0; rd < NW; ++rd) {
+            if (wv == rd) {
+#pragma unroll
+                for (int q = 0; q < NQ; ++q)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        double& ds = part[q][0][4 * v + l4][l16];
+                        double& dm = part[q][1][4 * v + l4][l16];
+                        ds = rd == 0 ? sa[q][v] : ds + sa[q][v];
+                        dm = rd == 0 ? ma[q][v] : dm + ma[q][v];
+                    }
+            }
+            __syncthreads();
+        }
+        for (int e = tid; e < NQ * 256; e += BS) {
+            const int q = e >> 8, a = (e >> 4) & 15, b = e & 15;
+            const int ga = 16 * (q / NT) + a, gb = 16 * (q % NT) + b;
+            if (ga < nbr && gb < nbr) {
+                Ss[ga * LDM + gb] = part[q][0][a][b];
+                Mm[ga * LDM + gb] = part[q][1][a][b];
+            }
+        }
+    }
+    __syncthreads();  // the partial slots are free from here: Z and W take their place
+    if (wv == 0) {
+        const bool conv = small_rayleigh_ritz_real<LDM>(nbr, Ss, Mm, Zm, Wt, th, perm, rot, lane);
+        report_ritz_status(kstat, status, k0, kk, nb, th, perm, conv, lane);
+    }
+    __syncthreads();
+    // X1 = X0 C[:, perm[b]], eight bands a pass, one thread per row (write_ritz)
+    if (tid < nb) evals[kk * nb + tid] = th[perm[tid]];
+    if (!evecs && !grads) return;
+    constexpr int BC = 8;
+    double2* out = evecs ? evecs + kk * (int64_t)nb * n : nullptr;
+    const double* k = kpts + 3 * kk;
+    for (int b0 = 0; b0 < nb; b0 += BC) {
+        double gx[BC], gy[BC], gz[BC];
+#pragma unroll
+        for (int u = 0; u < BC; ++u) gx[u] = gy[u] = gz[u] = 0.0;
+        for (int r = tid; r < n; r += BS) {
+            double acc[BC];
+#pragma unroll
+            for (int u = 0; u < BC; ++u) acc[u] = 0.0;
+            for (int a = 0; a < nbr; ++a) {
+                const double x = X[a * n + r];
+#pragma unroll
+                for (int u = 0; u < BC; ++u)
+                    if (b0 + u < nb) acc[u] = fma(x, Wt[a * LDM + perm[b0 + u]], acc[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < BC; ++u)
+                if (b0 + u < nb) {
+                    // imaginary part zero, NaN with a NaN real part
+                    if (out) out[(int64_t)(b0 + u) * n + r] = make_double2(acc[u], acc[u] - acc[u]);
+                    if (grads) {
+                        const double wt = acc[u] * acc[u];  // Hellmann-Feynman, kinetic term
+                        gx[u] += (k[0] + (double)G[3 * r]) * wt;
+                        gy[u] += (k[1] + (double)G[3 * r + 1]) * wt;
+                        gz[u] += (k[2] + (double)G[3 * r + 2]) * wt;
+                    }
+                }
+        }
+        if (grads) {
+#pragma unroll
+            for (int u = 0; u < BC; ++u)
+                for (int o = 32; o > 0; o >>= 1) {
+                    gx[u] += __shfl_xor(gx[u], o, 64);
+                    gy[u] += __shfl_xor(gy[u], o, 64);
+                    gz[u] += __shfl_xor(gz[u], o, 64);
+                }
+            if (lane == 0)
+#pragma unroll
+                for (int u = 0; u < BC; ++u) {
+                    red[(wv * BC + u) * 3 + 0] = gx[u];
+                    red[(wv * BC + u) * 3 + 1] = gy[u];
+                    red[(wv * BC + u) * 3 + 2] = gz[u];
+                }
+            __syncthreads();
+            if (tid < 3 * BC && b0 + tid / 3 < nb) {
+                double sum = 0.0;
+#pragma unroll
+                for (int w = 0; w < NW; ++w) sum += red[(w * BC + tid / 3) * 3 + tid % 3];
+                grads[3 * (kk * nb + b0 + tid / 3) + tid % 3] = sum * P.grad_pref * P.frac_to_phys;
+            }
+            __syncthreads();
+        }
+    }
+}
+
+hipError_t launch_refine_real(const double* dH, int n, const double* dX, int nbr, int nb, double* devals, double2* devecs,
+                              double* dgrads, const DevParams& P, const double* dk, const int32_t* dG, int64_t nk,
+                              const int* kstat, unsigned long long* status, int64_t k0, hipStream_t s) {
+    if (nbr > kNbrMax || nb > nbr) return hipErrorInvalidValue;
+    if (nbr <= 16)
+        hipLaunchKernelGGL((refine_real_kernel<kRefBS, 1>), dim3((unsigned)nk), dim3(kRefBS), 0, s, dH, n, dX, nbr, nb,
+                           devals, devecs, dgrads, P, dk, dG, kstat, status, k0);
+    else
+        hipLaunchKernelGGL((refine_real_kernel<kRefBS, 2>), dim3((unsigned)nk), dim3(kRefBS), 0, s, dH, n, dX, nbr, nb,
+                           devals, devecs, dgrads, P, dk, dG, kstat, status, k0);
+    return hipGetLastError();
+}
+
 const char* refine_kernel_name(int nbr) { return nbr <= 16 ? "refine_mfma_kernel" : "refine_mfma2_kernel"; }
 
 hipError_t launch_refine(const double2* dH, int n, int ld, double2* dX, int nbr, int nb, double* devals,

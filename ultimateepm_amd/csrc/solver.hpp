@@ -32,6 +32,9 @@ hipError_t launch_tridiag_blocked_c64(const TriPlan& tp, const double2* dH, int 
 
 hipError_t launch_assemble(const DevParams& P, const int32_t* dG, const double* dk, int64_t nk, double2* dH, int ld,
                            hipStream_t s);
+// The real parts alone (nk x n x n doubles), for a plan whose H(k) is real.
+hipError_t launch_assemble_real(const DevParams& P, const int32_t* dG, const double* dk, int64_t nk, double* dH, int ld,
+                                hipStream_t s);
 // Failure reporting.  A solve's device status is two words: the number of
 // k-points whose eigen-solve failed and the lowest index among them (all ones
 // when none); launch_status_reset clears it.  Inside a chunk, kstat (one int
@@ -55,6 +58,11 @@ hipError_t launch_tri_eig(const double* dd, const double* de, int n, int nb, int
 hipError_t launch_refine(const double2* dH, int n, int ld, double2* dX, int nbr, int nb, double* devals,
                          double2* devecs, double* dgrads, const DevParams& P, const double* dk, const int32_t* dG,
                          int64_t nk, const int* kstat, unsigned long long* status, int64_t k0, hipStream_t s);
+
+// launch_refine for a real H (nk x n x n) and real X (nk x nbr x n, read only).
+hipError_t launch_refine_real(const double* dH, int n, const double* dX, int nbr, int nb, double* devals, double2* devecs,
+                              double* dgrads, const DevParams& P, const double* dk, const int32_t* dG, int64_t nk,
+                              const int* kstat, unsigned long long* status, int64_t k0, hipStream_t s);
 
 // Name of the refinement kernel launch_refine runs for nbr Ritz vectors.
 const char* refine_kernel_name(int nbr);
@@ -91,6 +99,17 @@ hipError_t launch_tridiag_reg_c128(const double2* H, int64_t hk, int m, int ld, 
                                    double2* V, int ldv, int64_t vk, double* dd, double* de, double2* dtau, int64_t dk,
                                    double2* work, hipStream_t s);
 
+// The reduction of a real symmetric H (n x n doubles per k-point, both triangles)
+// in FP32 or FP64, n <= tridiag_real_max_n(f32): outputs as launch_tridiag_reg_c64,
+// reflectors and tau real (V column-major, leading dimension n); `work` provides
+// tridiag_real_work_bytes(n, f32) per k-point.
+int tridiag_real_max_n(bool f32);
+size_t tridiag_real_work_bytes(int n, bool f32);
+hipError_t launch_tridiag_real_f32(const double* dH, int n, int64_t nk, float* V, double* dd, double* de, float* dtau,
+                                   float* work, hipStream_t s);
+hipError_t launch_tridiag_real_f64(const double* dH, int n, int64_t nk, double* V, double* dd, double* de, double* dtau,
+                                   double* work, hipStream_t s);
+
 // Eigenvectors of H from those of T: cluster re-orthogonalisation of Z
 // ([k][band][row], n x nb per k), then x = Q z with the reflectors of the
 // reduction (FP64: over H; precision form: complex64 Vout), gradients when dgrads.
@@ -113,6 +132,14 @@ hipError_t launch_apply_q_c64(const float2* dV, int n, int ld, const float2* dta
                               double2* dX, const DevParams& P, const double* dk, const int32_t* dG, int64_t nk,
                               int bands_per_group, int lds_limit, hipStream_t s);
 bool apply_q_wy_fits(int n, int nb, int lds_limit);
+// x = Q z with real reflectors (n <= tridiag_real_max_n): the real Ritz basis of the
+// precision form, or the FP64 form's eigenvectors (dX null: not wanted) and
+// gradients (its last stage: adds the k-points kstat flags to status).
+hipError_t launch_apply_q_real_f32(const float* dV, int n, const float* dtau, const double* dZ, int nb, double* dX,
+                                   int64_t nk, hipStream_t s);
+hipError_t launch_apply_q_real_f64(const double* dV, int n, const double* dtau, const double* dZ, int nb, double2* dX,
+                                   double* dgrads, const DevParams& P, const double* dk, const int32_t* dG, int64_t nk,
+                                   const int* kstat, unsigned long long* status, int64_t k0, hipStream_t s);
 
 // Device-to-device copy (16-byte aligned pointers take the vector path).
 hipError_t launch_copy_bytes(void* dst, const void* src, uint64_t bytes, int num_cus, hipStream_t s);

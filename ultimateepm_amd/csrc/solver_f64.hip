@@ -17,6 +17,7 @@
 #include <cfloat>
 #include <cstdint>
 #include <cstdlib>
+#include <type_traits>
 
 #include "epm_physics.hpp"
 #include "solver.hpp"
@@ -151,26 +152,29 @@ __global__ __launch_bounds__(BS) void assemble_kernel(DevParams P, const int32_t
 // transpose above the diagonal, so both halves go out in 256-byte column
 // runs (the mirrored writes of assemble_kernel are one element per column).
 // Element values are assemble_kernel's, bit for bit.
-template <int BS>
+// T = double: only the real parts, for plans whose H(k) is real (the imaginary
+// parts are exactly zero there): half the bytes of the complex matrix.
+template <int BS, typename T>
 __global__ __launch_bounds__(BS) void assemble_tiled_kernel(DevParams P, const int32_t* __restrict__ G,
-                                                             const double* __restrict__ kpts,
-                                                             double2* __restrict__ H, int ld) {
+                                                             const double* __restrict__ kpts, T* __restrict__ H,
+                                                             int ld) {
+    constexpr bool kReal = std::is_same_v<T, double>;
     extern __shared__ __align__(16) unsigned char smem[];
     KState* ks = reinterpret_cast<KState*>(smem);
     __shared__ double2 vtab[kVPhaseTab];
-    __shared__ double2 T[BS / 64][16][17];
+    __shared__ T Tt[BS / 64][16][17];
     const int kk = blockIdx.x;
     const double* k = kpts + 3 * (size_t)kk;
     const int N = P.N;
     for (int i = threadIdx.x; i < N; i += BS) kstate_init(P, k, G, i, ks[i]);
     for (int t = threadIdx.x; t < kVPhaseTab; t += BS) vtab[t] = local_phase(P, t / 49 - 3, (t / 7) % 7 - 3, t % 7 - 3);
     __syncthreads();
-    double2* A = H + (size_t)kk * ld * P.dim;
+    T* A = H + (size_t)kk * ld * P.dim;
     const bool swap_exact = !(P.well != 0 && (P.need_l2_a || P.need_l2_c));
     const int nt = (N + 15) >> 4, ntiles = nt * (nt + 1) / 2;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int il = lane & 15, jq = lane >> 4;
-    double2(*Tw)[17] = T[wv];
+    T(*Tw)[17] = Tt[wv];
     for (int tile = wv; tile < ntiles; tile += BS / 64) {
         // tile -> (bi, bj), column-major over the lower triangle of tiles
         int bj = 0, rem = tile;
@@ -190,9 +194,14 @@ __global__ __launch_bounds__(BS) void assemble_tiled_kernel(DevParams P, const i
                 double re_ij, im_ij, re_ji, im_ji;
                 pair_terms(P, si, sj, gx, gy, gz, i == j, vtab, swap_exact, re_ij, im_ij, re_ji, im_ji);
                 const double hr = 0.5 * (re_ij + re_ji), hi = 0.5 * (im_ij - im_ji);
-                // the diagonal as assemble_kernel's mirrored write leaves it
-                A[i + (size_t)j * ld] = make_double2(hr, i == j ? -hi : hi);
-                Tw[jl][il] = make_double2(hr, hi);
+                if constexpr (kReal) {
+                    A[i + (size_t)j * ld] = hr;
+                    Tw[jl][il] = hr;
+                } else {
+                    // the diagonal as assemble_kernel's mirrored write leaves it
+                    A[i + (size_t)j * ld] = make_double2(hr, i == j ? -hi : hi);
+                    Tw[jl][il] = make_double2(hr, hi);
+                }
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -202,8 +211,9 @@ __global__ __launch_bounds__(BS) void assemble_tiled_kernel(DevParams P, const i
             const int rl = il, cl = jq + 4 * q;
             const int row = 16 * bj + rl, col = 16 * bi + cl;
             if (row < N && col < N && row < col) {
-                const double2 h = Tw[rl][cl];  // h(col, row)
-                A[row + (size_t)col * ld] = make_double2(h.x, -h.y);
+                const T h = Tw[rl][cl];  // h(col, row)
+                if constexpr (kReal) A[row + (size_t)col * ld] = h;
+                else A[row + (size_t)col * ld] = make_double2(h.x, -h.y);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -517,20 +527,35 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
 // ------------------------------------------------------------ launchers
 constexpr int kAsmBS = 256;
 
-hipError_t launch_assemble(const DevParams& P, const int32_t* dG, const double* dk, int64_t nk, double2* dH, int ld,
-                           hipStream_t s) {
+namespace {
+template <typename K, typename T>
+hipError_t launch_assemble_kernel(K kern, size_t fixed, const DevParams& P, const int32_t* dG, const double* dk,
+                                  int64_t nk, T* dH, int ld, hipStream_t s) {
     // one KState per basis vector in LDS beside the phase table (and the tiled
     // kernel's transpose slots): up to 766 vectors (860 with spin-orbit) in
     // the 160 KB of a CU
     const size_t shm = sizeof(KState) * (size_t)P.N;
-    const bool tiled = !P.soc;
-    const size_t fixed = sizeof(double2) * kVPhaseTab + (tiled ? sizeof(double2) * (kAsmBS / 64) * 16 * 17 : 0);
     if (shm + fixed > 163840) return hipErrorInvalidValue;
-    auto kern = tiled ? assemble_tiled_kernel<kAsmBS> : assemble_kernel<kAsmBS>;
     hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(kern, dim3((unsigned)nk), dim3(kAsmBS), shm, s, P, dG, dk, dH, ld);
     return hipGetLastError();
+}
+constexpr size_t kAsmTab = sizeof(double2) * kVPhaseTab, kAsmSlots = (kAsmBS / 64) * 16 * 17;
+}  // namespace
+
+hipError_t launch_assemble(const DevParams& P, const int32_t* dG, const double* dk, int64_t nk, double2* dH, int ld,
+                           hipStream_t s) {
+    if (P.soc) return launch_assemble_kernel(assemble_kernel<kAsmBS>, kAsmTab, P, dG, dk, nk, dH, ld, s);
+    return launch_assemble_kernel(assemble_tiled_kernel<kAsmBS, double2>, kAsmTab + kAsmSlots * sizeof(double2), P, dG, dk,
+                                  nk, dH, ld, s);
+}
+
+hipError_t launch_assemble_real(const DevParams& P, const int32_t* dG, const double* dk, int64_t nk, double* dH, int ld,
+                                hipStream_t s) {
+    if (P.soc) return hipErrorInvalidValue;
+    return launch_assemble_kernel(assemble_tiled_kernel<kAsmBS, double>, kAsmTab + kAsmSlots * sizeof(double), P, dG, dk, nk,
+                                  dH, ld, s);
 }
 
 hipError_t launch_tri_eig(const double* dd, const double* de, int n, int nb, int64_t nk, double* devals, double* dZ,
