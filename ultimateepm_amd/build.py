@@ -26,8 +26,8 @@ CXX = os.environ.get("CXX", "g++")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
-DEVICE_SOURCES = ["solver_f64.hip", "tridiag_blocked.hip", "refine.hip", "copy.hip", "tridiag_reg.hip", "tridiag_real.hip", "backtransform.hip",
-                  "tetra_dos.hip", "dielectric.hip", "noalloc.hip"]
+DEVICE_SOURCES = ["assemble.hip", "solver_f64.hip", "tridiag_blocked.hip", "refine.hip", "copy.hip", "tridiag_reg.hip",
+                  "tridiag_real.hip", "backtransform.hip", "tetra_dos.hip", "dielectric.hip", "noalloc.hip"]
 HOST_SOURCES = ["uepm_abi.cpp", "runtime.cpp", "msh_io.cpp", "bzmesh.cpp", "dielectric.cpp"]
 COMMON = ["-O3", "-fPIC", "-std=c++17", f"-I{INCLUDE}", f"-I{CSRC}"]
 DEVICE_FLAGS = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -36,7 +36,11 @@ DEVICE_FLAGS = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang
 
 # Per-file device flags.  refine.hip: MFMA accumulators in VGPRs (the default
 # heuristic shuttles them through AGPRs on every pass of the H X loop).
-FILE_FLAGS = {"refine.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+# assemble.hip: no machine-level hoisting out of loops, which would keep every
+# FP64 polynomial constant of the element loop in vector registers (156 -> 113,
+# four waves per SIMD instead of three).
+FILE_FLAGS = {"refine.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+              "assemble.hip": ["-mllvm", "-disable-machine-licm"]}
 
 
 def _run(cmd):

@@ -15,9 +15,11 @@
 // the Bessel functions: those are evaluated here in closed form (with power
 // series where the closed form cancels) instead of libstdc++'s
 // std::cyl_bessel_j(l + 1/2, x), which the reference calls per element.  The
-// one rearrangement is the non-local phase exp(2 pi i (tau/a) . (K_i - K_j)),
-// formed as exp(i theta_i) exp(-i theta_j) from per-vector values (a few ulp,
-// the size of the rounding of K_i - K_j itself).
+// rearrangements, each worth a few ulp of its term: the non-local phase
+// exp(2 pi i (tau/a) . (K_i - K_j)) and the spin-orbit phase are products of
+// per-vector ones, so is exp(-(K_i^2 + K_j^2) R^2 / 4) of a gaussian well,
+// divisions by |K_i| |K_j| and |K_i|^2 - |K_j|^2 are products with reciprocals,
+// and each element is formed hermitised at once.
 //
 // The per-basis-vector quantities (|K_i|, j_l(|K_i| R), SOC radial factors)
 // are k-dependent but element-independent, so they are computed once per
@@ -42,6 +44,7 @@ struct DevParams {
     int32_t need_l2_a, need_l2_c;  // A2 != 0
     int32_t period_a, period_c;    // SOC radial-factor periods
     int32_t same_r0;    // need_l0_a && need_l0_c && R0_a == R0_c
+    int32_t same_r2;    // need_l2_a && need_l2_c && R2_a == R2_c
     double a;           // lattice constant [m]
     double tau;         // a / 8 [m]
     double tpa;         // 2 pi / a
@@ -55,6 +58,13 @@ struct DevParams {
     double tau_over_a;  // (a / 8) / a
     double alpha0_a, dfbeta_a, A2_a, R0_a, R2_a, gpre_a;  // dfbeta = diag_factor * beta_0
     double alpha0_c, dfbeta_c, A2_c, R0_c, R2_c, gpre_c;  // gpre = 5 pi^1.5 R2^3 / Omega
+    // products the element loop would otherwise keep in vector registers (a double
+    // that every lane shares is a scalar operand only if the host forms it)
+    double w2_a, w2_c;                      // l = 2: V_pre A2 5 (square well), gpre A2 (gaussian)
+    double h2_a, h2_c;                      // R2^2 / 2 (gaussian)
+    struct Radius {
+        double R2, R3_2, R3_3;              // R^2, R^3 / 2, and for l = 0 R^3 / 3 (else 0)
+    } r0_a, r0_c, r2_a, r2_c;
     // spin-orbit
     double soc_kfac;    // (2 pi) / a
     double xi_a, xi_c;  // radial extents
@@ -104,55 +114,23 @@ __device__ __forceinline__ double sph_j(int l, double x) {
     }
 }
 
-// bessel_func.hpp:47-52
+// Modified spherical Bessel function i_2(x), x >= 0 (bessel_func.hpp:47-52:
+// ((x^2 + 3) sinh x - 3 x cosh x) / x^3).  That difference cancels like x^5
+// below x = 2; the ascending series (DLMF 10.53.3) does not, and costs no
+// exponential.  Above, sinh and cosh come from one exponential.
 __device__ __forceinline__ double mod_i2(double x) {
-    if (x == 0.0) return 0.0;
-    return ((x * x + 3) * sinh(x) - 3 * x * cosh(x)) / (x * x * x);
-}
-
-// Per-(k, i) quantities for the radial integrals of one radius R:
-// jm = j_{l-1}(|K| R), j0 = j_l(|K| R), jp = j_{l+1}(|K| R).
-struct BesselTriple {
-    double jm, j0, jp;
-};
-
-__device__ __forceinline__ BesselTriple bessel_triple(int l, double nK, double R) {
-    const double x = nK * R;
-    return {sph_j(l - 1, x), sph_j(l, x), sph_j(l + 1, x)};
-}
-
-// F_l_function (Material.cpp:87-109) from precomputed Bessel triples.
-__device__ __forceinline__ double F_l(double n1, double n2, double R, int l, const BesselTriple& b1,
-                                      const BesselTriple& b2) {
-    constexpr double EPSILON = 1.0e-4;
-    if (fabs(n1 - n2) > EPSILON) {
-        const double pre = (R * R) / (n1 * n1 - n2 * n2);
-        const double F = n1 * b1.jp * b2.j0 - n2 * b2.jp * b1.j0;
-        return pre * F;
-    } else if (n1 > EPSILON) {
-        const double pre = (R * R * R) / (2.0);
-        const double F = b1.j0 * b1.j0 - b1.jm * b1.jp;
-        return pre * F;
+    const double x2 = x * x;
+    if (x < 2.0) {
+        // x^2 / 15 sum_k prod_{i <= k} x^2 / (2 i (2 i + 5)); at x = 2 the thirteenth term is below 1e-17
+        double s = 1.0;
+#pragma unroll
+        for (int k = 12; k >= 1; --k) s = fma(s, x2 * (1.0 / (double)(2 * k * (2 * k + 5))), 1.0);
+        return x2 * (1.0 / 15.0) * s;
     }
-    return (l == 0) ? (R * R * R) / (3.0) : 0.0;
+    const double e = exp(x), m = 1.0 / e;
+    const double sh = 0.5 * (e - m), ch = 0.5 * (e + m);
+    return ((x2 + 3) * sh - 3 * x * ch) / (x2 * x);
 }
-
-// F_2_function_gaussian (Material.cpp:111-116)
-__device__ __forceinline__ double F_2_gauss(double n1, double n2, double R) {
-    const double arg = 0.5 * (R * R) * n1 * n2;
-    return mod_i2(arg) * exp(-0.25 * (n1 * n1 + n2 * n2) * R * R);
-}
-
-// Per-basis-vector state of one k-point.
-struct KState {
-    double kx, ky, kz;   // k + G_i, reduced
-    double Kx, Ky, Kz;   // (k + G_i) * 2 pi / a
-    double nK;           // |K|
-    BesselTriple b0a, b0c, b2a, b2c;  // l = 0 / l = 2 triples at R0 / R2 of anion / cation
-    double Ba, Bc;       // SOC radial factors B(|K|) of anion / cation
-    double pc, ps;       // cos / sin of 2 pi (tau/a) (kx + ky + kz): the non-local phase of a
-                         // pair (i, j) is exp(i (theta_i - theta_j))
-};
 
 // SpinOrbitFunctional.cpp:20-49 (period 2, 3, 4; others rejected on the host)
 __device__ __forceinline__ double soc_radial(int period, double Klen, double bohr, double xi) {
@@ -163,32 +141,94 @@ __device__ __forceinline__ double soc_radial(int period, double Klen, double boh
     return (5.0 - 3.0 * kappa * kappa) / (5.0 * (q * q * q * q * q));
 }
 
-__device__ __forceinline__ void kstate_init(const DevParams& P, const double* k, const int32_t* G, int i, KState& s) {
-    s.kx = k[0] + (double)G[3 * i];
-    s.ky = k[1] + (double)G[3 * i + 1];
-    s.kz = k[2] + (double)G[3 * i + 2];
-    s.Kx = s.kx * P.fourier;
-    s.Ky = s.ky * P.fourier;
-    s.Kz = s.kz * P.fourier;
-    s.nK = sqrt(s.Kx * s.Kx + s.Ky * s.Ky + s.Kz * s.Kz);
+// Per-basis-vector state of one k-point, in LDS as arrays of N doubles (lanes
+// of consecutive vectors then read consecutive words), with only the arrays
+// that the plan's terms use: the fewer bytes per k-point, the more k-points a
+// CU assembles at once.  Offsets in arrays; a radial integral takes three:
+//   j_l(x), j_{l+1}(x) and, for equal norms, j_l^2 - j_{l-1} j_{l+1}, x = |K| R
+// (a gaussian l = 2 well one: exp(-(|K| R)^2 / 4)).
+struct VecLayout {
+    int32_t k = 0;                    // k + G, reduced: 3 arrays
+    int32_t nK = 0;                   // |K|
+    int32_t ph = 0;                   // cos, sin of theta = 2 pi (tau/a) sum_c (k + G)_c
+    int32_t ik = 0;                   // 1 / |k + G|
+    int32_t l0a = 0, l0c = 0, l2a = 0, l2c = 0;  // radial integrals (cation: the anion's when the radii are equal)
+    int32_t B = 0;                    // spin-orbit radial factors of anion and cation
+    int32_t q = 0;                    // cos, sin of the spin-orbit phase of G
+    int32_t count = 0;                // arrays in all (and one int32 per vector after them: G, packed)
+};
+__host__ __device__ inline VecLayout vec_layout(const DevParams& P) {
+    VecLayout L;
+    int n = 0;
+    L.k = n; n += 3;
     if (P.nl) {
-        sincos(2.0 * 3.14159265358979323846 *
-                   (P.tau_over_a * s.kx + P.tau_over_a * s.ky + P.tau_over_a * s.kz),
-               &s.ps, &s.pc);
-        if (P.need_l0_a) s.b0a = bessel_triple(0, s.nK, P.R0_a);
-        if (P.need_l0_c) s.b0c = P.same_r0 ? s.b0a : bessel_triple(0, s.nK, P.R0_c);
+        const int l2 = P.well == 0 ? 3 : 1;
+        L.nK = n; n += 1;
+        L.ph = n; n += 2;
+        if (P.need_l2_a || P.need_l2_c) { L.ik = n; n += 1; }
+        if (P.need_l0_a) { L.l0a = n; n += 3; }
+        if (P.need_l0_c) { L.l0c = P.same_r0 ? L.l0a : n; n += P.same_r0 ? 0 : 3; }
+        if (P.need_l2_a) { L.l2a = n; n += l2; }
+        if (P.need_l2_c) { L.l2c = P.same_r2 ? L.l2a : n; n += P.same_r2 ? 0 : l2; }
+    }
+    if (P.soc) {
+        L.B = n; n += 2;
+        L.q = n; n += 2;
+    }
+    L.count = n;
+    return L;
+}
+__host__ __device__ inline size_t vec_bytes(const DevParams& P) {
+    return (sizeof(double) * (size_t)vec_layout(P).count + sizeof(int32_t)) * (size_t)P.N;
+}
+
+// G of a basis vector in one word: three components biased by 512
+__device__ __forceinline__ int32_t pack_g(int x, int y, int z) { return (x + 512) | (y + 512) << 10 | (z + 512) << 20; }
+
+__device__ __forceinline__ void radial_init(int l, double nK, double R, double* S, int N, int i) {
+    const double x = nK * R;
+    const double jm = sph_j(l - 1, x), j0 = sph_j(l, x), jp = sph_j(l + 1, x);
+    S[i] = j0;
+    S[N + i] = jp;
+    S[2 * N + i] = j0 * j0 - jm * jp;
+}
+
+__device__ __forceinline__ void vector_init(const DevParams& P, const VecLayout& L, const double* k, const int32_t* G,
+                                            int i, double* S, int32_t* Gp) {
+    const int N = P.N;
+    const int gx = G[3 * i], gy = G[3 * i + 1], gz = G[3 * i + 2];
+    const double kx = k[0] + (double)gx, ky = k[1] + (double)gy, kz = k[2] + (double)gz;
+    Gp[i] = pack_g(gx, gy, gz);
+    S[L.k * N + i] = kx;
+    S[(L.k + 1) * N + i] = ky;
+    S[(L.k + 2) * N + i] = kz;
+    const double Kx = kx * P.fourier, Ky = ky * P.fourier, Kz = kz * P.fourier;
+    const double nK = sqrt(Kx * Kx + Ky * Ky + Kz * Kz);
+    if (P.nl) {
+        S[L.nK * N + i] = nK;
+        double s, c;
+        sincos(2.0 * 3.14159265358979323846 * (P.tau_over_a * kx + P.tau_over_a * ky + P.tau_over_a * kz), &s, &c);
+        S[L.ph * N + i] = c;
+        S[(L.ph + 1) * N + i] = s;
+        if (P.need_l2_a || P.need_l2_c) S[L.ik * N + i] = P.fourier / nK;
+        if (P.need_l0_a) radial_init(0, nK, P.R0_a, S + L.l0a * N, N, i);
+        if (P.need_l0_c && !P.same_r0) radial_init(0, nK, P.R0_c, S + L.l0c * N, N, i);
         if (P.well == 0) {
-            if (P.need_l2_a) s.b2a = bessel_triple(2, s.nK, P.R2_a);
-            if (P.need_l2_c) s.b2c = bessel_triple(2, s.nK, P.R2_c);
+            if (P.need_l2_a) radial_init(2, nK, P.R2_a, S + L.l2a * N, N, i);
+            if (P.need_l2_c && !P.same_r2) radial_init(2, nK, P.R2_c, S + L.l2c * N, N, i);
+        } else {
+            if (P.need_l2_a) S[L.l2a * N + i] = exp(-0.25 * (nK * nK) * (P.R2_a * P.R2_a));
+            if (P.need_l2_c && !P.same_r2) S[L.l2c * N + i] = exp(-0.25 * (nK * nK) * (P.R2_c * P.R2_c));
         }
     }
     if (P.soc) {
-        // Kphys = kfac * K (SpinOrbitFunctional.cpp:109-110): same product as Kx above
-        // because soc_kfac == fourier (both (2 pi) / a).
-        const double px = s.kx * P.soc_kfac, py = s.ky * P.soc_kfac, pz = s.kz * P.soc_kfac;
-        const double L = sqrt(px * px + py * py + pz * pz);
-        s.Ba = soc_radial(P.period_a, L, P.bohr, P.xi_a);
-        s.Bc = soc_radial(P.period_c, L, P.bohr, P.xi_c);
+        // Kphys = kfac * K (SpinOrbitFunctional.cpp:109-110) is K above: soc_kfac == fourier
+        S[L.B * N + i] = soc_radial(P.period_a, nK, P.bohr, P.xi_a);
+        S[(L.B + 1) * N + i] = soc_radial(P.period_c, nK, P.bohr, P.xi_c);
+        double s, c;
+        sincos(P.soc_kfac * (P.tau * (double)gx + P.tau * (double)gy + P.tau * (double)gz), &s, &c);
+        S[L.q * N + i] = c;
+        S[(L.q + 1) * N + i] = s;
     }
 }
 
@@ -224,72 +264,91 @@ __device__ __forceinline__ void local_V(const DevParams& P, int gx, int gy, int 
     im = VA * cs.y;
 }
 
-// Material::compute_pseudopotential_non_local_correction (Material.cpp:139-208)
-__device__ __forceinline__ void nonlocal(const DevParams& P, const KState& a, const KState& b, double& re, double& im) {
-    const double n1 = a.nK, n2 = b.nK;
+// F_l (Material.cpp:87-109) of the pair (i, j), averaged over its two orders.
+// The general branch is symmetric in them.  Norms within 1e-4 of each other
+// take the first vector's own value: the mean of both orders, as the
+// hermitisation 0.5 (H + H^dagger) leaves it.  id: 1 / (n1^2 - n2^2).
+__device__ __forceinline__ double F_l(double n1, double n2, double id, const DevParams::Radius& R, const double* S, int N,
+                                      int i, int j) {
+    constexpr double EPSILON = 1.0e-4;
+    if (fabs(n1 - n2) > EPSILON) {
+        const double F = n1 * S[N + i] * S[j] - n2 * S[N + j] * S[i];
+        return R.R2 * id * F;
+    }
+    return 0.5 * ((n1 > EPSILON ? R.R3_2 * S[2 * N + i] : R.R3_3) + (n2 > EPSILON ? R.R3_2 * S[2 * N + j] : R.R3_3));
+}
+
+// Material::compute_pseudopotential_non_local_correction (Material.cpp:139-208),
+// hermitised: every factor is symmetric in the pair or (the phase) conjugated by
+// its exchange, so one evaluation serves both elements.
+__device__ __forceinline__ void nonlocal(const DevParams& P, const VecLayout& L, const double* S, int i, int j, double& re,
+                                         double& im) {
+    const int N = P.N;
+    const double n1 = S[L.nK * N + i], n2 = S[L.nK * N + j];
     double leg2 = 0.0;  // P_2(cos angle(K1, K2)), used by the l = 2 terms only
     if (P.need_l2_a || P.need_l2_c) {
-        const double dp = a.Kx * b.Kx + a.Ky * b.Ky + a.Kz * b.Kz;
-        const double np = n1 * n2;
-        const double cosang = (np < 1.0e-13) ? 1.0 : dp / (n1 * n2);
+        const double* kx = S + L.k * N;
+        const double dp = kx[i] * kx[j] + kx[N + i] * kx[N + j] + kx[2 * N + i] * kx[2 * N + j];
+        const double cosang = (n1 * n2 < 1.0e-13) ? 1.0 : dp * (S[L.ik * N + i] * S[L.ik * N + j]);
         leg2 = 0.5 * (3 * cosang * cosang - 1);
     }
     const double nn = n1 * n2 - P.kF2;
+    const bool any_F = P.need_l0_a || P.need_l0_c || P.well == 0;
+    const double id = any_F ? 1.0 / (n1 * n1 - n2 * n2) : 0.0;
     double Va = 0.0, Vc = 0.0;
-    double F0a = 0.0;
+    double F0 = 0.0, F2 = 0.0;
+    auto radial2 = [&](const DevParams::Radius& R, double h2, int at) {
+        if (P.well == 0) return F_l(n1, n2, id, R, S + at * N, N, i, j);
+        return mod_i2(h2 * (n1 * n2)) * (S[at * N + i] * S[at * N + j]);
+    };
     if (P.need_l0_a) {
-        F0a = F_l(n1, n2, P.R0_a, 0, a.b0a, b.b0a);
-        Va = P.V_pre * (P.alpha0_a + P.dfbeta_a * nn) * F0a;
+        F0 = F_l(n1, n2, id, P.r0_a, S + L.l0a * N, N, i, j);
+        Va = P.V_pre * (P.alpha0_a + P.dfbeta_a * nn) * F0;
     }
     if (P.need_l2_a) {
-        double V2;
-        if (P.well == 0) V2 = P.V_pre * P.A2_a * 5 * leg2 * F_l(n1, n2, P.R2_a, 2, a.b2a, b.b2a);
-        else V2 = P.gpre_a * P.A2_a * leg2 * F_2_gauss(n1, n2, P.R2_a);
-        Va += V2;
+        F2 = radial2(P.r2_a, P.h2_a, L.l2a);
+        Va += P.w2_a * leg2 * F2;
     }
     if (P.need_l0_c) {
-        // the same radius gives the same F_0 (the Bessel triples are equal too)
-        const double F0c = P.same_r0 ? F0a : F_l(n1, n2, P.R0_c, 0, a.b0c, b.b0c);
-        Vc = P.V_pre * (P.alpha0_c + P.dfbeta_c * nn) * F0c;
+        if (!P.same_r0) F0 = F_l(n1, n2, id, P.r0_c, S + L.l0c * N, N, i, j);
+        Vc = P.V_pre * (P.alpha0_c + P.dfbeta_c * nn) * F0;
     }
     if (P.need_l2_c) {
-        double V2;
-        if (P.well == 0) V2 = P.V_pre * P.A2_c * 5 * leg2 * F_l(n1, n2, P.R2_c, 2, a.b2c, b.b2c);
-        else V2 = P.gpre_c * P.A2_c * leg2 * F_2_gauss(n1, n2, P.R2_c);
-        Vc += V2;
+        if (!P.same_r2) F2 = radial2(P.r2_c, P.h2_c, L.l2c);
+        Vc += P.w2_c * leg2 * F2;
     }
     const double Vs = 1.0 * (Va + Vc) / 2.0;
     const double Vas = 1.0 * (Va - Vc) / 2.0;
     // cos / sin of 2 pi (tau/a) sum_c (K_a - K_b)_c from the per-vector phases
-    // (the reference forms the difference first; the two agree to rounding, and
-    // the product form keeps the (b, a) value the exact conjugate)
-    const double c = a.pc * b.pc + a.ps * b.ps;
-    const double s = a.ps * b.pc - a.pc * b.ps;
+    // (the reference forms the difference first; the two agree to rounding)
+    const double *pc = S + L.ph * N, *ps = pc + N;
+    const double c = pc[i] * pc[j] + ps[i] * ps[j];
+    const double s = ps[i] * pc[j] - pc[i] * ps[j];
     re = c * Vs;
     im = s * Vas;
 }
 
 // SpinOrbitCorrection::compute_soc_contribution (SpinOrbitFunctional.cpp:111-138):
-// s[0..3] = (s00, s01, s10, s11) as (re, im) pairs; K = k + G reduced.
-__device__ __forceinline__ void soc_block(const DevParams& P, const KState& a, const KState& b, int gx, int gy, int gz,
-                                          double* s) {
-    const double l1 = P.mu * a.Bc * b.Bc;
-    const double l2 = P.alpha_mu * a.Ba * b.Ba;
+// s[0..5] = s00, s01, s10 as (re, im) pairs; s11 = -s00.  Exchanging the pair
+// conjugate-transposes the block exactly, so it is its own hermitisation.
+__device__ __forceinline__ void soc_block(const DevParams& P, const VecLayout& L, const double* S, int i, int j, double* s) {
+    const int N = P.N;
+    const double *Ba = S + L.B * N, *Bc = Ba + N, *qc = S + L.q * N, *qs = qc + N;
+    const double l1 = P.mu * (Bc[i] * Bc[j]);
+    const double l2 = P.alpha_mu * (Ba[i] * Ba[j]);
     const double lsym = (l1 + l2) / 2.0;
     const double lanti = (l1 - l2) / 2.0;
-    const double cz = a.kx * b.ky - a.ky * b.kx;
-    const double cx = a.ky * b.kz - a.kz * b.ky;
-    const double cy = a.kx * b.kz - a.kz * b.kx;
-    const double Gtau = P.soc_kfac * (P.tau * (double)gx + P.tau * (double)gy + P.tau * (double)gz);
-    double sn, cs;
-    sincos(Gtau, &sn, &cs);
+    const double *kx = S + L.k * N, *ky = kx + N, *kz = ky + N;
+    const double cz = kx[i] * ky[j] - ky[i] * kx[j];
+    const double cx = ky[i] * kz[j] - kz[i] * ky[j];
+    const double cy = kx[i] * kz[j] - kz[i] * kx[j];
+    // the phase of G_i - G_j from the per-vector phases
+    const double cs = qc[i] * qc[j] + qs[i] * qs[j];
+    const double sn = qs[i] * qc[j] - qc[i] * qs[j];
     const double pr = lanti * sn, pi = -lsym * cs;
-    // (a + bi)(pr + i pi) = (a pr - b pi) + i (a pi + b pr)
-    s[0] = cz * pr - 0.0 * pi;  s[1] = cz * pi + 0.0 * pr;
-    s[2] = cx * pr - cy * pi;   s[3] = cx * pi + cy * pr;
-    s[4] = cx * pr + cy * pi;   s[5] = cx * pi - cy * pr;
-    const double mz = -(a.kx * b.ky - a.ky * b.kx);
-    s[6] = mz * pr - 0.0 * pi;  s[7] = mz * pi + 0.0 * pr;
+    s[0] = cz * pr;            s[1] = cz * pi;
+    s[2] = cx * pr - cy * pi;  s[3] = cx * pi + cy * pr;
+    s[4] = cx * pr + cy * pi;  s[5] = cx * pi - cy * pr;
 }
 
 #pragma clang fp contract(on)

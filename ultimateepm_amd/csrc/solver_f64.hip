@@ -1,13 +1,10 @@
-// solver_f64.hip — assembly and tridiagonal eigen-stage of the band solve on gfx950.
+// solver_f64.hip — tridiagonal eigen-stage of the band solve on gfx950.
 //
-//   (a) assemble_tiled_kernel / assemble_kernel  H(k) for a batch of k-points
-//                           (Hamiltonian::SetMatrix + the 0.5 (H + H^dagger)
-//                           step of Diagonalize, src/EPP/Hamiltonian.cpp:50-127)
 //   (c) tri_eig_wave_kernel bisection (Sturm counts, multisection) for the lowest
 //                           nb eigenvalues of T and inverse iteration for their
 //                           vectors, one wave per k
 //
-// The Householder reduction (b) lives in tridiag_reg.hip / tridiag_blocked.hip
+// The assembly (a) lives in assemble.hip, the Householder reduction (b) in tridiag_reg.hip / tridiag_blocked.hip
 // and the back-transform (d) in backtransform.hip; (b)-(d) replace
 // Eigen::SelfAdjointEigenSolver::compute (Hamiltonian.cpp:129): same
 // eigenvalues to within the backward-stability envelope of a Householder
@@ -17,209 +14,11 @@
 #include <cfloat>
 #include <cstdint>
 #include <cstdlib>
-#include <type_traits>
 
 #include "epm_physics.hpp"
 #include "solver.hpp"
 
 namespace uepm {
-
-// ------------------------------------------------------------ (a) assembly
-// h_ij and h_ji of the pair (i, j) before hermitisation and spin-orbit: V(G),
-// the kinetic diagonal and the non-local term.  h_ji comes from h_ij where
-// that is exact: the phase argument of V(G) negates exactly under i <-> j and
-// the device sincos is exactly odd / even there; the non-local phase is
-// cos / sin of theta_i - theta_j formed from the per-vector cos / sin, which
-// swap to the exact conjugate (products commute, no FMA contraction); the
-// square-well radial integrals are symmetric in |K_i|, |K_j| outside the
-// near-equal branch of F_l (which reads one side's Bessel values) -- so one
-// evaluation gives the reference's two-sided 0.5 (h_ij + conj(h_ji)) bit for
-// bit.  Gaussian l = 2 wells and near-equal norms are evaluated both ways.
-__device__ __forceinline__ void pair_terms(const DevParams& P, const KState& si, const KState& sj, int gx, int gy,
-                                           int gz, bool diag, const double2* vtab, bool swap_exact, double& re_ij,
-                                           double& im_ij, double& re_ji, double& im_ji) {
-    local_V(P, gx, gy, gz, re_ij, im_ij, vtab);
-    re_ji = re_ij;
-    im_ji = -im_ij;
-    if (diag) {
-        const double KG2 = P.kin * (si.kx * si.kx + si.ky * si.ky + si.kz * si.kz);
-        re_ij += KG2;
-        re_ji += KG2;
-    }
-    if (P.nl) {
-        double r1, i1, r2, i2;
-        nonlocal(P, si, sj, r1, i1);
-        if (swap_exact && fabs(si.nK - sj.nK) > 1.0e-4) {
-            r2 = r1;
-            i2 = -i1;
-        } else {
-            nonlocal(P, sj, si, r2, i2);
-        }
-        re_ij += r1; im_ij += i1;
-        re_ji += r2; im_ji += i2;
-    }
-}
-
-// One workgroup per k.  Per-basis-vector state in LDS, then every (i, j) pair
-// of the lower triangle: the stored value is the reference's
-// 0.5 (h_ij + conj(h_ji)) (its Diagonalize hermitisation), mirrored into the
-// upper triangle; h_ji is derived from h_ij where that is exact (below).
-// Output: column-major dim x dim, leading dimension ld, one matrix per k.
-template <int BS>
-__global__ __launch_bounds__(BS) void assemble_kernel(DevParams P, const int32_t* __restrict__ G,
-                                                       const double* __restrict__ kpts, double2* __restrict__ H,
-                                                       int ld) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    KState* ks = reinterpret_cast<KState*>(smem);
-    __shared__ double2 vtab[kVPhaseTab];
-    const int kk = blockIdx.x;
-    const double* k = kpts + 3 * (size_t)kk;
-    const int N = P.N;
-    for (int i = threadIdx.x; i < N; i += BS) kstate_init(P, k, G, i, ks[i]);
-    for (int t = threadIdx.x; t < kVPhaseTab; t += BS) vtab[t] = local_phase(P, t / 49 - 3, (t / 7) % 7 - 3, t % 7 - 3);
-    __syncthreads();
-    double2* A = H + (size_t)kk * ld * P.dim;
-    const int npairs = N * (N + 1) / 2;
-    // h_ji from h_ij where exact (pair_terms)
-    const bool swap_exact = !(P.well != 0 && (P.need_l2_a || P.need_l2_c));
-    // element t -> (i, j), column-major over the packed lower triangle; the
-    // first from the closed form, then advanced by BS per iteration
-    int t = threadIdx.x, j = 0, i = 0;
-    if (t < npairs) {
-        j = (int)((2.0 * N + 1.0 - sqrt((2.0 * N + 1.0) * (2.0 * N + 1.0) - 8.0 * t)) * 0.5);
-        while (j > 0 && j * (2 * N - j + 1) / 2 > t) --j;
-        while ((j + 1) * (2 * N - j) / 2 <= t) ++j;
-        i = j + (t - j * (2 * N - j + 1) / 2);
-    }
-    for (; t < npairs; t += BS) {
-        if (t != (int)threadIdx.x) {
-            i += BS;
-            while (i >= N && j < N - 1) {  // past the end of column j: continue at the diagonal of column j + 1
-                i -= N - (j + 1);
-                ++j;
-            }
-        }
-        const KState& si = ks[i];
-        const KState& sj = ks[j];
-        const int gx = G[3 * i] - G[3 * j], gy = G[3 * i + 1] - G[3 * j + 1], gz = G[3 * i + 2] - G[3 * j + 2];
-        double re_ij, im_ij, re_ji, im_ji;
-        pair_terms(P, si, sj, gx, gy, gz, i == j, vtab, swap_exact, re_ij, im_ij, re_ji, im_ji);
-        if (!P.soc) {
-            const double hr = 0.5 * (re_ij + re_ji), hi = 0.5 * (im_ij - im_ji);
-            A[i + (size_t)j * ld] = make_double2(hr, hi);
-            A[j + (size_t)i * ld] = make_double2(hr, -hi);
-        } else {
-            double s_ij[8], s_ji[8];
-            soc_block(P, si, sj, gx, gy, gz, s_ij);
-            soc_block(P, sj, si, -gx, -gy, -gz, s_ji);
-            // blocks: [[M+S00, S01],[S10, M+S11]]; element (row, col)
-            // (i, j) of block (p, q) pairs with (j, i) of block (q, p).
-            const int n0 = N;
-            // up-up
-            {
-                const double ar = re_ij + s_ij[0], ai = im_ij + s_ij[1];
-                const double br = re_ji + s_ji[0], bi = im_ji + s_ji[1];
-                const double hr = 0.5 * (ar + br), hi = 0.5 * (ai - bi);
-                A[i + (size_t)j * ld] = make_double2(hr, hi);
-                A[j + (size_t)i * ld] = make_double2(hr, -hi);
-            }
-            // down-down
-            {
-                const double ar = re_ij + s_ij[6], ai = im_ij + s_ij[7];
-                const double br = re_ji + s_ji[6], bi = im_ji + s_ji[7];
-                const double hr = 0.5 * (ar + br), hi = 0.5 * (ai - bi);
-                A[(i + n0) + (size_t)(j + n0) * ld] = make_double2(hr, hi);
-                A[(j + n0) + (size_t)(i + n0) * ld] = make_double2(hr, -hi);
-            }
-            // down-up (row i+N, col j) pairs with up-down (row j, col i+N)
-            {
-                const double hr = 0.5 * (s_ij[4] + s_ji[2]), hi = 0.5 * (s_ij[5] - s_ji[3]);
-                A[(i + n0) + (size_t)j * ld] = make_double2(hr, hi);
-                A[j + (size_t)(i + n0) * ld] = make_double2(hr, -hi);
-            }
-            if (i != j) {
-                // down-up (row j+N, col i) pairs with up-down (row i, col j+N)
-                const double hr = 0.5 * (s_ji[4] + s_ij[2]), hi = 0.5 * (s_ji[5] - s_ij[3]);
-                A[(j + n0) + (size_t)i * ld] = make_double2(hr, hi);
-                A[i + (size_t)(j + n0) * ld] = make_double2(hr, -hi);
-            }
-        }
-    }
-}
-
-// Without spin-orbit: each wave takes 16 x 16 tiles (bi >= bj) of the lower
-// triangle, writes the tile and, through its LDS slot, the conjugate
-// transpose above the diagonal, so both halves go out in 256-byte column
-// runs (the mirrored writes of assemble_kernel are one element per column).
-// Element values are assemble_kernel's, bit for bit.
-// T = double: only the real parts, for plans whose H(k) is real (the imaginary
-// parts are exactly zero there): half the bytes of the complex matrix.
-template <int BS, typename T>
-__global__ __launch_bounds__(BS) void assemble_tiled_kernel(DevParams P, const int32_t* __restrict__ G,
-                                                             const double* __restrict__ kpts, T* __restrict__ H,
-                                                             int ld) {
-    constexpr bool kReal = std::is_same_v<T, double>;
-    extern __shared__ __align__(16) unsigned char smem[];
-    KState* ks = reinterpret_cast<KState*>(smem);
-    __shared__ double2 vtab[kVPhaseTab];
-    __shared__ T Tt[BS / 64][16][17];
-    const int kk = blockIdx.x;
-    const double* k = kpts + 3 * (size_t)kk;
-    const int N = P.N;
-    for (int i = threadIdx.x; i < N; i += BS) kstate_init(P, k, G, i, ks[i]);
-    for (int t = threadIdx.x; t < kVPhaseTab; t += BS) vtab[t] = local_phase(P, t / 49 - 3, (t / 7) % 7 - 3, t % 7 - 3);
-    __syncthreads();
-    T* A = H + (size_t)kk * ld * P.dim;
-    const bool swap_exact = !(P.well != 0 && (P.need_l2_a || P.need_l2_c));
-    const int nt = (N + 15) >> 4, ntiles = nt * (nt + 1) / 2;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int il = lane & 15, jq = lane >> 4;
-    T(*Tw)[17] = Tt[wv];
-    for (int tile = wv; tile < ntiles; tile += BS / 64) {
-        // tile -> (bi, bj), column-major over the lower triangle of tiles
-        int bj = 0, rem = tile;
-        while (rem >= nt - bj) {
-            rem -= nt - bj;
-            ++bj;
-        }
-        const int bi = bj + rem;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int jl = jq + 4 * q;
-            const int i = 16 * bi + il, j = 16 * bj + jl;
-            if (i < N && j < N && i >= j) {
-                const KState& si = ks[i];
-                const KState& sj = ks[j];
-                const int gx = G[3 * i] - G[3 * j], gy = G[3 * i + 1] - G[3 * j + 1], gz = G[3 * i + 2] - G[3 * j + 2];
-                double re_ij, im_ij, re_ji, im_ji;
-                pair_terms(P, si, sj, gx, gy, gz, i == j, vtab, swap_exact, re_ij, im_ij, re_ji, im_ji);
-                const double hr = 0.5 * (re_ij + re_ji), hi = 0.5 * (im_ij - im_ji);
-                if constexpr (kReal) {
-                    A[i + (size_t)j * ld] = hr;
-                    Tw[jl][il] = hr;
-                } else {
-                    // the diagonal as assemble_kernel's mirrored write leaves it
-                    A[i + (size_t)j * ld] = make_double2(hr, i == j ? -hi : hi);
-                    Tw[jl][il] = make_double2(hr, hi);
-                }
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int rl = il, cl = jq + 4 * q;
-            const int row = 16 * bj + rl, col = 16 * bi + cl;
-            if (row < N && col < N && row < col) {
-                const T h = Tw[rl][cl];  // h(col, row)
-                if constexpr (kReal) A[row + (size_t)col * ld] = h;
-                else A[row + (size_t)col * ld] = make_double2(h.x, -h.y);
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
-}
 
 // ------------------------------------- (c) tridiagonal eigenvalues / vectors
 // Start vector of inverse iteration: a fixed pseudo-random value per (row, band).
@@ -525,39 +324,6 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
 }
 
 // ------------------------------------------------------------ launchers
-constexpr int kAsmBS = 256;
-
-namespace {
-template <typename K, typename T>
-hipError_t launch_assemble_kernel(K kern, size_t fixed, const DevParams& P, const int32_t* dG, const double* dk,
-                                  int64_t nk, T* dH, int ld, hipStream_t s) {
-    // one KState per basis vector in LDS beside the phase table (and the tiled
-    // kernel's transpose slots): up to 766 vectors (860 with spin-orbit) in
-    // the 160 KB of a CU
-    const size_t shm = sizeof(KState) * (size_t)P.N;
-    if (shm + fixed > 163840) return hipErrorInvalidValue;
-    hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(kern, dim3((unsigned)nk), dim3(kAsmBS), shm, s, P, dG, dk, dH, ld);
-    return hipGetLastError();
-}
-constexpr size_t kAsmTab = sizeof(double2) * kVPhaseTab, kAsmSlots = (kAsmBS / 64) * 16 * 17;
-}  // namespace
-
-hipError_t launch_assemble(const DevParams& P, const int32_t* dG, const double* dk, int64_t nk, double2* dH, int ld,
-                           hipStream_t s) {
-    if (P.soc) return launch_assemble_kernel(assemble_kernel<kAsmBS>, kAsmTab, P, dG, dk, nk, dH, ld, s);
-    return launch_assemble_kernel(assemble_tiled_kernel<kAsmBS, double2>, kAsmTab + kAsmSlots * sizeof(double2), P, dG, dk,
-                                  nk, dH, ld, s);
-}
-
-hipError_t launch_assemble_real(const DevParams& P, const int32_t* dG, const double* dk, int64_t nk, double* dH, int ld,
-                                hipStream_t s) {
-    if (P.soc) return hipErrorInvalidValue;
-    return launch_assemble_kernel(assemble_tiled_kernel<kAsmBS, double>, kAsmTab + kAsmSlots * sizeof(double), P, dG, dk, nk,
-                                  dH, ld, s);
-}
-
 hipError_t launch_tri_eig(const double* dd, const double* de, int n, int nb, int64_t nk, double* devals, double* dZ,
                           double* dW, int inv_sweeps, double abstol_rel, int* kstat, unsigned long long* status,
                           int64_t k0, hipStream_t s) {

@@ -715,6 +715,17 @@ int uepm_plan_create(uepm_ctx* ctx, const uepm_material* m, const int32_t* G, in
     P.R0_c = m->R0_cation;
     P.R2_c = m->R2_cation;
     P.gpre_c = 5.0 * std::pow(kPi, 1.5) * (std::pow(m->R2_cation, 3.0) / omega);
+    P.w2_a = P.well == 0 ? P.V_pre * P.A2_a * 5 : P.gpre_a * P.A2_a;
+    P.w2_c = P.well == 0 ? P.V_pre * P.A2_c * 5 : P.gpre_c * P.A2_c;
+    P.h2_a = 0.5 * (P.R2_a * P.R2_a);
+    P.h2_c = 0.5 * (P.R2_c * P.R2_c);
+    auto radius = [](double R, int l) {
+        return uepm::DevParams::Radius{R * R, (R * R * R) / (2.0), l == 0 ? (R * R * R) / (3.0) : 0.0};
+    };
+    P.r0_a = radius(P.R0_a, 0);
+    P.r0_c = radius(P.R0_c, 0);
+    P.r2_a = radius(P.R2_a, 2);
+    P.r2_c = radius(P.R2_c, 2);
     // F_0 contributes only when R0 != 0 (Material.cpp:159,180) and its
     // coefficient A_0 = alpha + diag*beta*(...) is not identically zero.
     P.need_l0_a = (m->R0_anion != 0.0) && (m->alpha_0_anion != 0.0 || m->beta_0_anion != 0.0);
@@ -722,6 +733,7 @@ int uepm_plan_create(uepm_ctx* ctx, const uepm_material* m, const int32_t* G, in
     P.need_l2_a = m->A2_anion != 0.0;
     P.need_l2_c = m->A2_cation != 0.0;
     P.same_r0 = P.need_l0_a && P.need_l0_c && m->R0_anion == m->R0_cation;
+    P.same_r2 = P.need_l2_a && P.need_l2_c && m->R2_anion == m->R2_cation;
     // SpinOrbitFunctional.cpp
     P.soc_kfac = (2.0 * kPi) / a;
     P.period_a = m->period_anion;
