@@ -41,13 +41,6 @@ int next(int n) {
     return size > 192 ? kSize[stage_of(n) + 1] : size > 128 ? 128 : size > 64 ? 64 : 0;
 }
 
-template <typename R, int RW, int CW, int NG, int MINW, typename THin>
-void row_stage(const THin* H, int64_t hk, int n, int ld, int64_t nk, R* V, int ldv, int64_t vk, double* dd, double* de,
-               R* dtau, int64_t dk, int s_end, R* B, int ldb, hipStream_t s) {
-    hipLaunchKernelGGL((tridiag_row_kernel<R, RW, CW, NG, MINW, THin>), dim3((unsigned)nk), dim3(64 * RW * CW), 0, s, H,
-                       hk, n, ld, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb);
-}
-
 // One stage.  Shapes and register budgets (waves per SIMD) are the fastest of a
 // sweep that did not spill in the steps; 16 x 16 lanes where a grid fits their
 // registers (four waves meet at a barrier instead of eight), 32 x 16 above.
@@ -61,7 +54,7 @@ void stage(const THin* H, int64_t hk, int n, int ld, int64_t nk, float* V, int l
     using S = r1<float>;
     constexpr bool kFromH = sizeof(THin) == sizeof(double);  // no stage hands over to these three
 #define UEPM_GRID(...) reg_stage<S, __VA_ARGS__>(H, hk, n, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s)
-#define UEPM_ROWS(...) row_stage<float, __VA_ARGS__, THin>(H, hk, n, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s)
+#define UEPM_ROWS(...) row_stage<S, __VA_ARGS__, 1>(H, hk, n, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s)
     switch (kSize[stage_of(n)]) {
         case 448:
             if constexpr (kFromH) UEPM_GRID(32, 14, 2, 1, THin, true, 30, true);
@@ -75,7 +68,7 @@ void stage(const THin* H, int64_t hk, int n, int ld, int64_t nk, float* V, int l
         case 160:
             if constexpr (kFromH) UEPM_GRID(16, 10, 4, 1, THin, false, 0, true);
             break;
-        case 128: UEPM_ROWS(2, 1, 8, 3); break;
+        case 128: UEPM_ROWS(2, 2, 4, 5); break;
         case 96:
             if constexpr (kFromH) UEPM_ROWS(2, 1, 6, 3);
             break;
@@ -88,7 +81,7 @@ void stage(const double* H, int64_t hk, int n, int ld, int64_t nk, double* V, in
            double* dtau, int64_t dk, int s_end, double* B, int ldb, hipStream_t s) {
     using S = r1<double>;
 #define UEPM_GRID(...) reg_stage<S, __VA_ARGS__>(H, hk, n, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s)
-#define UEPM_ROWS(...) row_stage<double, __VA_ARGS__, double>(H, hk, n, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s)
+#define UEPM_ROWS(...) row_stage<S, __VA_ARGS__, 1>(H, hk, n, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s)
     switch (kSize[stage_of(n)]) {
         case 320: UEPM_GRID(32, 10, 2, 1, double, true, 24, true); break;
         case 288: UEPM_GRID(32, 9, 2, 1, double, true, 0, true); break;

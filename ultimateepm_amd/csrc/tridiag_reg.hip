@@ -11,6 +11,7 @@
 
 #include "solver.hpp"
 #include "tridiag_grid.hpp"
+#include "tridiag_row.hpp"
 #include "wave_ops.hpp"
 
 namespace uepm {
@@ -279,7 +280,10 @@ hipError_t launch_tridiag_reg_c64_block(const float2* H, int64_t hk, int m, int 
 
 // ---- FP64: grids 192 (6 x 12, low-register, 256 VGPRs with a small spill), 160
 // (5 x 10, low-register) and 128 (4 x 8), one workgroup per CU; 96 (3 x 6,
-// low-register, 128 VGPRs) and 64 (2 x 4), two.  A larger FP64 matrix runs the
+// low-register, 128 VGPRs), two.  The last 64 steps run one row per lane in two
+// column waves, four workgroups per CU (tridiag_row.hpp; 4096 blocks of 64 take
+// 0.59 ms, a 2 x 4 grid 1.48; blocks of 27 in one wave 0.14; at 96 the grid is
+// the faster, 1.27 ms for 32 steps against 1.50).  A larger FP64 matrix runs the
 // blocked reduction first and hands over its trailing block at a panel boundary.
 namespace {
 constexpr int kNumGrids64 = 5;
@@ -301,8 +305,14 @@ void grid64_stage(int g, const double2* H, int64_t hk, int m, int ld, int64_t nk
         case 0: reg_stage<c2<double>, 32, 6, 1, IN, double2, true, NL64_192>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         case 1: reg_stage<c2<double>, 32, 5, 1, IN, double2, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         case 2: reg_stage<c2<double>, 32, 4, 1, IN, double2>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 3: reg_stage<c2<double>, 32, 3, 4, IN, double2, true, NL64_96>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        default: reg_stage<c2<double>, 32, 2, 4, IN, double2>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        // hands both triangles to the row kernel
+        case 3: reg_stage<c2<double>, 32, 3, 4, IN, double2, true, NL64_96, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        default:
+            if constexpr (IN != 0) {
+                if (m <= 32) row_stage<c2<double>, 1, 1, 2, 2, IN>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
+                else row_stage<c2<double>, 1, 2, 2, 2, IN>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
+            }
+            break;
     }
 }
 }  // namespace
@@ -327,6 +337,7 @@ hipError_t launch_tridiag_reg_c128(const double2* H, int64_t hk, int m, int ld, 
                                    double2* V, int ldv, int64_t vk, double* dd, double* de, double2* dtau, int64_t dk,
                                    double2* work, hipStream_t s) {
     if (m < 1 || m > kGrid64[0] || nk <= 0) return hipErrorInvalidValue;
+    if (!hermitian_full && grid64_of(m) == kNumGrids64 - 1) return hipErrorInvalidValue;  // the row kernel reads both triangles
     // the first grid reads the block's rows (the conjugate upper triangle) when
     // the whole Hermitian matrix is there, its lower columns otherwise
     auto first = [&](int s_end, double2* B, int ldb) {
