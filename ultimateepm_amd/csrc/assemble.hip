@@ -13,16 +13,19 @@
 #include <cstdint>
 
 #include "epm_physics.hpp"
+#include "scalars.hpp"
 #include "solver.hpp"
 
 namespace uepm {
 
 // What a plan's H(k) is stored as.
-enum class HForm { kComplex, kReal, kSpinor };
+enum class HForm { kComplex, kReal, kSpinor, kQuaternion };
 template <HForm F>
 struct HElem { using T = double2; };
 template <>
 struct HElem<HForm::kReal> { using T = double; };
+template <>
+struct HElem<HForm::kQuaternion> { using T = q4<double>; };
 
 // One workgroup per k.  Per-basis-vector state in LDS, then 16 x 16 tiles of
 // pairs (i, j), i >= j, one wave a tile: each wave evaluates its pairs once
@@ -34,6 +37,8 @@ struct HElem<HForm::kReal> { using T = double; };
 //   kReal    the real parts alone, where the imaginary parts are exactly zero
 //   kSpinor  2N x 2N: blocks [[M + S00, S01], [S10, M - S00]], each tile of pairs
 //            writing its four blocks (and their transposes) in turn
+//   kQuaternion  N x N: u = M + S00 and d = S10 of each spinor block, which is
+//            [[u, -conj(d)], [d, conj(u)]] where the antisymmetric terms vanish
 template <int BS, HForm F>
 __global__ __launch_bounds__(BS, 4) void assemble_kernel(DevParams P, const int32_t* __restrict__ G,
                                                       const double* __restrict__ kpts,
@@ -42,7 +47,8 @@ __global__ __launch_bounds__(BS, 4) void assemble_kernel(DevParams P, const int3
     extern __shared__ __align__(16) unsigned char smem[];
     double* S = reinterpret_cast<double*>(smem);
     __shared__ double2 vtab[kVPhaseTab];
-    __shared__ T Tt[BS / 64][F == HForm::kSpinor ? 4 : 16][17];
+    constexpr bool kSoc = F == HForm::kSpinor || F == HForm::kQuaternion;
+    __shared__ T Tt[BS / 64][kSoc ? 4 : 16][17];
     const int kk = blockIdx.x;
     const double* k = kpts + 3 * (size_t)kk;
     const int N = P.N;
@@ -51,7 +57,7 @@ __global__ __launch_bounds__(BS, 4) void assemble_kernel(DevParams P, const int3
     for (int i = threadIdx.x; i < N; i += BS) vector_init(P, L, k, G, i, S, Gp);
     for (int t = threadIdx.x; t < kVPhaseTab; t += BS) vtab[t] = local_phase(P, t / 49 - 3, (t / 7) % 7 - 3, t % 7 - 3);
     __syncthreads();
-    T* A = H + (size_t)kk * ld * P.dim;
+    T* A = H + (size_t)kk * ld * (F == HForm::kQuaternion ? N : P.dim);
     const int nt = (N + 15) >> 4, ntiles = nt * (nt + 1) / 2;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int il = lane & 15, jq = lane >> 4;
@@ -90,7 +96,7 @@ __global__ __launch_bounds__(BS, 4) void assemble_kernel(DevParams P, const int3
                     re += r;
                     im += m;
                 }
-                if constexpr (F == HForm::kSpinor) soc_block(P, L, S, i, j, so);
+                if constexpr (kSoc) soc_block(P, L, S, i, j, so);
             }
             if constexpr (F == HForm::kReal) {
                 if (in) A[i + (size_t)j * ld] = Tw[jl][il] = re;
@@ -100,23 +106,29 @@ __global__ __launch_bounds__(BS, 4) void assemble_kernel(DevParams P, const int3
                 // the blocks in turn: element (row r0 + i, column c0 + j), and its conjugate at
                 // (c0 + j, r0 + i) through four rows of the slot (runs of four elements); the
                 // diagonal of an off-diagonal block has a transpose of its own
-                auto put = [&](int r0, int c0, double x, double y) {
-                    if (in) A[(r0 + i) + (size_t)(c0 + j) * ld] = Tw[jq][il] = make_double2(x, y);
+                auto put = [&](int r0, int c0, T h) {
+                    if (in) A[(r0 + i) + (size_t)(c0 + j) * ld] = Tw[jq][il] = h;
                     wsync();
                     const int j2 = 16 * bj + 4 * q + (lane & 3), i2 = 16 * bi + (lane >> 2);
                     if (i2 < N && j2 < N && (i2 > j2 || (i2 == j2 && r0 != c0))) {
-                        const double2 h = Tw[lane & 3][lane >> 2];
-                        A[(c0 + j2) + (size_t)(r0 + i2) * ld] = make_double2(h.x, -h.y);
+                        const T t = Tw[lane & 3][lane >> 2];
+                        T& to = A[(c0 + j2) + (size_t)(r0 + i2) * ld];
+                        if constexpr (F == HForm::kQuaternion) to = conj_if(t, true);
+                        else to = make_double2(t.x, -t.y);
                     }
                     wsync();
                 };
-                put(0, 0, re + so[0], im + so[1]);
-                put(N, N, re - so[0], im - so[1]);
-                put(N, 0, so[4], so[5]);
-                put(0, N, so[2], so[3]);
+                if constexpr (F == HForm::kQuaternion) {
+                    put(0, 0, T{re + so[0], im + so[1], so[4], so[5]});
+                } else {
+                    put(0, 0, make_double2(re + so[0], im + so[1]));
+                    put(N, N, make_double2(re - so[0], im - so[1]));
+                    put(N, 0, make_double2(so[4], so[5]));
+                    put(0, N, make_double2(so[2], so[3]));
+                }
             }
         }
-        if constexpr (F != HForm::kSpinor) {
+        if constexpr (!kSoc) {
             wsync();
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -142,7 +154,7 @@ hipError_t launch_assemble_form(const DevParams& P, const int32_t* dG, const dou
     // the per-vector arrays (at most 164 bytes a vector) beside the phase table and
     // the transpose slots: 576 vectors take 118 of the 160 KB of a CU
     const size_t shm = vec_bytes(P);
-    const size_t fixed = sizeof(double2) * kVPhaseTab + (kAsmBS / 64) * (F == HForm::kSpinor ? 4 : 16) * 17 * sizeof(typename HElem<F>::T);
+    const size_t fixed = sizeof(double2) * kVPhaseTab + (kAsmBS / 64) * (F == HForm::kSpinor || F == HForm::kQuaternion ? 4 : 16) * 17 * sizeof(typename HElem<F>::T);
     if (shm + fixed > 163840) return hipErrorInvalidValue;
     auto kern = assemble_kernel<kAsmBS, F>;
     hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
@@ -162,6 +174,12 @@ hipError_t launch_assemble_real(const DevParams& P, const int32_t* dG, const dou
                                 hipStream_t s) {
     if (P.soc) return hipErrorInvalidValue;
     return launch_assemble_form<HForm::kReal>(P, dG, dk, nk, dH, ld, s);
+}
+
+hipError_t launch_assemble_quaternion(const DevParams& P, const int32_t* dG, const double* dk, int64_t nk, q4<double>* dH,
+                                      int ld, hipStream_t s) {
+    if (!P.soc) return hipErrorInvalidValue;
+    return launch_assemble_form<HForm::kQuaternion>(P, dG, dk, nk, dH, ld, s);
 }
 
 }  // namespace uepm

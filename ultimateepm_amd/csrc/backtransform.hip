@@ -22,6 +22,7 @@
 
 #include "epm_physics.hpp"
 #include "row_ops.hpp"
+#include "scalars.hpp"
 #include "solver.hpp"
 #include "wave_ops.hpp"
 
@@ -443,6 +444,239 @@ hipError_t launch_apply_q_real_f64(const double* dV, int n, const double* dtau, 
                                    double* dgrads, const DevParams& P, const double* dk, const int32_t* dG, int64_t nk,
                                    const int* kstat, unsigned long long* status, int64_t k0, hipStream_t s) {
     return apply_q_real<double, double2>(dV, n, dtau, dZ, nb, dX, dgrads, P, dk, dG, nk, kstat, status, k0, s);
+}
+
+// ---------------------------------------------------------------------------
+// x = Q z for quaternion reflectors: apply_q_real_kernel's scheme with four
+// components per row, the rows spread over W waves (64 NQ rows each, wave w the
+// blocks q W + w), whose shares of s = v^H x meet in LDS, one barrier a
+// reflector.  Band b' holds a Kramers pair: the spinors (u; d) and (-conj(d);
+// conj(u)).  T = q4<double>: the quaternion Ritz basis for the refinement; T =
+// double2: the pair as eigenvectors 2 b' and 2 b' + 1 of the nb, with gradients.
+template <typename R>
+struct QGroup {
+    R x[16], y[16], z[16], w[16];
+};
+template <typename R, int W, int NQ, typename T>
+__global__ __launch_bounds__(64 * W, sizeof(R) == 4 ? 3 : 2) void apply_q_quaternion_kernel(
+    const q4<R>* __restrict__ V, int n, const q4<R>* __restrict__ tauall, const double* __restrict__ Z, int nbq, int nb,
+    T* __restrict__ X, double* __restrict__ grads, DevParams P, const double* __restrict__ kpts,
+    const int32_t* __restrict__ G, const int* __restrict__ kstat, unsigned long long* __restrict__ status, int64_t k0) {
+    constexpr bool kRitz = sizeof(T) == sizeof(q4<double>);
+    __shared__ q4<R> part[2][W][16];
+    __shared__ double gsum[W][16][3];
+    const int64_t kk = blockIdx.x;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, g16 = lane & 48;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (status && blockIdx.y == 0 && threadIdx.x == 0 && kstat[kk]) {
+        atomicAdd(&status[0], 1ull);
+        atomicMin(&status[1], (unsigned long long)(k0 + kk));
+    }
+    const int b = 16 * blockIdx.y + l16;
+    const bool live = b < nbq;
+    const q4<R>* Vk = V + kk * (int64_t)n * n;
+    const q4<R>* tau = tauall + kk * n;
+    const double* z = Z + (kk * nbq + (live ? b : nbq - 1)) * (int64_t)n;
+    auto block = [&](int q) { return 64 * (q * W + wv); };  // first row of this wave's block q
+
+    QGroup<R> x[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int i = block(q) + g16 + r;
+            x[q].x[r] = (R)z[i < n ? i : n - 1] * (live && i < n ? R(1) : R(0));
+            x[q].y[r] = x[q].z[r] = x[q].w[r] = R(0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    auto vload = [&](int j, int q) -> q4<R> { return Vk[min(block(q) + lane, n - 1) + (int64_t)j * n]; };
+    q4<R> v[NQ], vn[NQ], t{}, tn{};
+    if (n >= 2) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) vn[q] = vload(n - 2, q);
+        tn = tau[n - 2];
+    } else if (n == 1) {
+        tn = tau[0];
+    }
+    for (int j = n - 2; j >= 0; --j) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) v[q] = vn[q];
+        t = tn;
+        {
+            const int jn = j > 0 ? j - 1 : 0;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+                if (block(q) + 63 > jn) vn[q] = vload(jn, q);
+            tn = tau[jn];
+        }
+        R ax[4] = {0, 0, 0, 0}, ay[4] = {0, 0, 0, 0}, az[4] = {0, 0, 0, 0}, aw[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+            if (block(q) + 63 > j) {
+                const int i = block(q) + lane;
+                v[q] = sel(i > j + 1 && i < n, v[q], sc_real<q4<R>>(i == j + 1 ? R(1) : R(0)));
+                const q4<R> a = v[q];
+                // conj(a) x (scalars.hpp, fma_cab)
+                rowop::dot16(ax, a.x, x[q].x);
+                rowop::dot16(ax, a.y, x[q].y);
+                rowop::dot16(ax, a.z, x[q].z);
+                rowop::dot16(ax, a.w, x[q].w);
+                rowop::dot16(ay, a.x, x[q].y);
+                rowop::dot16(ay, -a.y, x[q].x);
+                rowop::dot16(ay, a.z, x[q].w);
+                rowop::dot16(ay, -a.w, x[q].z);
+                rowop::dot16(az, a.x, x[q].z);
+                rowop::dot16(az, -a.y, x[q].w);
+                rowop::dot16(az, -a.z, x[q].x);
+                rowop::dot16(az, a.w, x[q].y);
+                rowop::dot16(aw, a.x, x[q].w);
+                rowop::dot16(aw, a.y, x[q].z);
+                rowop::dot16(aw, -a.z, x[q].y);
+                rowop::dot16(aw, -a.w, x[q].x);
+            }
+        auto total = [](const R (&a)[4]) -> R {  // over the accumulators and the four rows of the wave
+            R s = (a[0] + a[1]) + (a[2] + a[3]);
+            wave::Words<R> w0(s), w1(s);
+#pragma unroll
+            for (int i = 0; i < wave::Words<R>::n; ++i) wave::swap16(w0.w[i], w1.w[i]);
+            s = w0.value() + w1.value();
+            wave::Words<R> w2(s), w3(s);
+#pragma unroll
+            for (int i = 0; i < wave::Words<R>::n; ++i) wave::swap32(w2.w[i], w3.w[i]);
+            return w2.value() + w3.value();
+        };
+        q4<R> s{total(ax), total(ay), total(az), total(aw)};
+        if constexpr (W > 1) {
+            // two buffers by parity: the next write of this one comes after the next barrier
+            if (lane < 16) part[j & 1][wv][lane] = s;
+            __syncthreads();
+            s = part[j & 1][0][l16];
+#pragma unroll
+            for (int w = 1; w < W; ++w) s = add(s, part[j & 1][w][l16]);
+        }
+        const q4<R> p = scale(mul(t, s), R(-1));
+        int j1 = j;
+        asm volatile("" : "+s"(j1));  // keep the two passes' branches apart (apply_q_real_kernel)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+            if (block(q) + 63 > j1) {
+                const q4<R> a = v[q];
+                // x += a p (scalars.hpp, fma_ab)
+                rowop::axpy16(x[q].x, a.x, p.x);
+                rowop::axpy16(x[q].x, a.y, -p.y);
+                rowop::axpy16(x[q].x, a.z, -p.z);
+                rowop::axpy16(x[q].x, a.w, -p.w);
+                rowop::axpy16(x[q].y, a.x, p.y);
+                rowop::axpy16(x[q].y, a.y, p.x);
+                rowop::axpy16(x[q].y, a.z, -p.w);
+                rowop::axpy16(x[q].y, a.w, p.z);
+                rowop::axpy16(x[q].z, a.x, p.z);
+                rowop::axpy16(x[q].z, a.y, p.w);
+                rowop::axpy16(x[q].z, a.z, p.x);
+                rowop::axpy16(x[q].z, a.w, -p.y);
+                rowop::axpy16(x[q].w, a.x, p.w);
+                rowop::axpy16(x[q].w, a.y, -p.z);
+                rowop::axpy16(x[q].w, a.z, p.y);
+                rowop::axpy16(x[q].w, a.w, p.x);
+            }
+    }
+    const double* k = kpts + 3 * kk;
+    double sx = 0.0, sy = 0.0, sz = 0.0;
+    int ge = g16, ne = n;
+    asm volatile("" : "+v"(ge), "+s"(ne));  // recompute the rows' tests (apply_q_real_kernel)
+    T* xo = nullptr;
+    const bool second = !kRitz && 2 * b + 1 < nb;
+    if (X && live) xo = kRitz ? X + (kk * nbq + b) * (int64_t)n : X + (kk * nb + 2 * b) * (int64_t)(2 * n);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int i = block(q) + ge + r;
+            if (i < ne) {
+                const double ux = x[q].x[r], uy = x[q].y[r], dx = x[q].z[r], dy = x[q].w[r];
+                if (xo) {
+                    if constexpr (kRitz) {
+                        xo[i] = q4<double>{ux, uy, dx, dy};
+                    } else {
+                        xo[i] = make_double2(ux, uy);
+                        xo[n + i] = make_double2(dx, dy);
+                        if (second) {
+                            xo[2 * n + i] = make_double2(-dx, dy);
+                            xo[3 * n + i] = make_double2(ux, -uy);
+                        }
+                    }
+                }
+                if (grads) {
+                    const double w = (ux * ux + uy * uy) + (dx * dx + dy * dy);  // Hellmann-Feynman, kinetic term
+                    sx += (k[0] + (double)G[3 * i]) * w;
+                    sy += (k[1] + (double)G[3 * i + 1]) * w;
+                    sz += (k[2] + (double)G[3 * i + 2]) * w;
+                }
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (grads) {
+        for (int o = 16; o < 64; o <<= 1) {
+            sx += __shfl_xor(sx, o, 64);
+            sy += __shfl_xor(sy, o, 64);
+            sz += __shfl_xor(sz, o, 64);
+        }
+        if (g16 == 0) {
+            gsum[wv][l16][0] = sx;
+            gsum[wv][l16][1] = sy;
+            gsum[wv][l16][2] = sz;
+        }
+        __syncthreads();
+        if (threadIdx.x < 48) {
+            const int bb = threadIdx.x / 3, c = threadIdx.x % 3, level = 16 * blockIdx.y + bb;
+            double g = 0.0;
+#pragma unroll
+            for (int w = 0; w < W; ++w) g += gsum[w][bb][c];
+            g = g * P.grad_pref * P.frac_to_phys;
+            for (int u = 0; u < 2; ++u)
+                if (level < nbq && 2 * level + u < nb) grads[3 * (kk * nb + 2 * level + u) + c] = g;
+        }
+    }
+}
+
+namespace {
+template <typename R, typename T>
+hipError_t apply_q_quaternion(const q4<R>* dV, int n, const q4<R>* dtau, const double* dZ, int nbq, int nb, T* dX,
+                              double* dgrads, const DevParams& P, const double* dk, const int32_t* dG, int64_t nk,
+                              const int* kstat, unsigned long long* status, int64_t k0, hipStream_t s) {
+    const dim3 grid((unsigned)nk, (unsigned)((nbq + 15) / 16));
+    switch ((n + 63) / 64) {  // one wave per 64 rows
+        case 1:
+            hipLaunchKernelGGL((apply_q_quaternion_kernel<R, 1, 1, T>), grid, dim3(64), 0, s, dV, n, dtau, dZ, nbq, nb, dX,
+                               dgrads, P, dk, dG, kstat, status, k0);
+            break;
+        case 2:
+            hipLaunchKernelGGL((apply_q_quaternion_kernel<R, 2, 1, T>), grid, dim3(128), 0, s, dV, n, dtau, dZ, nbq, nb, dX,
+                               dgrads, P, dk, dG, kstat, status, k0);
+            break;
+        case 3:
+            hipLaunchKernelGGL((apply_q_quaternion_kernel<R, 3, 1, T>), grid, dim3(192), 0, s, dV, n, dtau, dZ, nbq, nb, dX,
+                               dgrads, P, dk, dG, kstat, status, k0);
+            break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_apply_q_quaternion_f32(const q4<float>* dV, int n, const q4<float>* dtau, const double* dZ, int nbq,
+                                         q4<double>* dX, int64_t nk, hipStream_t s) {
+    return apply_q_quaternion<float, q4<double>>(dV, n, dtau, dZ, nbq, 2 * nbq, dX, nullptr, DevParams{}, nullptr, nullptr,
+                                                 nk, nullptr, nullptr, 0, s);
+}
+hipError_t launch_apply_q_quaternion_f64(const q4<double>* dV, int n, const q4<double>* dtau, const double* dZ, int nb,
+                                         double2* dX, double* dgrads, const DevParams& P, const double* dk,
+                                         const int32_t* dG, int64_t nk, const int* kstat, unsigned long long* status,
+                                         int64_t k0, hipStream_t s) {
+    return apply_q_quaternion<double, double2>(dV, n, dtau, dZ, (nb + 1) / 2, nb, dX, dgrads, P, dk, dG, nk, kstat, status,
+                                               k0, s);
 }
 
 // ---------------------------------------------------------------------------

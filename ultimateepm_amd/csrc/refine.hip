@@ -18,6 +18,7 @@
 #include <cstdlib>
 
 #include "epm_physics.hpp"
+#include "scalars.hpp"
 #include "solver.hpp"
 
 namespace uepm {
@@ -694,76 +695,91 @@ __global__ __launch_bounds__(BS, 2) void refine_mfma2_kernel(const double2* __re
 // The same refinement for a real H(k) (and so real X0, Ritz vectors and small
 // problem): a quarter of the MFMAs, half the bytes.
 
-// The small real symmetric problem on nbr <= LDM Ritz vectors, in one wave, as
-// small_rayleigh_ritz does it: Cholesky S = L L^T, M' = L^-1 M L^-T, round-robin
-// Jacobi M' = Z Theta Z^T, C = L^-T Z (in Wt), Ritz values th and the order perm.
-template <int LDM>
-__device__ bool small_rayleigh_ritz_real(int nbr, double* __restrict__ Ss, double* __restrict__ Mm,
-                                         double* __restrict__ Zm, double* __restrict__ Wt, double* __restrict__ th,
-                                         int* __restrict__ perm, double2* __restrict__ rot, int lane) {
+// The small Hermitian problem on nbr <= LDM Ritz vectors over S = r1<double> or
+// q4<double>, in one wave, as small_rayleigh_ritz does it: Cholesky S = L L^H, M' =
+// L^-1 M L^-H, round-robin Jacobi M' = Z Theta Z^H, C = L^-H Z (in Wt), Ritz values
+// th and the order perm.  Products keep their order (quaternions).
+template <int LDM, typename S>
+__device__ bool small_rayleigh_ritz_of(int nbr, S* __restrict__ Ss, S* __restrict__ Mm, S* __restrict__ Zm,
+                                       S* __restrict__ Wt, double* __restrict__ th, int* __restrict__ perm,
+                                       double2* __restrict__ rot, S* __restrict__ phase, int lane) {
     const int i = lane;
+    const S zero{}, one = sc_real<S>(1.0);
+    auto csub = [](S acc, S a, S b) {  // acc - a b
+        fma_ab(acc, scale(a, -1.0), b);
+        return acc;
+    };
     for (int j = 0; j < nbr; ++j) {
-        const double ljj = sqrt(Ss[j * LDM + j]);
+        const double ljj = sqrt(Ss[j * LDM + j].x);
         const double rl = 1.0 / ljj;
         wsync();
-        if (i > j && i < nbr) Ss[i * LDM + j] *= rl;
-        if (i == 0) Ss[j * LDM + j] = ljj;
+        if (i > j && i < nbr) Ss[i * LDM + j] = scale(Ss[i * LDM + j], rl);
+        if (i == 0) Ss[j * LDM + j] = sc_real<S>(ljj);
         wsync();
         for (int e = i; e < LDM * LDM; e += 64) {
             const int r = e / LDM, c = e % LDM;
-            if (c > j && r >= c && r < nbr) Ss[r * LDM + c] -= Ss[r * LDM + j] * Ss[c * LDM + j];
+            if (c > j && r >= c && r < nbr)
+                Ss[r * LDM + c] = csub(Ss[r * LDM + c], Ss[r * LDM + j], conj_if(Ss[c * LDM + j], true));
         }
         wsync();
     }
-    // Wt = L^-1 M (lane = column of M), then U = L^-1 Wt^T (lane = row of Wt): M' = U^T.
-    // Columns stay in registers; a row's terms are subtracted in ascending order.
-    auto lower = [&](double (&v)[LDM]) {
+    // Wt = L^-1 M (lane = column of M), then U = L^-1 Wt^H (lane = row of Wt): M' = U^H.
+    // A row's terms are subtracted in ascending order; a real column stays in registers.
+    auto lower = [&](auto get, auto put) {
+        if constexpr (S::NC == 1) {
+            S v[LDM];
 #pragma unroll
-        for (int r = 0; r < LDM; ++r)
-            if (r < nbr) {
-                double s = v[r];
+            for (int r = 0; r < LDM; ++r)
+                if (r < nbr) {
+                    S t = get(r);
 #pragma unroll
-                for (int k = 0; k < r; ++k) s = fma(-Ss[r * LDM + k], v[k], s);
-                v[r] = s * (1.0 / Ss[r * LDM + r]);
-            }
-    };
-    if (i < nbr) {
-        double v[LDM];
-#pragma unroll
-        for (int r = 0; r < LDM; ++r) v[r] = r < nbr ? Mm[r * LDM + i] : 0.0;
-        lower(v);
-#pragma unroll
-        for (int r = 0; r < LDM; ++r)
-            if (r < nbr) Wt[r * LDM + i] = v[r];
-    }
-    wsync();
-    if (i < nbr) {
-        double v[LDM];
-#pragma unroll
-        for (int r = 0; r < LDM; ++r) v[r] = r < nbr ? Wt[i * LDM + r] : 0.0;
-        lower(v);
-#pragma unroll
-        for (int c = 0; c < LDM; ++c)
-            if (c < nbr) {
-                Mm[i * LDM + c] = v[c];
-                Zm[i * LDM + c] = i == c ? 1.0 : 0.0;
-            }
-    }
-    wsync();
-    if (i < nbr)
-        for (int c = i + 1; c < nbr; ++c) {  // symmetrise
-            const double h = 0.5 * (Mm[i * LDM + c] + Mm[c * LDM + i]);
-            Mm[i * LDM + c] = h;
-            Mm[c * LDM + i] = h;
+                    for (int k = 0; k < r; ++k) t = csub(t, Ss[r * LDM + k], v[k]);
+                    v[r] = scale(t, 1.0 / Ss[r * LDM + r].x);
+                    put(r, v[r]);
+                }
         }
+    };
+    if constexpr (S::NC == 1) {
+        if (i < nbr) lower([&](int r) { return Mm[r * LDM + i]; }, [&](int r, S v) { Wt[r * LDM + i] = v; });
+        wsync();
+        if (i < nbr) lower([&](int r) { return Wt[i * LDM + r]; }, [&](int r, S v) { Mm[i * LDM + r] = v; });
+    } else {
+        if (i < nbr)
+            for (int r = 0; r < nbr; ++r) {
+                S t = Mm[r * LDM + i];
+                for (int k = 0; k < r; ++k) t = csub(t, Ss[r * LDM + k], Wt[k * LDM + i]);
+                Wt[r * LDM + i] = scale(t, 1.0 / Ss[r * LDM + r].x);
+            }
+        wsync();
+        if (i < nbr)
+            for (int r = 0; r < nbr; ++r) {
+                S t = conj_if(Wt[i * LDM + r], true);
+                for (int k = 0; k < r; ++k) t = csub(t, Ss[r * LDM + k], Zm[k * LDM + i]);
+                Zm[r * LDM + i] = scale(t, 1.0 / Ss[r * LDM + r].x);
+            }
+        wsync();
+        if (i < nbr)
+            for (int c = 0; c < nbr; ++c) Mm[i * LDM + c] = conj_if(Zm[c * LDM + i], true);
+    }
+    wsync();
+    if (i < nbr) {
+        for (int c = 0; c < nbr; ++c) Zm[i * LDM + c] = i == c ? one : zero;
+        for (int c = i + 1; c < nbr; ++c) {  // hermitise
+            const S h = scale(add(Mm[i * LDM + c], conj_if(Mm[c * LDM + i], true)), 0.5);
+            Mm[i * LDM + c] = h;
+            Mm[c * LDM + i] = conj_if(h, true);
+        }
+        Mm[i * LDM + i] = sc_real<S>(Mm[i * LDM + i].x);
+    }
     wsync();
     // the rotation test, the rounds and the stopping rules of small_rayleigh_ritz
     const int m = (nbr + 1) & ~1, half = m >> 1;
     auto negligible = [&](int p, int q) {
-        const double ac = fabs(Mm[p * LDM + q]);
-        const double a = Mm[p * LDM + p], b = Mm[q * LDM + q];
-        const double scale = fabs(a) + fabs(b) + 1e-300;
-        return ac <= 1e-15 * scale || ac * ac <= 1e-13 * scale * fabs(b - a);
+        const S c = Mm[p * LDM + q];
+        const double c2v = dot_acc(c, c, 0.0);
+        const double a = Mm[p * LDM + p].x, b = Mm[q * LDM + q].x;
+        const double scale_ = fabs(a) + fabs(b) + 1e-300;
+        return c2v <= 1e-30 * scale_ * scale_ || c2v <= 1e-13 * scale_ * fabs(b - a);
     };
     auto all_negligible = [&]() {
         bool big = false;
@@ -790,21 +806,25 @@ __device__ bool small_rayleigh_ritz_real(int nbr, double* __restrict__ Ss, doubl
             if (i < half) {
                 int p = elem(i), q = elem(m - 1 - i);
                 if (p > q) { const int t = p; p = q; q = t; }
-                double2 g = make_double2(1.0, 0.0);  // cs, sn with the element's sign
+                double2 g = make_double2(1.0, 0.0);  // cs, sn
+                S ph = one;                          // conj(c) / |c|, c the pair's element (a sign when real)
                 if (q < nbr && !negligible(p, q)) {
                     did = true;
-                    const double c = Mm[p * LDM + q];
-                    const double tau_ = (Mm[q * LDM + q] - Mm[p * LDM + p]) / (2.0 * c);
+                    const S c = Mm[p * LDM + q];
+                    const double ac = sqrt(dot_acc(c, c, 0.0));
+                    ph = scale(conj_if(c, true), 1.0 / ac);
+                    const double tau_ = (Mm[q * LDM + q].x - Mm[p * LDM + p].x) / (2.0 * ac);
                     const double t = (tau_ >= 0 ? 1.0 : -1.0) / (fabs(tau_) + sqrt(1.0 + tau_ * tau_));
                     const double cs = 1.0 / sqrt(1.0 + t * t);
                     g = make_double2(cs, t * cs);
                 }
                 rot[i] = g;
+                phase[i] = ph;
             }
             wsync();
             if (__any(did)) {
                 rotated = true;
-                // columns: M <- M G, Z <- Z G with G = [[cs, sn], [-sn, cs]] on (p, q)
+                // columns: M <- M G, Z <- Z G with G = [[cs, sn], [-ph sn, ph cs]] on (p, q)
                 for (int task = i; task < half * LDM; task += 64) {
                     const int k = task / LDM, row = task % LDM;
                     if (row >= nbr) continue;
@@ -812,15 +832,16 @@ __device__ bool small_rayleigh_ritz_real(int nbr, double* __restrict__ Ss, doubl
                     if (p > q) { const int t = p; p = q; q = t; }
                     if (q >= nbr) continue;
                     const double2 g = rot[k];
-                    const double mp = Mm[row * LDM + p], mq = Mm[row * LDM + q];
-                    Mm[row * LDM + p] = mp * g.x - mq * g.y;
-                    Mm[row * LDM + q] = mp * g.y + mq * g.x;
-                    const double zp = Zm[row * LDM + p], zq = Zm[row * LDM + q];
-                    Zm[row * LDM + p] = zp * g.x - zq * g.y;
-                    Zm[row * LDM + q] = zp * g.y + zq * g.x;
+                    const S ph = phase[k];
+                    const S mp = Mm[row * LDM + p], mq = mul(Mm[row * LDM + q], ph);
+                    Mm[row * LDM + p] = axpy(-g.y, mq, scale(mp, g.x));
+                    Mm[row * LDM + q] = axpy(g.y, mp, scale(mq, g.x));
+                    const S zp = Zm[row * LDM + p], zq = mul(Zm[row * LDM + q], ph);
+                    Zm[row * LDM + p] = axpy(-g.y, zq, scale(zp, g.x));
+                    Zm[row * LDM + q] = axpy(g.y, zp, scale(zq, g.x));
                 }
                 wsync();
-                // rows: M <- G^T M
+                // rows: M <- G^H M
                 for (int task = i; task < half * LDM; task += 64) {
                     const int k = task / LDM, col = task % LDM;
                     if (col >= nbr) continue;
@@ -828,12 +849,20 @@ __device__ bool small_rayleigh_ritz_real(int nbr, double* __restrict__ Ss, doubl
                     if (p > q) { const int t = p; p = q; q = t; }
                     if (q >= nbr) continue;
                     const double2 g = rot[k];
-                    const double rp = Mm[p * LDM + col], rq = Mm[q * LDM + col];
-                    // the rotated pair's own off-diagonal element is zero by construction
-                    const bool own = g.y != 0.0 && (col == p || col == q);
-                    const double np = rp * g.x - rq * g.y, nq = rp * g.y + rq * g.x;
-                    Mm[p * LDM + col] = own && col == q ? 0.0 : np;
-                    Mm[q * LDM + col] = own && col == p ? 0.0 : nq;
+                    const S rp = Mm[p * LDM + col], rq = mul(conj_if(phase[k], true), Mm[q * LDM + col]);
+                    S np = axpy(-g.y, rq, scale(rp, g.x)), nq = axpy(g.y, rp, scale(rq, g.x));
+                    if (g.y != 0.0) {
+                        // a rotated pair's own off-diagonal element is zero and its diagonal real by construction
+                        if (col == p) {
+                            np = sc_real<S>(np.x);
+                            nq = zero;
+                        } else if (col == q) {
+                            np = zero;
+                            nq = sc_real<S>(nq.x);
+                        }
+                    }
+                    Mm[p * LDM + col] = np;
+                    Mm[q * LDM + col] = nq;
                 }
                 wsync();
             }
@@ -845,24 +874,28 @@ __device__ bool small_rayleigh_ritz_real(int nbr, double* __restrict__ Ss, doubl
     }
     if (!converged) converged = all_negligible();
     wsync();
-    // C = L^-T Z (back substitution, lane = column of Z)
+    // C = L^-H Z (back substitution, lane = column of Z)
     if (i < nbr) {
-        double v[LDM];
+        if constexpr (S::NC == 1) {
+            S v[LDM];
 #pragma unroll
-        for (int r = 0; r < LDM; ++r) v[r] = r < nbr ? Zm[r * LDM + i] : 0.0;
+            for (int r = LDM - 1; r >= 0; --r)
+                if (r < nbr) {
+                    S t = Zm[r * LDM + i];
 #pragma unroll
-        for (int r = LDM - 1; r >= 0; --r)
-            if (r < nbr) {
-                double s = v[r];
-#pragma unroll
-                for (int k = r + 1; k < LDM; ++k)
-                    if (k < nbr) s = fma(-Ss[k * LDM + r], v[k], s);
-                v[r] = s * (1.0 / Ss[r * LDM + r]);
+                    for (int k = r + 1; k < LDM; ++k)
+                        if (k < nbr) t = csub(t, conj_if(Ss[k * LDM + r], true), v[k]);
+                    v[r] = scale(t, 1.0 / Ss[r * LDM + r].x);
+                    Wt[r * LDM + i] = v[r];
+                }
+        } else {
+            for (int r = nbr - 1; r >= 0; --r) {
+                S t = Zm[r * LDM + i];
+                for (int k = r + 1; k < nbr; ++k) t = csub(t, conj_if(Ss[k * LDM + r], true), Wt[k * LDM + i]);
+                Wt[r * LDM + i] = scale(t, 1.0 / Ss[r * LDM + r].x);
             }
-#pragma unroll
-        for (int r = 0; r < LDM; ++r)
-            if (r < nbr) Wt[r * LDM + i] = v[r];
-        th[i] = Mm[i * LDM + i];
+        }
+        th[i] = Mm[i * LDM + i].x;
         perm[i] = i;
     }
     wsync();
@@ -897,6 +930,7 @@ __global__ __launch_bounds__(BS, NT == 1 ? 4 : 3) void refine_real_kernel(
     __shared__ double th[LDM];
     __shared__ int perm[LDM];
     __shared__ double2 rot[LDM / 2 + 1];
+    __shared__ r1<double> phase[LDM / 2 + 1];
     __shared__ double red[3 * 8 * NW];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int l16 = lane & 15, l4 = lane >> 4;
@@ -997,7 +1031,10 @@ __global__ __launch_bounds__(BS, NT == 1 ? 4 : 3) void refine_real_kernel(
     }
     __syncthreads();  // the partial slots are free from here: Z and W take their place
     if (wv == 0) {
-        const bool conv = small_rayleigh_ritz_real<LDM>(nbr, Ss, Mm, Zm, Wt, th, perm, rot, lane);
+        using S = r1<double>;
+        const bool conv = small_rayleigh_ritz_of<LDM, S>(nbr, reinterpret_cast<S*>(Ss), reinterpret_cast<S*>(Mm),
+                                                         reinterpret_cast<S*>(Zm), reinterpret_cast<S*>(Wt), th, perm, rot,
+                                                         phase, lane);
         report_ritz_status(kstat, status, k0, kk, nb, th, perm, conv, lane);
     }
     __syncthreads();
@@ -1071,6 +1108,199 @@ hipError_t launch_refine_real(const double* dH, int n, const double* dX, int nbr
     else
         hipLaunchKernelGGL((refine_real_kernel<kRefBS, 2>), dim3((unsigned)nk), dim3(kRefBS), 0, s, dH, n, dX, nbr, nb,
                            devals, devecs, dgrads, P, dk, dG, kstat, status, k0);
+    return hipGetLastError();
+}
+
+// The same refinement for a quaternion H(k), N x N, and m <= 16 quaternion Ritz
+// vectors, each a Kramers pair: S, M and the small problem are m x m.  On FP64
+// MFMA the quaternion product is sixteen real ones; the layout is
+// refine_mfma_kernel's, four components wide.
+template <int BS>
+__global__ __launch_bounds__(BS, 2) void refine_quaternion_kernel(
+    const q4<double>* __restrict__ H, int n, const q4<double>* __restrict__ Xall, int m, int nb,
+    double* __restrict__ evals, double2* __restrict__ evecs, double* __restrict__ grads, DevParams P,
+    const double* __restrict__ kpts, const int32_t* __restrict__ G, const int* __restrict__ kstat,
+    unsigned long long* __restrict__ status, int64_t k0) {
+    using Q = q4<double>;
+    constexpr int NW = BS / 64, LDM = 16, KU = 4;
+    // per-wave partials in turn (one slot), then Z and W
+    __shared__ __align__(32) double part[2][4][16][16];
+    __shared__ Q Mm[LDM * LDM], Ss[LDM * LDM], Wt[LDM * LDM];
+    static_assert(sizeof(part) >= LDM * LDM * sizeof(Q), "Z fits in the partial slot");
+    Q* Zm = reinterpret_cast<Q*>(&part[0][0][0][0]);
+    __shared__ double th[LDM];
+    __shared__ int perm[LDM];
+    __shared__ double2 rot[LDM / 2 + 1];
+    __shared__ Q phase[LDM / 2 + 1];
+    __shared__ double red[3 * 4 * NW];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int l16 = lane & 15, l4 = lane >> 4;
+    const int64_t kk = blockIdx.x;
+    const Q* A = H + kk * (int64_t)n * n;
+    const Q* X = Xall + kk * (int64_t)m * n;  // X[b * n + r]
+    const double bm = l16 < m ? 1.0 : 0.0;
+    const Q* Xb = X + (l16 < m ? l16 : 0) * (int64_t)n;
+    struct Acc {
+        dbl4 x, y, z, w;
+    };
+    // acc += (conj)a b, component by component (scalars.hpp, fma_ab and fma_cab)
+    auto mac = [](Acc& c, const Q& a, const Q& b) {
+        c.x = mfma64(a.x, b.x, c.x);
+        c.x = mfma64(-a.y, b.y, c.x);
+        c.x = mfma64(-a.z, b.z, c.x);
+        c.x = mfma64(-a.w, b.w, c.x);
+        c.y = mfma64(a.x, b.y, c.y);
+        c.y = mfma64(a.y, b.x, c.y);
+        c.y = mfma64(-a.z, b.w, c.y);
+        c.y = mfma64(a.w, b.z, c.y);
+        c.z = mfma64(a.x, b.z, c.z);
+        c.z = mfma64(a.y, b.w, c.z);
+        c.z = mfma64(a.z, b.x, c.z);
+        c.z = mfma64(-a.w, b.y, c.z);
+        c.w = mfma64(a.x, b.w, c.w);
+        c.w = mfma64(-a.y, b.z, c.w);
+        c.w = mfma64(a.z, b.y, c.w);
+        c.w = mfma64(a.w, b.x, c.w);
+    };
+    const dbl4 z4 = {0, 0, 0, 0};
+    Acc sa{z4, z4, z4, z4}, ma{z4, z4, z4, z4};
+    const int ntile = (n + 15) >> 4;
+    for (int t = wv; t < ntile; t += NW) {
+        const int row = 16 * t + l16;
+        const Q* Ar = A + (row < n ? row : n - 1);
+        const double mrow = row < n ? 1.0 : 0.0;
+        Acc y{z4, z4, z4, z4};
+        for (int c0 = 0; c0 < n; c0 += 4 * KU) {
+            Q h[KU], x[KU];
+#pragma unroll
+            for (int u = 0; u < KU; ++u) {
+                const int col = c0 + 4 * u + l4, cc = col < n ? col : n - 1;
+                const double mc = col < n ? 1.0 : 0.0;
+                h[u] = scale(Ar[(int64_t)cc * n], mrow * mc);
+                x[u] = scale(Xb[cc], bm * mc);
+            }
+#pragma unroll
+            for (int u = 0; u < KU; ++u) mac(y, h[u], x[u]);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = 16 * t + 4 * v + l4;
+            const Q x = scale(Xb[r < n ? r : n - 1], r < n ? bm : 0.0);
+            const Q xc = conj_if(x, true);
+            mac(sa, xc, x);
+            mac(ma, xc, Q{y.x[v], y.y[v], y.z[v], y.w[v]});
+        }
+    }
+    for (int rd = 0; rd < NW; ++rd) {
+        if (wv == rd) {
+            const dbl4 vals[2][4] = {{sa.x, sa.y, sa.z, sa.w}, {ma.x, ma.y, ma.z, ma.w}};
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        double& to = part[f][c][4 * v + l4][l16];
+                        to = rd == 0 ? vals[f][c][v] : to + vals[f][c][v];
+                    }
+        }
+        __syncthreads();
+    }
+    static_assert(BS == 256, "one (a, b) entry of S and M per thread");
+    {
+        const int a = tid >> 4, b = tid & 15;
+        if (a < m && b < m) {
+            Ss[a * LDM + b] = Q{part[0][0][a][b], part[0][1][a][b], part[0][2][a][b], part[0][3][a][b]};
+            Mm[a * LDM + b] = Q{part[1][0][a][b], part[1][1][a][b], part[1][2][a][b], part[1][3][a][b]};
+        }
+    }
+    __syncthreads();  // the partial slot is free from here: Z takes its place
+    // levels of the nb bands asked for; the small problem's Ritz values are one per pair
+    const int nlev = (nb + 1) / 2;
+    if (wv == 0) {
+        const bool conv = small_rayleigh_ritz_of<LDM, Q>(m, Ss, Mm, Zm, Wt, th, perm, rot, phase, lane);
+        report_ritz_status(kstat, status, k0, kk, nlev, th, perm, conv, lane);
+    }
+    __syncthreads();
+    if (tid < nb) evals[kk * nb + tid] = th[perm[tid >> 1]];
+    if (!evecs && !grads) return;
+    // X1 = X0 C[:, perm[b]], four levels a pass, one thread per row; each level's spinor
+    // (u; d) and its partner (-conj(d); conj(u))
+    constexpr int BC = 4;
+    double2* out = evecs ? evecs + kk * (int64_t)nb * (2 * n) : nullptr;
+    const double* k = kpts + 3 * kk;
+    for (int b0 = 0; b0 < nlev; b0 += BC) {
+        double gx[BC], gy[BC], gz[BC];
+#pragma unroll
+        for (int u = 0; u < BC; ++u) gx[u] = gy[u] = gz[u] = 0.0;
+        for (int r = tid; r < n; r += BS) {
+            Q acc[BC];
+#pragma unroll
+            for (int u = 0; u < BC; ++u) acc[u] = Q{};
+            for (int a = 0; a < m; ++a) {
+                const Q x = X[a * n + r];
+#pragma unroll
+                for (int u = 0; u < BC; ++u)
+                    if (b0 + u < nlev) fma_ab(acc[u], x, Wt[a * LDM + perm[b0 + u]]);
+            }
+#pragma unroll
+            for (int u = 0; u < BC; ++u)
+                if (b0 + u < nlev) {
+                    const Q q = acc[u];
+                    if (out) {
+                        double2* to = out + (int64_t)(2 * (b0 + u)) * (2 * n) + r;
+                        to[0] = make_double2(q.x, q.y);
+                        to[n] = make_double2(q.z, q.w);
+                        if (2 * (b0 + u) + 1 < nb) {
+                            to[2 * n] = make_double2(-q.z, q.w);
+                            to[3 * n] = make_double2(q.x, -q.y);
+                        }
+                    }
+                    if (grads) {
+                        const double wt = dot_acc(q, q, 0.0);  // Hellmann-Feynman, kinetic term
+                        gx[u] += (k[0] + (double)G[3 * r]) * wt;
+                        gy[u] += (k[1] + (double)G[3 * r + 1]) * wt;
+                        gz[u] += (k[2] + (double)G[3 * r + 2]) * wt;
+                    }
+                }
+        }
+        if (grads) {
+#pragma unroll
+            for (int u = 0; u < BC; ++u)
+                for (int o = 32; o > 0; o >>= 1) {
+                    gx[u] += __shfl_xor(gx[u], o, 64);
+                    gy[u] += __shfl_xor(gy[u], o, 64);
+                    gz[u] += __shfl_xor(gz[u], o, 64);
+                }
+            if (lane == 0)
+#pragma unroll
+                for (int u = 0; u < BC; ++u) {
+                    red[(wv * BC + u) * 3 + 0] = gx[u];
+                    red[(wv * BC + u) * 3 + 1] = gy[u];
+                    red[(wv * BC + u) * 3 + 2] = gz[u];
+                }
+            __syncthreads();
+            if (tid < 3 * 2 * BC) {
+                const int band = 2 * b0 + tid / 3, u = tid / 6, c = tid % 3;
+                if (band < nb) {
+                    double sum = 0.0;
+#pragma unroll
+                    for (int w = 0; w < NW; ++w) sum += red[(w * BC + u) * 3 + c];
+                    grads[3 * (kk * nb + band) + c] = sum * P.grad_pref * P.frac_to_phys;
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
+hipError_t launch_refine_quaternion(const q4<double>* dH, int n, const q4<double>* dX, int m, int nb, double* devals,
+                                    double2* devecs, double* dgrads, const DevParams& P, const double* dk,
+                                    const int32_t* dG, int64_t nk, const int* kstat, unsigned long long* status, int64_t k0,
+                                    hipStream_t s) {
+    if (m > 16 || nb > 2 * m) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(refine_quaternion_kernel<kRefBS>, dim3((unsigned)nk), dim3(kRefBS), 0, s, dH, n, dX, m, nb, devals,
+                       devecs, dgrads, P, dk, dG, kstat, status, k0);
     return hipGetLastError();
 }
 

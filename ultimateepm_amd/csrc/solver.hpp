@@ -6,6 +6,7 @@
 #include <cstdint>
 
 #include "epm_physics.hpp"
+#include "scalars.hpp"
 
 namespace uepm {
 
@@ -35,6 +36,9 @@ hipError_t launch_assemble(const DevParams& P, const int32_t* dG, const double* 
 // The real parts alone (nk x n x n doubles), for a plan whose H(k) is real.
 hipError_t launch_assemble_real(const DevParams& P, const int32_t* dG, const double* dk, int64_t nk, double* dH, int ld,
                                 hipStream_t s);
+// The quaternion form (nk x N x N) of a spin-orbit plan of equal atoms.
+hipError_t launch_assemble_quaternion(const DevParams& P, const int32_t* dG, const double* dk, int64_t nk, q4<double>* dH,
+                                      int ld, hipStream_t s);
 // Failure reporting.  A solve's device status is two words: the number of
 // k-points whose eigen-solve failed and the lowest index among them (all ones
 // when none); launch_status_reset clears it.  Inside a chunk, kstat (one int
@@ -63,6 +67,13 @@ hipError_t launch_refine(const double2* dH, int n, int ld, double2* dX, int nbr,
 hipError_t launch_refine_real(const double* dH, int n, const double* dX, int nbr, int nb, double* devals, double2* devecs,
                               double* dgrads, const DevParams& P, const double* dk, const int32_t* dG, int64_t nk,
                               const int* kstat, unsigned long long* status, int64_t k0, hipStream_t s);
+
+// launch_refine for a quaternion H (nk x n x n) and m quaternion vectors (nk x m x n,
+// read only), each a Kramers pair of the nb <= 2 m bands written.
+hipError_t launch_refine_quaternion(const q4<double>* dH, int n, const q4<double>* dX, int m, int nb, double* devals,
+                                    double2* devecs, double* dgrads, const DevParams& P, const double* dk,
+                                    const int32_t* dG, int64_t nk, const int* kstat, unsigned long long* status, int64_t k0,
+                                    hipStream_t s);
 
 // Name of the refinement kernel launch_refine runs for nbr Ritz vectors.
 const char* refine_kernel_name(int nbr);
@@ -111,6 +122,17 @@ hipError_t launch_tridiag_real_f32(const double* dH, int n, int64_t nk, float* V
 hipError_t launch_tridiag_real_f64(const double* dH, int n, int64_t nk, double* V, double* dd, double* de, double* dtau,
                                    double* work, hipStream_t s);
 
+// The same for a quaternion H (n x n per k-point, n <= tridiag_quaternion_max_n): T
+// is n x n and holds each Kramers pair's level once.
+int tridiag_quaternion_max_n(bool f32);
+size_t tridiag_quaternion_work_bytes(int n, bool f32);
+hipError_t launch_tridiag_quaternion_f32(const q4<double>* dH, int n, int64_t nk, q4<float>* V, double* dd, double* de,
+                                         q4<float>* dtau, q4<float>* work, hipStream_t s);
+hipError_t launch_tridiag_quaternion_f64(const q4<double>* dH, int n, int64_t nk, q4<double>* V, double* dd, double* de,
+                                         q4<double>* dtau, q4<double>* work, hipStream_t s);
+// Kramers pairs: devals[k][b] = levels[k][b / 2], b < nb ((nb + 1) / 2 levels per k).
+hipError_t launch_pair_levels(const double* levels, int nb, int64_t nk, double* devals, hipStream_t s);
+
 // Eigenvectors of H from those of T: cluster re-orthogonalisation of Z
 // ([k][band][row], n x nb per k), then x = Q z with the reflectors of the
 // reduction (FP64: over H; precision form: complex64 Vout), gradients when dgrads.
@@ -141,6 +163,16 @@ hipError_t launch_apply_q_real_f32(const float* dV, int n, const float* dtau, co
 hipError_t launch_apply_q_real_f64(const double* dV, int n, const double* dtau, const double* dZ, int nb, double2* dX,
                                    double* dgrads, const DevParams& P, const double* dk, const int32_t* dG, int64_t nk,
                                    const int* kstat, unsigned long long* status, int64_t k0, hipStream_t s);
+
+// x = Q z with quaternion reflectors: the Ritz basis (nk x nbq x n), or the FP64
+// form's spinor eigenvectors (nk x nb x 2n: bands 2 b' and 2 b' + 1 of level b') and
+// gradients, as launch_apply_q_real_f64.
+hipError_t launch_apply_q_quaternion_f32(const q4<float>* dV, int n, const q4<float>* dtau, const double* dZ, int nbq,
+                                         q4<double>* dX, int64_t nk, hipStream_t s);
+hipError_t launch_apply_q_quaternion_f64(const q4<double>* dV, int n, const q4<double>* dtau, const double* dZ, int nb,
+                                         double2* dX, double* dgrads, const DevParams& P, const double* dk,
+                                         const int32_t* dG, int64_t nk, const int* kstat, unsigned long long* status,
+                                         int64_t k0, hipStream_t s);
 
 // Device-to-device copy (16-byte aligned pointers take the vector path).
 hipError_t launch_copy_bytes(void* dst, const void* src, uint64_t bytes, int num_cus, hipStream_t s);

@@ -340,6 +340,17 @@ hipError_t launch_tri_eig(const double* dd, const double* de, int n, int nb, int
     return hipGetLastError();
 }
 
+__global__ void pair_levels_kernel(const double* __restrict__ levels, int nb, int64_t n, double* __restrict__ evals) {
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (t < n) evals[t] = levels[t / nb * ((nb + 1) / 2) + t % nb / 2];
+}
+
+hipError_t launch_pair_levels(const double* levels, int nb, int64_t nk, double* devals, hipStream_t s) {
+    const int64_t n = nk * nb;
+    hipLaunchKernelGGL(pair_levels_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, levels, nb, n, devals);
+    return hipGetLastError();
+}
+
 // status[0] = 0 failed k-points, status[1] = no first index (a kernel node, so
 // that a solve captured into a graph clears it on every replay)
 __global__ void status_reset_kernel(unsigned long long* status) {

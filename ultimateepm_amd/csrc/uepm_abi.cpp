@@ -89,6 +89,24 @@ Sizes plan_sizes(const uepm_plan* p, int64_t chunk) {
         z.kstat = sizeof(int) * (size_t)chunk;
         return z;
     }
+    if (p->quat) {
+        // N x N quaternions; vectors and T are one per Kramers pair
+        const int N = p->N, m = (nbr + 1) / 2;
+        const size_t r = 4 * (mixed ? sizeof(float) : sizeof(double));
+        z.d = z.e = sizeof(double) * (size_t)N * chunk;
+        z.H = 4 * sizeof(double) * (size_t)N * N * chunk;
+        z.Vf = r * (size_t)N * N * chunk;
+        z.tauf = r * (size_t)N * chunk;
+        z.S32 = uepm::tridiag_quaternion_work_bytes(N, mixed) * chunk;
+        z.Ev = sizeof(double) * (size_t)m * chunk;
+        if (mixed) z.X0 = 4 * sizeof(double) * (size_t)N * m * chunk;
+        if (stage_vec) {
+            z.Z = sizeof(double) * (size_t)N * m * chunk;
+            z.W = sizeof(double) * 4 * (size_t)N * m * chunk;
+        }
+        z.kstat = sizeof(int) * (size_t)chunk;
+        return z;
+    }
     z.H = sizeof(double2) * (size_t)n * n * chunk;
     z.tau = sizeof(double2) * (size_t)n * chunk;
     if (mixed) {
@@ -194,6 +212,11 @@ void plan_apply_config(uepm_plan* p) {
     // two equal non-local terms), so the real kernels take the plan.  Si N = 181, 12
     // bands and vectors: precision form 29.1 -> 15.1 ms per 16,001 k-points, FP64
     // 22.1 -> 7.9 ms per 6,000.
+    // With spin-orbit the same crystal's H(k) is a quaternion matrix of half the
+    // dimension, and every level a Kramers pair found once: Ge, dim 274, 16 bands,
+    // precision form 19.7 -> 9.2 ms per 3,000 k-points, FP64 18.3 -> 5.0 ms per 961.
+    p->quat = p->inversion && (p->flags & UEPM_SOC) && p->soc_symmetric && p->cfg.tridiag != 1 &&
+              p->N <= uepm::tridiag_quaternion_max_n(mixed);
     p->real = p->inversion && !(p->flags & UEPM_SOC) && p->cfg.tridiag != 1 && p->dim <= uepm::tridiag_real_max_n(mixed);
     const int bs = p->cfg.tri_block == 256 ? 256 : 512;
     p->tp = uepm::tri_plan(p->dim, (int)sizeof(double2), p->ctx->lds_limit, bs);
@@ -288,6 +311,12 @@ int solve_chunks(uepm_plan* p, const double* dk, int64_t nk, double* devals, dou
         p->stage_name[kBack] = mixed ? "cluster_orth+apply_q_real_kernel<f32>" : "cluster_orth+apply_q_real_kernel<f64>";
         p->stage_name[kRefine] = "refine_real_kernel";
     }
+    if (p->quat) {
+        p->stage_name[kTridiag] = mixed ? "tridiag_quaternion<f32>" : "tridiag_quaternion<f64>";
+        p->stage_name[kBack] = mixed ? "cluster_orth+apply_q_quaternion_kernel<f32>"
+                                     : "cluster_orth+apply_q_quaternion_kernel<f64>";
+        p->stage_name[kRefine] = "refine_quaternion_kernel";
+    }
     // the chunks; on an error the side stream is still joined into the caller's
     auto run_chunks = [&]() -> int {
         for (int ci = 0; ci < nchunks; ++ci) {
@@ -340,6 +369,51 @@ int solve_chunks(uepm_plan* p, const double* dk, int64_t nk, double* devals, dou
                 HIP_OK(rec(ci, kRefine, 0));
                 HIP_OK(uepm::launch_refine_real(Hr, n, reinterpret_cast<double*>(w.X0), nbr, nb, devals + c0 * nb, Xc, gc,
                                                 p->P, kc, p->G.as<int32_t>(), c, ks, status, c0, cs));
+                HIP_OK(rec(ci, kRefine, 1));
+                continue;
+            }
+            if (p->quat) {
+                // the stages below in quaternion arithmetic, one vector per Kramers pair
+                const int N = p->N, m = (nbr + 1) / 2;
+                auto* Hq = reinterpret_cast<uepm::q4<double>*>(w.H);
+                auto* Vq32 = reinterpret_cast<uepm::q4<float>*>(w.Vf);
+                auto* Vq64 = reinterpret_cast<uepm::q4<double>*>(w.Vf);
+                auto* tq32 = reinterpret_cast<uepm::q4<float>*>(w.tauf);
+                auto* tq64 = reinterpret_cast<uepm::q4<double>*>(w.tauf);
+                auto* Xq = reinterpret_cast<uepm::q4<double>*>(w.X0);
+                HIP_OK(rec(ci, kAssemble, 0));
+                HIP_OK(uepm::launch_assemble_quaternion(p->P, p->G.as<int32_t>(), kc, c, Hq, N, cs));
+                HIP_OK(rec(ci, kAssemble, 1));
+                HIP_OK(rec(ci, kTridiag, 0));
+                if (mixed)
+                    HIP_OK(uepm::launch_tridiag_quaternion_f32(Hq, N, c, Vq32, w.d, w.e, tq32,
+                                                               reinterpret_cast<uepm::q4<float>*>(w.S32), cs));
+                else
+                    HIP_OK(uepm::launch_tridiag_quaternion_f64(Hq, N, c, Vq64, w.d, w.e, tq64,
+                                                               reinterpret_cast<uepm::q4<double>*>(w.S32), cs));
+                HIP_OK(rec(ci, kTridiag, 1));
+                HIP_OK(rec(ci, kTriEig, 0));
+                HIP_OK(uepm::launch_tri_eig(w.d, w.e, N, m, c, w.Ev, stage_vec ? w.Z : nullptr, stage_vec ? w.W : nullptr,
+                                            !stage_vec ? 0 : mixed ? kMixedInvSweeps : kFp64InvSweeps,
+                                            mixed ? kMixedBisectTol : 0.0, stage_vec ? ks : nullptr,
+                                            stage_vec ? nullptr : status, c0, cs));
+                if (!mixed) HIP_OK(uepm::launch_pair_levels(w.Ev, nb, c, devals + c0 * nb, cs));
+                HIP_OK(rec(ci, kTriEig, 1));
+                if (!stage_vec) continue;
+                double2* Xc = devecs ? reinterpret_cast<double2*>(devecs) + (size_t)c0 * nb * n : nullptr;
+                double* gc = dgrads ? dgrads + 3 * c0 * nb : nullptr;
+                HIP_OK(rec(ci, kBack, 0));
+                HIP_OK(uepm::launch_cluster_orth(w.d, w.e, w.Ev, w.Z, N, m, c, cs));
+                if (mixed)
+                    HIP_OK(uepm::launch_apply_q_quaternion_f32(Vq32, N, tq32, w.Z, m, Xq, c, cs));
+                else
+                    HIP_OK(uepm::launch_apply_q_quaternion_f64(Vq64, N, tq64, w.Z, nb, Xc, gc, p->P, kc,
+                                                               p->G.as<int32_t>(), c, ks, status, c0, cs));
+                HIP_OK(rec(ci, kBack, 1));
+                if (!mixed) continue;
+                HIP_OK(rec(ci, kRefine, 0));
+                HIP_OK(uepm::launch_refine_quaternion(Hq, N, Xq, m, nb, devals + c0 * nb, Xc, gc, p->P, kc,
+                                                      p->G.as<int32_t>(), c, ks, status, c0, cs));
                 HIP_OK(rec(ci, kRefine, 1));
                 continue;
             }
@@ -753,6 +827,7 @@ int uepm_plan_create(uepm_ctx* ctx, const uepm_material* m, const int32_t* G, in
         p->inversion = p->inversion && P.need_l0_a == P.need_l0_c && P.need_l2_a == P.need_l2_c &&
                        P.alpha0_a == P.alpha0_c && P.dfbeta_a == P.dfbeta_c && P.A2_a == P.A2_c && P.R0_a == P.R0_c &&
                        P.R2_a == P.R2_c && P.gpre_a == P.gpre_c;
+    p->soc_symmetric = soc && P.period_a == P.period_c && P.xi_a == P.xi_c && P.mu == P.alpha_mu;
     plan_apply_config(p);
     hipError_t e = p->G.ensure(sizeof(int32_t) * 3 * (size_t)N);
     if (e == hipSuccess) e = hipMemcpy(p->G.p, G, sizeof(int32_t) * 3 * (size_t)N, hipMemcpyHostToDevice);

@@ -103,7 +103,9 @@ struct uepm_plan {
     uepm::TriPlan tp{}, tp32{};
     uepm_config cfg{};    // requested configuration (0 fields = automatic)
     bool inversion = false;  // equal atoms: no antisymmetric form factors, cation = anion non-local terms
+    bool soc_symmetric = false;  // equal spin-orbit terms of cation and anion
     bool real = false;       // H(k) is real symmetric and the real kernels run (plan_apply_config)
+    bool quat = false;       // H(k) is quaternion (spin-orbit, equal atoms) and the quaternion kernels run
     bool tri_reg = false; // register-resident complex64 reduction (precision form, dim <= 288)
     int bt_bands = 16;    // bands per workgroup of the reflector-by-reflector back-transform
     bool bt_wy = false;   // the blocked MFMA back-transform instead (complex64 or FP64 by form)
