@@ -1,11 +1,11 @@
 // solver_f64.hip — tridiagonal eigen-stage of the band solve on gfx950.
 //
 //   (c) tri_eig_wave_kernel bisection (Sturm counts, multisection) for the lowest
-//                           nb eigenvalues of T and inverse iteration for their
-//                           vectors, one wave per k
+//                           nb eigenvalues of T, one wave per k
+//       tri_vec_kernel      inverse iteration for their vectors, one lane per band
 //
-// The assembly (a) lives in assemble.hip, the Householder reduction (b) in tridiag_reg.hip / tridiag_blocked.hip
-// and the back-transform (d) in backtransform.hip; (b)-(d) replace
+// The assembly (a) lives in assemble.hip, the Householder reduction (b) in
+// tridiag_*.hip and the back-transform (d) in backtransform.hip; (b)-(d) replace
 // Eigen::SelfAdjointEigenSolver::compute (Hamiltonian.cpp:129): same
 // eigenvalues to within the backward-stability envelope of a Householder
 // reduction, eigenvectors up to phase (and basis inside degenerate clusters).
@@ -32,60 +32,72 @@ __device__ __forceinline__ double lane_rand(uint32_t i, uint32_t b) {
     return (double)(h >> 8) * (1.0 / 8388608.0) - 1.0;
 }
 
-// Wave-per-k variant: the d, e of a k-point are staged in LDS (16 n bytes of
-// dynamic LDS) and read from there by every Sturm count and inverse-iteration
-// sweep; lanes = bands x S shifts (multisection: one sweep narrows the bracket
-// of every band S+1-fold); inverse iteration on the first lane of a band.
+// 1/x: hardware reciprocal and Newton steps to full precision
 __device__ __forceinline__ double rcp_nr64(double x) {
     double r = __builtin_amdgcn_rcp(x);
     r = fma(fma(-x, r, 1.0), r, r);
     return fma(fma(-x, r, 1.0), r, r);
 }
 
-// 1/x from v_rcp_f64 and one Newton step: the Sturm recurrence is backward
-// stable, and an error of a few ulp in a pivot moves only the counts of
-// probes within rounding of an eigenvalue
-__device__ __forceinline__ double rcp_nr64_1(double x) {
-    const double r = __builtin_amdgcn_rcp(x);
-    return fma(fma(-x, r, 1.0), r, r);
-}
-
-// number of eigenvalues of T below x (Sturm count, pivmin-guarded)
-__device__ __forceinline__ int sturm_count_u(const double* __restrict__ d, const double* __restrict__ e, int n,
-                                             double x, double pivmin) {
-    double q = d[0] - x;
-    if (fabs(q) < pivmin) q = -pivmin;
-    int c = q < 0.0;
-    int i = 1;
-    for (; i + 8 <= n; i += 8) {
-        double dd[8], ee[8];
+// number of eigenvalues of T below x: sign changes of the leading principal
+// minors p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2}, T scaled to norm 1..2 and e^2
+// held above 2^-120 (so that no two neighbours vanish and eight steps stay in
+// range; the pair is rescaled by a power of two every eight).  One multiply-add
+// long per step, against a reciprocal and its Newton step for the quotients
+// p_i / p_{i-1}; the two have the same backward error.  n and the LDS arrays are
+// padded to whole pairs of blocks of eight (kSturmPad, rows that change no sign).
+__device__ __forceinline__ int sturm_count(const double* __restrict__ sd, const double* __restrict__ se2, int np, double x) {
+    struct Block {
+        double d[8], e[8];
+    };
+    auto load = [&](Block& r, int i) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            dd[u] = d[i + u];
-            ee[u] = e[i + u - 1];
+            r.d[u] = sd[i + u];
+            r.e[u] = se2[i + u];
         }
+    };
+    double p = 1.0, pp = 0.0;
+    unsigned signs = 0;  // sign bits of the last minors, the newest lowest
+    int c = 0;
+    auto step = [&](const Block& r) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            q = (dd[u] - x) - (ee[u] * ee[u]) * rcp_nr64_1(q);
-            if (fabs(q) < pivmin) q = -pivmin;
-            c += q < 0.0;
+            const double pn = fma(r.d[u] - x, p, -(r.e[u] * pp));
+            signs = __builtin_amdgcn_alignbit(signs, (unsigned)__double2hiint(pn), 31);
+            pp = p;
+            p = pn;
         }
-    }
-    for (; i < n; ++i) {
-        q = (d[i] - x) - (e[i - 1] * e[i - 1]) * rcp_nr64_1(q);
-        if (fabs(q) < pivmin) q = -pivmin;
-        c += q < 0.0;
+        c += __popc((signs ^ signs >> 1) & 0xffu);
+        const int ex = __builtin_amdgcn_frexp_exp(fmax(fabs(p), fabs(pp)));
+        p = __builtin_amdgcn_ldexp(p, -ex);
+        pp = __builtin_amdgcn_ldexp(pp, -ex);
+    };
+    Block r0, r1;  // the block after the current one is always in flight
+    load(r0, 0);
+    for (int i = 0; i < np; i += 16) {
+        load(r1, i + 8);
+        step(r0);
+        load(r0, i + 16 < np ? i + 16 : i);
+        step(r1);
     }
     return c;
 }
+// d of a padding row: far above every probe, so p keeps its sign
+constexpr double kSturmPad = 16.0;
 
-// abstol_rel: bisection also stops once a bracket is narrower than
-// abstol_rel * ||T||_inf (0: to the rounding level of the eigenvalue itself).
+// Eigenvalues of T by multisection, one wave per k-point and 64 / S bands (S probes
+// per band): a sweep narrows the bracket of every band S + 1-fold.  d and e^2,
+// scaled, sit in LDS, uniform reads across the wave.  abstol_rel: a bracket
+// narrower than abstol_rel ||T||_inf is final (0: the rounding level of the
+// eigenvalue, or a sixteenth of ||T||'s where that is more).  At N = 181,
+// 16 bands, 4096 k-points (two chunks in flight) it takes 0.26 ms against 0.45 ms
+// with the ratio form of the count (a division a row) and unpadded rows; bound by
+// FP64 issue, and at one k-point by the chain of fmas (69 us for 11 sweeps).
 template <int S>
 __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __restrict__ dall,
-                                                          const double* __restrict__ eall, int n, int nb, int64_t nk,
-                                                          double* __restrict__ evals, double* __restrict__ Z,
-                                                          double* __restrict__ W, int inv_sweeps,
+                                                          const double* __restrict__ eall, int n, int nb,
+                                                          double* __restrict__ evals, double* __restrict__ tnorms,
                                                           double abstol_rel, int* __restrict__ kstat,
                                                           unsigned long long* __restrict__ status, int64_t k0) {
     constexpr int NBW = 64 / S;  // bands per wave
@@ -95,24 +107,33 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
     const bool live = b < nb;
     const double* d = dall + kk * n;
     const double* e = eall + kk * n;
-    // Gershgorin interval and scale (wave-uniform)
-    double lo = DBL_MAX, hi = -DBL_MAX, emax2 = 0.0, tnorm = 0.0;
+    extern __shared__ double tri_lds[];
+    const int np = (n + 15) & ~15;
+    double* const sd = tri_lds;
+    double* const se2 = tri_lds + np;
+    // Gershgorin interval and scale
+    double lo = DBL_MAX, hi = -DBL_MAX, tnorm = 0.0;
     bool finite = true;
-    for (int i = 0; i < n; ++i) {
-        const double el = i > 0 ? fabs(e[i - 1]) : 0.0;
-        const double er = i + 1 < n ? fabs(e[i]) : 0.0;
-        finite = finite && isfinite(d[i]) && isfinite(er);
-        lo = fmin(lo, d[i] - el - er);
-        hi = fmax(hi, d[i] + el + er);
-        emax2 = fmax(emax2, er * er);
-        tnorm = fmax(tnorm, fabs(d[i]) + el + er);
+    for (int i = lane; i < n; i += 64) {
+        const double di = d[i], el = i > 0 ? fabs(e[i - 1]) : 0.0, er = i + 1 < n ? fabs(e[i]) : 0.0;
+        finite = finite && isfinite(di) && isfinite(er);
+        lo = fmin(lo, di - el - er);
+        hi = fmax(hi, di + el + er);
+        tnorm = fmax(tnorm, fabs(di) + el + er);
     }
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = fmin(lo, __shfl_xor(lo, o, 64));
+        hi = fmax(hi, __shfl_xor(hi, o, 64));
+        tnorm = fmax(tnorm, __shfl_xor(tnorm, o, 64));
+    }
+    finite = __all(finite) && isfinite(tnorm);
     // A non-finite T (a non-finite k-point, or H(k) overflowing) has no
     // eigen-decomposition (the reference's Eigen solver reports NoConvergence,
-    // Hamiltonian.cpp:130-133): NaN eigenvalues and vectors, and the k-point is
-    // flagged -- in kstat for a later stage to report, or in status directly
-    // when this is the last stage.  Both conditions are the same in every wave.
+    // Hamiltonian.cpp:130-133): NaN eigenvalues (and, in tri_vec_kernel, vectors), and
+    // the k-point is flagged -- in kstat for a later stage to report, or in status
+    // directly when this is the last stage.  Both conditions are the same in every wave.
     if (blockIdx.y == 0 && lane == 0) {
+        if (tnorms) tnorms[kk] = tnorm;
         if (kstat) kstat[kk] = finite ? 0 : 1;
         else if (status && !finite) {
             atomicAdd(&status[0], 1ull);
@@ -120,29 +141,23 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
         }
     }
     if (!finite) {
-        if (live && sub == 0) {
-            evals[kk * nb + b] = __builtin_nan("");
-            if (inv_sweeps > 0)
-                for (int i = 0; i < n; ++i) Z[(size_t)(kk * nb + b) * n + i] = __builtin_nan("");
-        }
+        if (live && sub == 0) evals[kk * nb + b] = __builtin_nan("");
         return;
     }
-    // d and e in LDS: the Sturm counts re-read them every probe sweep, and the
-    // inverse iteration every sweep (3-8% off a launch alone, against reading
-    // them from global memory; the same values, so the same results)
-    extern __shared__ double tri_lds[];
-    double* const sd = tri_lds;
-    double* const se = tri_lds + n;
-    for (int i = lane; i < n; i += 64) {
-        sd[i] = d[i];
-        se[i] = e[i];
+    // scaled by a power of two (exact) to 1 <= ||T|| < 2
+    const int ex = tnorm > 0.0 ? 1 - __builtin_amdgcn_frexp_exp(tnorm) : 0;
+    auto scaled = [&](double v) { return __builtin_amdgcn_ldexp(v, ex); };
+    for (int i = lane; i < np; i += 64) {
+        const double ei = i > 0 && i < n ? scaled(e[i - 1]) : 0.0;
+        sd[i] = i < n ? scaled(d[i]) : kSturmPad;
+        se2[i] = i < n ? fmax(ei * ei, 0x1p-120) : 0.0;
     }
     __syncthreads();
-    const double pivmin = DBL_MIN * fmax(1.0, emax2);
     const double eps = DBL_EPSILON;
-    lo -= 2.0 * eps * tnorm + pivmin;
-    hi += 2.0 * eps * tnorm + pivmin;
-    const double abstol = abstol_rel * tnorm;
+    tnorm = scaled(tnorm);
+    lo = scaled(lo) - 2.0 * eps * tnorm - 0x1p-58;  // and what the floor of e^2 may move
+    hi = scaled(hi) + 2.0 * eps * tnorm + 0x1p-58;
+    const double abstol = fmax(abstol_rel, eps / 16.0) * tnorm;
     // two shared sweeps first: the wave's 64 lanes probe one interval that holds
     // every band of the wave, and each band takes the probes around its index
     // (a count c at x puts eigenvalues 0..c-1 below x and c.. at or above it)
@@ -152,7 +167,7 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
         double L = lo, U = hi;
         for (int sw = 0; sw < 2; ++sw) {
             const double x = L + (double)(lane + 1) * ((U - L) / 65.0);
-            const int cnt = sturm_count_u(sd, se, n, x, pivmin);
+            const int cnt = sturm_count(sd, se2, np, x);
             double nlo = lo, nhi = hi;
             for (int u = 0; u < 64; ++u) {
                 const int cu = __shfl(cnt, u, 64);
@@ -169,10 +184,10 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
     // multisection: lane `sub` of a band probes lo + (sub+1) (hi-lo)/(S+1)
     for (int it = 0; it < 200; ++it) {
         const double w = hi - lo;
-        const bool done = !live || w <= 2.0 * eps * fmax(fabs(lo), fabs(hi)) + 4.0 * pivmin || w <= abstol;
+        const bool done = !live || w <= 2.0 * eps * fmax(fabs(lo), fabs(hi)) || w <= abstol;
         if (__all(done)) break;
-        const double x = lo + (double)(sub + 1) * (w / (double)(S + 1));
-        const int cnt = done ? 0 : sturm_count_u(sd, se, n, x, pivmin);
+        const double x = lo + (double)(sub + 1) * (w * (1.0 / (double)(S + 1)));
+        const int cnt = done ? 0 : sturm_count(sd, se2, np, x);
         // gather the S probes of this band
         double nlo = lo, nhi = hi;
 #pragma unroll
@@ -183,7 +198,7 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
             else nlo = fmax(nlo, xu);
         }
         if (!done) {
-            if (nlo >= nhi || nlo <= lo && nhi >= hi) {  // no progress possible (rounding): stop here
+            if (nlo >= nhi || (nlo <= lo && nhi >= hi)) {  // no progress possible (rounding): stop here
                 lo = hi = 0.5 * (lo + hi);
             } else {
                 lo = nlo;
@@ -191,152 +206,146 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
             }
         }
     }
-    const double lam = 0.5 * (lo + hi);
-    if (live && sub == 0) evals[kk * nb + b] = lam;
-    if (inv_sweeps <= 0 || !live || sub != 0) return;
+    if (live && sub == 0) evals[kk * nb + b] = __builtin_amdgcn_ldexp(0.5 * (lo + hi), -ex);
+}
 
-    // Inverse iteration with an LU factorisation of T - lam I with partial
-    // pivoting (rows k, k+1 interchanged when |e_k| > |pivot|), inv_sweeps
-    // sweeps from a fixed pseudo-random start.  Each forward sweep recomputes the
-    // multipliers and interchanges (the same operations, so the same values)
-    // instead of reading them back, and each iterate's 1/max scaling is
-    // applied when the next sweep reads it: the interleaved work arrays (over
-    // the nk * nb (k, band) pairs) hold only the U factor and the iterate.
-    const int64_t T = nk * nb;
-    const int64_t t = kk * nb + b;
-    double* __restrict__ U0 = W;                      // reciprocal pivots
-    double* __restrict__ U1 = W + (size_t)n * T;      // first super-diagonal
-    double* __restrict__ U2 = W + (size_t)2 * n * T;  // second super-diagonal
-    double* __restrict__ X = W + (size_t)3 * n * T;   // forward result, then iterate (unscaled)
-#define IDX(i) ((size_t)(i) * T + t)
-    // The loads of PB rows are issued together ahead of their use (each row is
-    // read before this sweep overwrites it), so a sweep waits on memory once
-    // per PB rows instead of once per row.
-    constexpr int PB = 4;
-    const double tiny = eps * tnorm;
-    double sc = 1.0;  // scaling of the iterate in X
-    for (int iter = 0; iter < inv_sweeps; ++iter) {
-        const bool first = iter == 0;
-        // forward: factor row k, apply the interchange and the multiplier
-        double a = sd[0] - lam;
-        double c = n > 1 ? se[0] : 0.0;
-        double yk = first ? lane_rand(0u, (uint32_t)b) : X[IDX(0)] * sc;
-        for (int k0 = 0; k0 + 1 < n; k0 += PB) {
-            double xn[PB];
-            if (!first) {
+// Eigenvectors of T by inverse iteration, one lane per (k, band): LU factorisation
+// of T - lam I with partial pivoting (rows k, k+1 interchanged when |e_k| >
+// |pivot|), `sweeps` sweeps from a fixed pseudo-random start.
+//
+// The factors of n rows and 16 bands do not fit registers or LDS, and writing them
+// out and back bounded the stage (nineteen words a row and band over two sweeps).  Here a
+// sweep goes forward once keeping only the elimination's state at every kRows-th
+// row, then walks those blocks backwards: each is eliminated again in registers
+// (the same operations, so the same values) and substituted back at once.  A sweep
+// reads the previous iterate twice and writes one (work arrays interleaved over
+// the (k, band) pairs, one coalesced access a row); the last one writes Z, not
+// normalised: cluster_orth_kernel does that.  N = 181, 16 bands, 4096 k-points, two
+// chunks in flight: 0.33 ms against 0.58 ms with the factors in memory.
+constexpr int kRows = 8;
+__global__ __launch_bounds__(64, 2) void tri_vec_kernel(const double* __restrict__ dall, const double* __restrict__ eall,
+                                                        int n, int nb, int64_t T, const double* __restrict__ evals,
+                                                        const double* __restrict__ tnorms, const int* __restrict__ kstat,
+                                                        double* __restrict__ W, double* __restrict__ Z, int sweeps) {
+    const int64_t t = blockIdx.x * (int64_t)64 + threadIdx.x;
+    if (t >= T) return;
+    const int64_t kk = t / nb;
+    const uint32_t b = (uint32_t)(t - kk * nb);
+    double* z = Z + t * n;
+    if (kstat[kk]) {
+        for (int i = 0; i < n; ++i) z[i] = __builtin_nan("");
+        return;
+    }
+    const double* d = dall + kk * n;
+    const double* e = eall + kk * n;
+    const double lam = evals[t], tiny = DBL_EPSILON * tnorms[kk];
+    const int nblk = (n - 1 + kRows - 1) / kRows;  // blocks of eliminated rows 0 .. n - 2
+    double* __restrict__ C = W + (size_t)2 * n * T;  // (a, c, y) at every block's first row
+    struct State {
+        double a, c, y;  // pivot row: a x_k + c x_{k+1} (+ ...) = y
+    };
+    double sc = 1.0;  // scaling of the previous iterate
+    for (int iter = 0; iter < sweeps; ++iter) {
+        const double* __restrict__ Xin = W + (size_t)(iter & 1) * n * T;          // previous iterate (iter > 0)
+        double* __restrict__ Xout = W + (size_t)((iter & 1) ^ 1) * n * T;
+        const bool first = iter == 0, last = iter == sweeps - 1;
+        // the rows k0 .. k0 + kRows - 1: d, e and the right-hand side one row ahead
+        struct Rows {
+            double e[kRows + 1], d[kRows], y[kRows];
+        };
+        auto load = [&](int k0, Rows& r) {
 #pragma unroll
-                for (int u = 0; u < PB; ++u) xn[u] = (k0 + 1 + u < n) ? X[IDX(k0 + 1 + u)] : 0.0;
-            }
-#pragma unroll
-            for (int u = 0; u < PB; ++u) {
+            for (int u = 0; u < kRows; ++u) {
                 const int k = k0 + u;
-                if (k + 1 >= n) break;
-                const double sub_ = se[k];
-                const double dn = sd[k + 1] - lam;
-                const double en = (k + 2 < n) ? se[k + 1] : 0.0;
-                double yk1 = first ? lane_rand((uint32_t)(k + 1), (uint32_t)b) : xn[u] * sc;
-                double mult;
-                if (fabs(a) >= fabs(sub_)) {
-                    if (a == 0.0) a = tiny;
-                    const double ra = rcp_nr64(a);
-                    mult = sub_ * ra;
-                    if (first) {
-                        U0[IDX(k)] = ra;
-                        U1[IDX(k)] = c;
-                        U2[IDX(k)] = 0.0;
-                    }
-                    a = dn - mult * c;
-                    c = en;
-                } else {
-                    const double rs = rcp_nr64(sub_);
-                    mult = a * rs;
-                    if (first) {
-                        U0[IDX(k)] = rs;
-                        U1[IDX(k)] = dn;
-                        U2[IDX(k)] = en;
-                    }
-                    a = c - mult * dn;
-                    c = -mult * en;
-                    const double tmp = yk;
-                    yk = yk1;
-                    yk1 = tmp;
-                }
-                yk1 -= mult * yk;
-                X[IDX(k)] = yk;
-                yk = yk1;
+                r.e[u] = e[min(k, n - 1)];
+                r.d[u] = d[min(k + 1, n - 1)];
+                if (!first) r.y[u] = Xin[(size_t)min(k + 1, n - 1) * T + t];
             }
+            r.e[kRows] = e[min(k0 + kRows, n - 1)];
+        };
+        // eliminates row k = k0 + u: multipliers and interchange applied to the state;
+        // out: reciprocal pivot, first and second super-diagonal of U, forward result
+        auto eliminate = [&](State& s, const Rows& r, int k, int u, double* out) {
+            const double sub = r.e[u];
+            const double dn = r.d[u] - lam;
+            const double en = k + 2 < n ? r.e[u + 1] : 0.0;
+            const double y1 = first ? lane_rand((uint32_t)(k + 1), b) : r.y[u] * sc;
+            const bool keep = fabs(s.a) >= fabs(sub);
+            const double piv = keep ? (s.a == 0.0 ? tiny : s.a) : sub;
+            const double rp = rcp_nr64(piv);
+            const double mult = (keep ? sub : s.a) * rp;
+            const double u1 = keep ? s.c : dn, u2 = keep ? 0.0 : en;
+            const double top = keep ? s.y : y1, bot = keep ? y1 : s.y;
+            s.a = (keep ? dn : s.c) - mult * u1;
+            s.c = keep ? en : -mult * en;
+            s.y = bot - mult * top;
+            if (out) {
+                out[0] = rp;
+                out[1] = u1;
+                out[2] = u2;
+                out[3] = top;
+            }
+        };
+        State s{d[0] - lam, n > 1 ? e[0] : 0.0, first ? lane_rand(0u, b) : Xin[t] * sc};
+        for (int blk = 0; blk < nblk; ++blk) {
+            C[(size_t)(3 * blk) * T + t] = s.a;
+            C[(size_t)(3 * blk + 1) * T + t] = s.c;
+            C[(size_t)(3 * blk + 2) * T + t] = s.y;
+            Rows r;
+            load(kRows * blk, r);
+#pragma unroll
+            for (int u = 0; u < kRows; ++u)
+                if (kRows * blk + u + 1 < n) eliminate(s, r, kRows * blk + u, u, nullptr);
         }
-        // the last pivot is the same every sweep
-        if (a == 0.0) a = tiny;
-        const double ra_last = rcp_nr64(a);
-        if (first) U0[IDX(n - 1)] = ra_last;
-        // back substitution
-        double x2 = 0.0, x1 = yk * ra_last;
-        X[IDX(n - 1)] = x1;
+        auto put = [&](int k, double x) {
+            if (last) z[k] = x;
+            else Xout[(size_t)k * T + t] = x;
+        };
+        double x1 = s.y * rcp_nr64(s.a == 0.0 ? tiny : s.a), x2 = 0.0;
+        put(n - 1, x1);
         double amax = fabs(x1);
-        for (int k1 = n - 2; k1 >= 0; k1 -= PB) {
-            double xv[PB], u0[PB], u1[PB], u2[PB];
+        for (int blk = nblk - 1; blk >= 0; --blk) {
+            State q{C[(size_t)(3 * blk) * T + t], C[(size_t)(3 * blk + 1) * T + t], C[(size_t)(3 * blk + 2) * T + t]};
+            Rows r;
+            load(kRows * blk, r);
+            double f[kRows][4];
 #pragma unroll
-            for (int u = 0; u < PB; ++u) {
-                const int k = k1 - u;
-                if (k < 0) break;
-                xv[u] = X[IDX(k)];
-                u0[u] = U0[IDX(k)];
-                u1[u] = U1[IDX(k)];
-                u2[u] = U2[IDX(k)];
-            }
+            for (int u = 0; u < kRows; ++u)
+                if (kRows * blk + u + 1 < n) eliminate(q, r, kRows * blk + u, u, f[u]);
 #pragma unroll
-            for (int u = 0; u < PB; ++u) {
-                const int k = k1 - u;
-                if (k < 0) break;
-                const double xk = (xv[u] - u1[u] * x1 - u2[u] * x2) * u0[u];
-                X[IDX(k)] = xk;
-                x2 = x1;
-                x1 = xk;
-                amax = fmax(amax, fabs(xk));
+            for (int u = kRows - 1; u >= 0; --u) {
+                const int k = kRows * blk + u;
+                if (k + 1 < n) {
+                    const double x = (f[u][3] - f[u][1] * x1 - f[u][2] * x2) * f[u][0];
+                    put(k, x);
+                    x2 = x1;
+                    x1 = x;
+                    amax = fmax(amax, fabs(x));
+                }
             }
         }
         sc = 1.0 / amax;
     }
-    double nrm = 0.0;
-    for (int i0 = 0; i0 < n; i0 += PB) {
-        double xv[PB];
-#pragma unroll
-        for (int u = 0; u < PB; ++u) xv[u] = (i0 + u < n) ? X[IDX(i0 + u)] : 0.0;
-#pragma unroll
-        for (int u = 0; u < PB; ++u) {
-            if (i0 + u >= n) break;
-            const double xi = xv[u] * sc;
-            nrm += xi * xi;
-        }
-    }
-    const double sn = 1.0 / sqrt(nrm);
-    double* z = Z + (size_t)t * n;
-    for (int i0 = 0; i0 < n; i0 += PB) {
-        double xv[PB];
-#pragma unroll
-        for (int u = 0; u < PB; ++u) xv[u] = (i0 + u < n) ? X[IDX(i0 + u)] : 0.0;
-#pragma unroll
-        for (int u = 0; u < PB; ++u)
-            if (i0 + u < n) z[i0 + u] = (xv[u] * sc) * sn;
-    }
-#undef IDX
 }
 
 // ------------------------------------------------------------ launchers
 hipError_t launch_tri_eig(const double* dd, const double* de, int n, int nb, int64_t nk, double* devals, double* dZ,
                           double* dW, int inv_sweeps, double abstol_rel, int* kstat, unsigned long long* status,
                           int64_t k0, hipStream_t s) {
-    const size_t shm = sizeof(double) * 2 * (size_t)n;  // d and e of the k-point
-    if (nb <= 16)
-        hipLaunchKernelGGL(tri_eig_wave_kernel<4>, dim3((unsigned)nk, 1), dim3(64), shm, s, dd, de, n, nb, nk, devals,
-                           dZ, dW, inv_sweeps, abstol_rel, kstat, status, k0);
-    else if (nb <= 32)
-        hipLaunchKernelGGL(tri_eig_wave_kernel<2>, dim3((unsigned)nk, 1), dim3(64), shm, s, dd, de, n, nb, nk, devals,
-                           dZ, dW, inv_sweeps, abstol_rel, kstat, status, k0);
-    else
-        hipLaunchKernelGGL(tri_eig_wave_kernel<1>, dim3((unsigned)nk, (unsigned)((nb + 63) / 64)), dim3(64), shm, s, dd,
-                           de, n, nb, nk, devals, dZ, dW, inv_sweeps, abstol_rel, kstat, status, k0);
+    const size_t shm = sizeof(double) * 2 * (size_t)((n + 15) & ~15);  // d and e^2 of the k-point
+    const int64_t T = nk * nb;
+    // the work array holds two iterates, the elimination states and, last, the norms
+    double* tnorms = inv_sweeps > 0 ? dW + (size_t)4 * n * T - nk : nullptr;
+    auto eig = [&](auto kern, int bands) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)nk, (unsigned)((nb + bands - 1) / bands)), dim3(64), shm, s, dd, de, n, nb,
+                           devals, tnorms, abstol_rel, kstat, status, k0);
+    };
+    if (nb <= 16) eig(tri_eig_wave_kernel<4>, 16);
+    else if (nb <= 32) eig(tri_eig_wave_kernel<2>, 32);
+    else eig(tri_eig_wave_kernel<1>, 64);
+    if (inv_sweeps > 0)
+        hipLaunchKernelGGL(tri_vec_kernel, dim3((unsigned)((T + 63) / 64)), dim3(64), 0, s, dd, de, n, nb, T, devals, tnorms,
+                           kstat, dW, dZ, inv_sweeps);
     return hipGetLastError();
 }
 
