@@ -33,6 +33,7 @@ DATAPATH = {
     ("fp64", "tridiag_reg_kernel"): "VALU FP64 (78.6 TF/s, equal to the FP64 MFMA rate)",
     ("mixed", "tridiag_blocked_kernel"): "VALU FP32 symmetric products, MFMA FP32 panel updates (157.3 TF/s either way)",
     ("mixed", "tridiag_blocked+reg_kernel"): "VALU FP32 symmetric products, MFMA FP32 panel updates, then the register grids",
+    ("mixed", "tridiag_strip+reg_kernel"): "VALU FP32 (157.3 TF/s, the FP32 MFMA rate too): no MFMA in the register-grid chain",
     ("fp64", "tridiag_blocked_kernel"): "VALU FP64 symmetric products, MFMA FP64 panel updates (78.6 TF/s either way)",
     ("fp64", "tridiag_blocked+reg_kernel"): "VALU FP64 symmetric products, MFMA FP64 panel updates, then the register grids",
 }

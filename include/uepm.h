@@ -202,7 +202,7 @@ int uepm_plan_last_timing(const uepm_plan* plan, int stage, double* ms, int64_t*
 /* ---- configuration, tuning and workspace -----------------------------------
  * No counterpart in the reference (its solve has no tunables). */
 typedef struct uepm_config {
-    int32_t tridiag;   /* 0 automatic (UEPM_MIXED plans above dim 288: LDS-blocked
+    int32_t tridiag;   /* 0 automatic (UEPM_MIXED plans above dim 384: LDS-blocked
                           leading steps, then the register grids); 1 LDS-blocked
                           reduction only; 2 register-resident complex64 reduction
                           (UEPM_MIXED plans, dim <= 288)                              */

@@ -53,8 +53,8 @@ int64_t plan_chunk(const uepm_plan* p, int64_t nk) {
 }
 
 namespace {
-// Trailing size of the precision form's blocked reduction (n > 288) that the
-// register grids take over; 0 when the configuration asks for the blocked kernel.
+// Trailing size that the register grids (with the strip kernel up to n = 384) take over
+// in the precision form above n = 288, after a blocked reduction if less than n; 0 when the configuration asks for the blocked kernel.
 int mixed_c64_tail(const uepm_plan* p) {
     if (p->tri_reg || p->cfg.tridiag == 1 || p->dim <= uepm::tridiag_reg_max_n()) return 0;
     return uepm::tridiag_reg_c64_tail(p->dim);
@@ -298,6 +298,7 @@ int solve_chunks(uepm_plan* p, const double* dk, int64_t nk, double* devals, dou
     };
     bool used[kNumStages] = {true, true, true, stage_vec, mixed};
     p->stage_name[kTridiag] = mixed ? (p->tri_reg              ? "tridiag_reg_kernel<c64>"
+                                       : mixed_c64_tail(p) == n ? "tridiag_strip+reg_kernel<c64>"
                                        : mixed_c64_tail(p) > 0 ? "tridiag_blocked+reg_kernel<c64>"
                                                                : "tridiag_blocked_kernel<c64>")
                                     : uepm::tridiag_reg_c128_tail(n) == n ? "tridiag_reg_kernel<c128>"
@@ -425,11 +426,11 @@ int solve_chunks(uepm_plan* p, const double* dk, int64_t nk, double* devals, dou
                 // complex64 back-transform, FP64 Rayleigh-Ritz on the FP64 H(k)
                 float2* Vc = w.Vf;
                 HIP_OK(rec(ci, kTridiag, 0));
-                if (p->tri_reg)
+                if (p->tri_reg || mixed_c64_tail(p) == n)
                     HIP_OK(uepm::launch_tridiag_reg_c64(Hc, n, n, c, Vc, w.d, w.e,
                                                         w.tauf, w.S32, cs));
                 else {
-                    // n > 288: the blocked reduction for the leading steps, the register grids
+                    // n > 384: the blocked reduction for the leading steps, the register grids
                     // for the trailing block it leaves in place in Vc
                     const int t = mixed_c64_tail(p);
                     const int s0 = n - t;
