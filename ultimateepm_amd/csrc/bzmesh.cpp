@@ -664,13 +664,13 @@ int uepm_bzmesh_dos_device(uepm_bzmesh* m, int32_t band, int32_t n_points, doubl
     if (band < 0 || band >= m->nb) return fail(UEPM_ERR_OUT_OF_RANGE, "uepm_bzmesh_dos: band index out of range");
     HIP_OK(hipSetDevice(m->ctx->device));
     const int slices = uepm::tetra_dos_slices(m->nt, n_points);
-    HIP_OK(m->window.ensure(sizeof(int2) * std::max<int64_t>(m->nt, 1)));
+    HIP_OK(m->window.ensure(sizeof(uepm::TetraRange) * std::max<int64_t>(m->nt, 1)));
     HIP_OK(m->partial.ensure(sizeof(double) * slices * n_points));
     const double* Eb = m->Eb.as<double>() + static_cast<int64_t>(band) * m->nv;
     const double* Gb = m->Gb.as<double>() + 3 * static_cast<int64_t>(band) * m->nv;
     HIP_OK(uepm::launch_tetra_dos(m->pos.as<double>(), m->dtet.as<int32_t>(), m->det.as<double>(),
                                   wedge_only ? m->wedge.as<uint8_t>() : nullptr, m->nt, Eb, Gb, n_points, e_min, e_max,
-                                  reduce_bz_factor, spin_degeneracy, wedge_only ? 48.0 : 1.0, m->window.as<int2>(),
+                                  reduce_bz_factor, spin_degeneracy, wedge_only ? 48.0 : 1.0, m->window.as<uepm::TetraRange>(),
                                   m->partial.as<double>(), d_energies, d_dos, static_cast<hipStream_t>(stream)));
     return UEPM_OK;
 }

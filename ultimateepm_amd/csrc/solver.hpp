@@ -187,11 +187,15 @@ hipError_t launch_bands_to_band_major(const double* E, const double* G, int64_t 
                                       double* Eb, double* Gb, hipStream_t s);
 // Slices of the tetrahedron list per energy group (a function of nt only); the
 // partial-sum workspace holds tetra_dos_slices(nt, n_points) x n_points
-// doubles, the window nt int2.
+// doubles, the ranges nt entries.
+struct TetraRange {
+    double emin, emax;  // of the corners
+    int lo, hi;         // samples it may cut (empty: lo > hi)
+};
 int tetra_dos_slices(int64_t nt, int n_points);
 hipError_t launch_tetra_dos(const double* pos, const int32_t* tet, const double* det, const uint8_t* in_wedge,
                             int64_t nt, const double* Eb, const double* Gb, int n_points, double e_min, double e_max,
-                            double reduce_bz_factor, double spin_degeneracy, double wedge_factor, int2* window,
+                            double reduce_bz_factor, double spin_degeneracy, double wedge_factor, TetraRange* range,
                             double* partial, double* energies, double* dos, hipStream_t s);
 
 // Dielectric-function sums (dielectric.hip): eigenpairs at k (Ek, Xk) and

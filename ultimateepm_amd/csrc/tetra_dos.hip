@@ -7,15 +7,21 @@
 // on the energy grid of compute_dos_band_at_band_auto, :889-916).
 //
 // Work split: one energy group of kEnergiesPerGroup samples x one slice of the
-// tetrahedra per workgroup.  A per-band prepass stores each tetrahedron's
-// sample-index window (8 bytes), so the scan that decides which tetrahedra
-// cut an energy group reads 8 B per tetrahedron from L2; only the cutting
-// ones load their corners, energies and gradients.  Partial sums per
-// (slice, energy) go to a workspace and a second kernel adds the slices in
-// slice order: the result does not depend on scheduling.
+// tetrahedra per workgroup.  A per-band prepass stores each tetrahedron's energy
+// range and sample-index window (24 bytes, read from L2 by every group).  A block
+// of kBlock tetrahedra is first turned into the list of (energy, tetrahedron) pairs
+// that cut, energy by energy in tetrahedron order, and the list is then worked off
+// one pair per lane: about a tenth of the pairs cut, so a lane per tetrahedron left
+// the waves to their slowest lane: 56k tetrahedra, 500 samples took 0.95 ms a band,
+// with the lists 0.28, with the fewer divisions and no arc tangents of tetra_dos_at
+// 0.21, bound by FP64 issue.  An energy's contributions are added in the order of its
+// own list, and partial sums per (slice, energy) go to a workspace that a second
+// kernel adds in slice order: the result depends neither on scheduling nor on the
+// other energies of the grid.
 //
 // Every expression follows the reference's operation order with contraction
-// off, so a tetrahedron's contribution rounds as the reference's does.
+// off, so a tetrahedron's contribution rounds as the reference's does (the corners'
+// angles only rank them, and are compared by a function that rises with the angle).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -28,7 +34,8 @@
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kEnergiesPerGroup = 8;
+constexpr int kEnergiesPerGroup = 4;  // one wave each in the sums
+constexpr int kBlock = 1024;          // tetrahedra per list: 4 per lane, 40 KB of LDS at worst
 
 struct V3 {
     double x, y, z;
@@ -75,66 +82,60 @@ __global__ void bands_to_band_major_kernel(const double* __restrict__ E, const d
     }
 }
 
-// Sample-index window [lo, hi] of every tetrahedron for one band.  It is a
-// filter only (one sample of slack on each side); the exact test
-// E < min || E > max is repeated per sample in the DOS kernel.
+// Energy range and sample-index window [lo, hi] of every tetrahedron for one band.
+// The window is a filter (one sample of slack on each side) that keeps what is
+// outside the wedge or has no energy at all out; the range is the exact test.
 __global__ void tetra_window_kernel(const int32_t* __restrict__ tet, const uint8_t* __restrict__ in_wedge, int64_t nt,
                                     const double* __restrict__ Eb, double e0, double step, int n_points,
-                                    int2* __restrict__ window) {
+                                    uepm::TetraRange* __restrict__ range) {
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (t >= nt) return;
-    int2 w = make_int2(1, 0);  // empty
+    uepm::TetraRange w{0.0, 0.0, 1, 0};  // empty
     if (!in_wedge || in_wedge[t]) {
-        const double a = Eb[tet[4 * t]], b = Eb[tet[4 * t + 1]], c = Eb[tet[4 * t + 2]], d = Eb[tet[4 * t + 3]];
-        const double mn = fmin(fmin(a, b), fmin(c, d)), mx = fmax(fmax(a, b), fmax(c, d));
+        const double e[4] = {Eb[tet[4 * t]], Eb[tet[4 * t + 1]], Eb[tet[4 * t + 2]], Eb[tet[4 * t + 3]]};
+        const double mn = fmin(fmin(e[0], e[1]), fmin(e[2], e[3])), mx = fmax(fmax(e[0], e[1]), fmax(e[2], e[3]));
+        w.emin = w.emax = e[0];
+        for (int j = 1; j < 4; ++j) {
+            if (e[j] < w.emin) w.emin = e[j];
+            if (w.emax < e[j]) w.emax = e[j];
+        }
         if (mn <= mx) {
             const double flo = floor((mn - e0) / step) - 1.0, fhi = ceil((mx - e0) / step) + 1.0;
             if (fhi >= 0.0 && flo <= static_cast<double>(n_points - 1)) {
-                w.x = flo < 0.0 ? 0 : static_cast<int>(flo);
-                w.y = fhi > static_cast<double>(n_points - 1) ? n_points - 1 : static_cast<int>(fhi);
+                w.lo = flo < 0.0 ? 0 : static_cast<int>(flo);
+                w.hi = fhi > static_cast<double>(n_points - 1) ? n_points - 1 : static_cast<int>(fhi);
             }
         }
     }
-    window[t] = w;
+    range[t] = w;
 }
 
 struct TetraBand {
-    V3 p[4];      // corner positions (1/m)
-    V3 g[4];      // corner gradients of the band (eV m)
-    V3 edge[3];   // p1-p0, p2-p0, p3-p0
-    double e[4];  // corner energies (eV)
-    double det;   // 6 x signed volume
+    int v[4];      // corners
     double emin, emax;
     double es[4];  // corner energies, ascending
-    V3 ps[4];      // corners in that order
+    V3 ps[4];      // corners in that order (1/m)
 };
 
-__device__ __forceinline__ void load_tetra(TetraBand& T, const double* pos, const int32_t* tet, const double* det,
-                                  const double* Eb, const double* Gb, int64_t t) {
-    int e_idx[4];
+__device__ __forceinline__ void load_tetra(TetraBand& T, const double* pos, const int32_t* tet, const double* Eb, int64_t t) {
+    double v[4];
+    V3 q[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        e_idx[j] = tet[4 * t + j];
-        T.p[j] = load3(pos, e_idx[j]);
-        T.g[j] = load3(Gb, e_idx[j]);
-        T.e[j] = Eb[e_idx[j]];
+        T.v[j] = tet[4 * t + j];
+        q[j] = load3(pos, T.v[j]);
+        v[j] = Eb[T.v[j]];
     }
-    T.edge[0] = sub(T.p[1], T.p[0]);
-    T.edge[1] = sub(T.p[2], T.p[0]);
-    T.edge[2] = sub(T.p[3], T.p[0]);
-    T.det = det[t];
-    T.emin = T.e[0];
-    T.emax = T.e[0];
+    T.emin = v[0];
+    T.emax = v[0];
 #pragma unroll
     for (int j = 1; j < 4; ++j) {
-        if (T.e[j] < T.emin) T.emin = T.e[j];
-        if (T.emax < T.e[j]) T.emax = T.e[j];
+        if (v[j] < T.emin) T.emin = v[j];
+        if (T.emax < v[j]) T.emax = v[j];
     }
     // five-comparator network (Tetra::pre_compute_sorted_slots_per_band,
     // mesh_tetra.cpp:287-315); the corners move with their energies, so the
     // sorted data needs no dynamic indexing.
-    double v[4] = {T.e[0], T.e[1], T.e[2], T.e[3]};
-    V3 q[4] = {T.p[0], T.p[1], T.p[2], T.p[3]};
 #define UEPM_CSWAP(a, b)                \
     if (v[a] > v[b]) {                  \
         const double tv = v[a];         \
@@ -157,43 +158,32 @@ __device__ __forceinline__ void load_tetra(TetraBand& T, const double* pos, cons
     }
 }
 
-// Contribution of one tetrahedron at one energy (states / (eV m^3), before the
-// mesh-level factors).
-__device__ __forceinline__ double tetra_dos_at(const TetraBand& T, double energy) {
+// Contribution of tetrahedron t at one energy (states / (eV m^3), before the
+// mesh-level factors).  What the gradients need is loaded only after the polygon is
+// done (its corners are in the caches): both at once take 215 registers.
+__device__ __forceinline__ double tetra_dos_at(const TetraBand& T, const double* pos, const double* det, const double* Gb,
+                                               int64_t t, double energy) {
     if (energy < T.emin || energy > T.emax) return 0.0;
     const double e_0 = T.es[0], e_1 = T.es[1], e_2 = T.es[2], e_3 = T.es[3];
     const V3 P0 = T.ps[0], P1 = T.ps[1], P2 = T.ps[2], P3 = T.ps[3];
-    // iso-energy polygon (Tetra::compute_band_iso_energy_surface, mesh_tetra.cpp:339-395)
+    // iso-energy polygon (Tetra::compute_band_iso_energy_surface, mesh_tetra.cpp:339-395):
+    // corner i at l of the way from A to B; the three cases differ in what goes in, so a
+    // wave that has all three divides four times, not ten
+    const bool low = energy < e_1 && energy >= e_0, mid = !low && energy < e_2 && energy >= e_1;
+    const int n = mid ? 4 : 3;
     V3 iso[4];
-    int n;
-    iso[3] = {0.0, 0.0, 0.0};
-    if (energy < e_1 && energy >= e_0) {
-        const double lU = (energy - e_0) / (e_1 - e_0);
-        const double lV = (energy - e_0) / (e_2 - e_0);
-        const double lW = (energy - e_0) / (e_3 - e_0);
-        iso[0] = add(scale(1.0 - lU, P0), scale(lU, P1));
-        iso[1] = add(scale(1.0 - lV, P0), scale(lV, P2));
-        iso[2] = add(scale(1.0 - lW, P0), scale(lW, P3));
-        n = 3;
-    } else if (energy < e_2 && energy >= e_1) {
-        const double lU = (energy - e_0) / (e_2 - e_0);
-        const double lV = (energy - e_0) / (e_3 - e_0);
-        const double lW = (e_2 - energy) / (e_2 - e_1);
-        const double lX = (energy - e_1) / (e_3 - e_1);
-        iso[0] = add(scale(1.0 - lU, P0), scale(lU, P2));
-        iso[1] = add(scale(1.0 - lV, P0), scale(lV, P3));
-        iso[2] = add(scale(lW, P1), scale(1.0 - lW, P2));
-        iso[3] = add(scale(1.0 - lX, P1), scale(lX, P3));
-        n = 4;
-    } else {
-        const double lU = (e_3 - energy) / (e_3 - e_2);
-        const double lV = (e_3 - energy) / (e_3 - e_1);
-        const double lW = (e_3 - energy) / (e_3 - e_0);
-        iso[0] = add(scale(lU, P2), scale(1.0 - lU, P3));
-        iso[1] = add(scale(lV, P1), scale(1.0 - lV, P3));
-        iso[2] = add(scale(lW, P0), scale(1.0 - lW, P3));
-        n = 3;
-    }
+    auto corner = [&](double num, double den, V3 A, V3 B) {
+        const double l = num / den;
+        return add(scale(1.0 - l, A), scale(l, B));
+    };
+    auto pick = [](bool b, V3 x, V3 y) { return V3{b ? x.x : y.x, b ? x.y : y.y, b ? x.z : y.z}; };
+    const double up = energy - e_0, down = e_3 - energy;
+    const V3 P = pick(low || mid, P0, P3);
+    iso[0] = corner(low || mid ? up : down, low ? e_1 - e_0 : mid ? e_2 - e_0 : e_3 - e_2, P, pick(low, P1, P2));
+    iso[1] = corner(low || mid ? up : down, low ? e_2 - e_0 : mid ? e_3 - e_0 : e_3 - e_1, P, pick(low, P2, pick(mid, P3, P1)));
+    iso[2] = corner(low ? up : mid ? e_2 - energy : down, mid ? e_2 - e_1 : e_3 - e_0, pick(low, P0, pick(mid, P2, P3)),
+                    pick(low, P3, pick(mid, P1, P0)));
+    iso[3] = corner(energy - e_1, e_3 - e_1, P1, P3);  // n = 4 only
     // cyclic order around the centroid (order_cyclic, mesh_tetra.cpp:402-450).
     // Loops run to 4 with a guard so every array index is static (registers,
     // no scratch); the stable sort by angle becomes a stable rank.
@@ -217,7 +207,11 @@ __device__ __forceinline__ double tetra_dos_at(const TetraBand& T, double energy
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const V3 d = sub(iso[i], c);
-        ang[i] = i < n ? atan2(dot(d, v), dot(d, u)) : 0.0;
+        // y / (|x| + |y|), continued over the four quadrants: increases with the angle of
+        // (x, y) from -pi to pi, which is all that the ranks need
+        const double y = dot(d, v), x = dot(d, u), s = fabs(x) + fabs(y);
+        const double a = s > 0.0 ? y / s : 0.0;
+        ang[i] = i >= n ? 0.0 : x < 0.0 ? copysign(2.0, y) - a : a;
     }
     int rank[4];
 #pragma unroll
@@ -250,20 +244,26 @@ __device__ __forceinline__ double tetra_dos_at(const TetraBand& T, double energy
     if (!(A > 0.0)) return 0.0;
     // mean of 1/|grad E| at the polygon corners, gradients interpolated
     // barycentrically (interpolate_gradient_energy_at_band, mesh_tetra.cpp:214-230)
+    int c0 = T.v[0], c1 = T.v[1], c2 = T.v[2], c3 = T.v[3];
+    asm volatile("" : "+v"(c0), "+v"(c1), "+v"(c2), "+v"(c3));  // the corners again, not kept
+    const V3 p0 = load3(pos, c0);
+    const V3 edge[3] = {sub(load3(pos, c1), p0), sub(load3(pos, c2), p0), sub(load3(pos, c3), p0)};
+    const V3 grad[4] = {load3(Gb, c0), load3(Gb, c1), load3(Gb, c2), load3(Gb, c3)};
+    const double dt = det[t];
     double inv_grad_sum = 0.0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         if (i >= n) break;
-        const V3 v1 = sub(iso[i], T.p[0]);
-        const double l2 = triple(v1, T.edge[1], T.edge[2]) / T.det;
-        const double l3 = triple(v1, T.edge[2], T.edge[0]) / T.det;
-        const double l4 = triple(v1, T.edge[0], T.edge[1]) / T.det;
+        const V3 v1 = sub(iso[i], p0);
+        const double l2 = triple(v1, edge[1], edge[2]) / dt;
+        const double l3 = triple(v1, edge[2], edge[0]) / dt;
+        const double l4 = triple(v1, edge[0], edge[1]) / dt;
         const double l1 = 1.0 - l2 - l3 - l4;
         V3 g = {0.0, 0.0, 0.0};
-        g = add(g, scale(l1, T.g[0]));
-        g = add(g, scale(l2, T.g[1]));
-        g = add(g, scale(l3, T.g[2]));
-        g = add(g, scale(l4, T.g[3]));
+        g = add(g, scale(l1, grad[0]));
+        g = add(g, scale(l2, grad[1]));
+        g = add(g, scale(l3, grad[2]));
+        g = add(g, scale(l4, grad[3]));
         const double gn = norm(g);
         const double g_min = 1e-12;
         inv_grad_sum += 1.0 / (gn < g_min ? g_min : gn);
@@ -280,42 +280,72 @@ __device__ inline double wave_sum(double x) {
 
 __global__ void __launch_bounds__(kThreads) tetra_dos_kernel(
     const double* __restrict__ pos, const int32_t* __restrict__ tet, const double* __restrict__ det,
-    const int2* __restrict__ window, int64_t nt, int64_t per_slice, const double* __restrict__ Eb,
+    const uepm::TetraRange* __restrict__ range, int64_t nt, int64_t per_slice, const double* __restrict__ Eb,
     const double* __restrict__ Gb, double e0, double step, int n_points, double* __restrict__ partial) {
-    const int g0 = blockIdx.x * kEnergiesPerGroup;
-    const int g1 = min(g0 + kEnergiesPerGroup, n_points) - 1;
+    constexpr int NW = kThreads / 64, PT = kBlock / kThreads, NG = kEnergiesPerGroup;
+    static_assert(NG == NW && NG * PT * NW == 64, "one wave scans the counts and each sums one energy");
+    __shared__ double val[NG * kBlock];
+    __shared__ uint16_t list[NG * kBlock];
+    __shared__ int count[64];    // cutting tetrahedra by (energy, tetrahedron round, wave)
+    __shared__ int offset[65];   // their exclusive sums: where each group of the list starts
+    const int g0 = blockIdx.x * NG;
     const int64_t t_begin = blockIdx.y * per_slice;
     const int64_t t_end = min(nt, t_begin + per_slice);
-    double acc[kEnergiesPerGroup];
-#pragma unroll
-    for (int j = 0; j < kEnergiesPerGroup; ++j) acc[j] = 0.0;
-    for (int64_t t = t_begin + threadIdx.x; t < t_end; t += kThreads) {
-        const int2 w = window[t];
-        const int lo = max(w.x, g0), hi = min(w.y, g1);
-        if (lo > hi) continue;
-        TetraBand T;
-        load_tetra(T, pos, tet, det, Eb, Gb, t);
-        for (int i = lo; i <= hi; ++i) {
-            const double energy = e0 + static_cast<double>(i) * step;
-            const double c = tetra_dos_at(T, energy);
-#pragma unroll
-            for (int j = 0; j < kEnergiesPerGroup; ++j)
-                if (j == i - g0) acc[j] += c;
-        }
-    }
-    __shared__ double part[kThreads / 64][kEnergiesPerGroup];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double acc = 0.0;  // of energy g0 + wave, in lane 0
+    for (int64_t t0 = t_begin; t0 < t_end; t0 += kBlock) {
+        uint64_t cut[NG][PT];
 #pragma unroll
-    for (int j = 0; j < kEnergiesPerGroup; ++j) {
-        const double s = wave_sum(acc[j]);
-        if (lane == 0) part[wave][j] = s;
+        for (int k = 0; k < PT; ++k) {
+            const int64_t t = t0 + k * kThreads + threadIdx.x;
+            const uepm::TetraRange w = range[min(t, nt - 1)];
+#pragma unroll
+            for (int j = 0; j < NG; ++j) {
+                const int i = g0 + j;
+                const double energy = e0 + static_cast<double>(i) * step;
+                cut[j][k] = __ballot(t < t_end && i < n_points && w.lo <= i && i <= w.hi &&
+                                     !(energy < w.emin || energy > w.emax));
+                if (lane == 0) count[(j * PT + k) * NW + wave] = __popcll(cut[j][k]);
+            }
+        }
+        __syncthreads();
+        if (wave == 0) {
+            int s = count[lane];
+            for (int o = 1; o < 64; o <<= 1) {
+                const int u = __shfl_up(s, o, 64);
+                if (lane >= o) s += u;
+            }
+            offset[lane + 1] = s;
+            if (lane == 0) offset[0] = 0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < PT; ++k)
+#pragma unroll
+            for (int j = 0; j < NG; ++j)
+                if (cut[j][k] >> lane & 1)
+                    list[offset[(j * PT + k) * NW + wave] + __popcll(cut[j][k] & ((1ull << lane) - 1))] =
+                        static_cast<uint16_t>(k * kThreads + threadIdx.x);
+        __syncthreads();
+        const int total = offset[64];
+        for (int q = threadIdx.x; q < total; q += kThreads) {
+            int j = 0;
+            for (int u = 1; u < NG; ++u) j += q >= offset[u * PT * NW];
+            TetraBand T;
+            const int64_t t = t0 + list[q];
+            load_tetra(T, pos, tet, Eb, t);
+            val[q] = tetra_dos_at(T, pos, det, Gb, t, e0 + static_cast<double>(g0 + j) * step);
+        }
+        __syncthreads();
+        {
+            double s = 0.0;
+            const int q1 = offset[(wave + 1) * PT * NW];
+            for (int q = offset[wave * PT * NW] + lane; q < q1; q += 64) s += val[q];
+            acc += wave_sum(s);
+        }
+        // (the next block writes count before its first barrier, offset and list after it)
     }
-    __syncthreads();
-    if (threadIdx.x < kEnergiesPerGroup && g0 + (int)threadIdx.x < n_points) {
-        double s = 0.0;
-        for (int w = 0; w < kThreads / 64; ++w) s += part[w][threadIdx.x];
-        partial[blockIdx.y * (int64_t)n_points + g0 + threadIdx.x] = s;
-    }
+    if (lane == 0 && g0 + wave < n_points) partial[blockIdx.y * (int64_t)n_points + g0 + wave] = acc;
 }
 
 // Adds the slices in order and applies the mesh factors in the reference's
@@ -368,17 +398,17 @@ int tetra_dos_slices(int64_t nt, int n_points) {
 
 hipError_t launch_tetra_dos(const double* pos, const int32_t* tet, const double* det, const uint8_t* in_wedge,
                             int64_t nt, const double* Eb, const double* Gb, int n_points, double e_min, double e_max,
-                            double reduce_bz_factor, double spin_degeneracy, double wedge_factor, int2* window,
+                            double reduce_bz_factor, double spin_degeneracy, double wedge_factor, TetraRange* range,
                             double* partial, double* energies, double* dos, hipStream_t s) {
     const double step = (e_max - e_min) / static_cast<double>(n_points - 1);
     const int slices = tetra_dos_slices(nt, n_points);
     if (nt > 0) {
         const unsigned tb = static_cast<unsigned>((nt + kThreads - 1) / kThreads);
         hipLaunchKernelGGL(tetra_window_kernel, dim3(tb), dim3(kThreads), 0, s, tet, in_wedge, nt, Eb, e_min, step,
-                           n_points, window);
+                           n_points, range);
         const int64_t per_slice = (nt + slices - 1) / slices;
         const unsigned groups = static_cast<unsigned>((n_points + kEnergiesPerGroup - 1) / kEnergiesPerGroup);
-        hipLaunchKernelGGL(tetra_dos_kernel, dim3(groups, slices), dim3(kThreads), 0, s, pos, tet, det, window, nt,
+        hipLaunchKernelGGL(tetra_dos_kernel, dim3(groups, slices), dim3(kThreads), 0, s, pos, tet, det, range, nt,
                            per_slice, Eb, Gb, e_min, step, n_points, partial);
     }
     const unsigned fb = static_cast<unsigned>((n_points + kThreads - 1) / kThreads);
