@@ -84,10 +84,14 @@ UEPM_SC R dot_acc(q4<R> a, q4<R> b, R acc) {
 UEPM_SC R imag2(r1<R>) { return R(0); }
 UEPM_SC R imag2(c2<R> a) { return a.y * a.y; }
 UEPM_SC R imag2(q4<R> a) { return fma(a.y, a.y, fma(a.z, a.z, a.w * a.w)); }
-// no imaginary part
-UEPM_SC bool is_real(r1<R>) { return true; }
-UEPM_SC bool is_real(c2<R> a) { return a.y == R(0); }
-UEPM_SC bool is_real(q4<R> a) { return a.y == R(0) && a.z == R(0) && a.w == R(0); }
+// Whether a column whose elements below its first one, al, have the squared norm xn2
+// takes a reflector: not when they are all below 1e-15 (FP64: 1e-145), far under the
+// rounding of any matrix here, where 1 / |x|^2 (and |x|^2) would leave the range.  (NaN does.)
+template <typename S>
+__device__ __forceinline__ bool reflects(typename S::R xn2, S al) {
+    using R = typename S::R;
+    return !(xn2 + imag2(al) <= (sizeof(R) == 4 ? R(1e-30) : R(1e-290)));
+}
 
 // f a + b for a real f
 UEPM_SC r1<R> axpy(R f, r1<R> a, r1<R> b) { return {fma(f, a.x, b.x)}; }

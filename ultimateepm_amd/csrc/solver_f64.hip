@@ -238,7 +238,11 @@ __global__ __launch_bounds__(64, 2) void tri_vec_kernel(const double* __restrict
     }
     const double* d = dall + kk * n;
     const double* e = eall + kk * n;
-    const double lam = evals[t], tiny = DBL_EPSILON * tnorms[kk];
+    const double lam = evals[t];
+    // smallest pivot: under the rounding of T, and large enough that a run of equal
+    // levels with next to no coupling cannot grow the iterate out of range
+    const double tiny = fmax(0x1p-10 * DBL_EPSILON * tnorms[kk], DBL_MIN);
+    auto at_least_tiny = [&](double a) { return fabs(a) < tiny ? copysign(tiny, a) : a; };
     const int nblk = (n - 1 + kRows - 1) / kRows;  // blocks of eliminated rows 0 .. n - 2
     double* __restrict__ C = W + (size_t)2 * n * T;  // (a, c, y) at every block's first row
     struct State {
@@ -270,10 +274,11 @@ __global__ __launch_bounds__(64, 2) void tri_vec_kernel(const double* __restrict
             const double dn = r.d[u] - lam;
             const double en = k + 2 < n ? r.e[u + 1] : 0.0;
             const double y1 = first ? lane_rand((uint32_t)(k + 1), b) : r.y[u] * sc;
-            const bool keep = fabs(s.a) >= fabs(sub);
-            const double piv = keep ? (s.a == 0.0 ? tiny : s.a) : sub;
+            const double a = at_least_tiny(s.a);
+            const bool keep = fabs(a) >= fabs(sub);
+            const double piv = keep ? a : sub;
             const double rp = rcp_nr64(piv);
-            const double mult = (keep ? sub : s.a) * rp;
+            const double mult = (keep ? sub : a) * rp;
             const double u1 = keep ? s.c : dn, u2 = keep ? 0.0 : en;
             const double top = keep ? s.y : y1, bot = keep ? y1 : s.y;
             s.a = (keep ? dn : s.c) - mult * u1;
@@ -301,7 +306,7 @@ __global__ __launch_bounds__(64, 2) void tri_vec_kernel(const double* __restrict
             if (last) z[k] = x;
             else Xout[(size_t)k * T + t] = x;
         };
-        double x1 = s.y * rcp_nr64(s.a == 0.0 ? tiny : s.a), x2 = 0.0;
+        double x1 = s.y * rcp_nr64(at_least_tiny(s.a)), x2 = 0.0;
         put(n - 1, x1);
         double amax = fabs(x1);
         for (int blk = nblk - 1; blk >= 0; --blk) {

@@ -9,24 +9,30 @@
 // i = r + 32 l, j = c + 16 m (cyclic in both directions, so every lane keeps
 // a share of the shrinking trailing matrix until the end).  Only blocks
 // (l, m) that can hold i >= j are stored: 42 complex values per lane at
-// dim <= 192.  Blocks below the 32 x 32 diagonal super-blocks hold A(i, j);
-// the two blocks of a row block that lie in its diagonal super-block hold
-// A(i, j) / 2 for every element, above the diagonal too, so that each pair
-// (i, j), (j, i) of a super-block is stored twice at half weight.  The
-// symmetric product then treats every stored element alike: A(i, j) feeds
-// row i (A v_j) and column j (conj(A) v_i).  A grid whose blocks
+// dim <= 192.  The blocks of a row block that lie in its diagonal super-block
+// (32 x 32) hold both triangles: their elements feed row i of the symmetric product
+// only (A v_j), the elements of the other blocks row i and column j (conj(A) v_i).
+// A grid whose blocks
 // do not all fit its register budget keeps its last NL blocks in LDS instead,
 // in lane-private slots (slot-major, so a wave's accesses are consecutive).
 //
-// Step s (LAPACK xHETD2, lower, restated; H_s = I - tau v v^H, v[s+1] = 1):
-//   a. the lanes of column s put x = A(s+1:, s) in LDS              | barrier
-//   b. every wave forms beta, tau, v from x (redundantly)
-//   c. y = A v: row sums across the 16 lanes of a row group (DPP), column
+// Step s (LAPACK xHETD2, lower, restated; H_s = I - tau v v^H, v[s+1] = 1, and
+// v = u sc with u = A(s+1:, s) but for u[s+1] = alpha - beta):
+//   a. the lanes of column s put A(s+1:, s) in LDS                   | barrier
+//   b. every wave forms beta, tau, sc from it (redundantly)
+//   c. y = A u: row sums across the 16 lanes of a row group (DPP), column
 //      sums across the 4 row groups of a wave (row swaps), one
-//      partial per wave in LDS; each lane also sums its share of v^H A v,
-//      so p^H v = conj(tau) v^H A v needs no separate dot product      | barrier
+//      partial per wave in LDS; each lane also sums its share of u^H A u,
+//      so w^H u needs no separate dot product                         | barrier
 //   d. y = sum of the partials, one row per lane                       | barrier
-//   e. w = tau y - (1/2)|tau|^2 (v^H A v) v; A -= v w^H + w v^H on the live blocks
+//   e. w = y ts - (1/2)|ts|^2 (u^H A u) u with ts = sc tau conj(sc);
+//      A -= u w^H + w u^H on the live blocks
+// (u is the column itself: rows and columns of it are read from LDS where v would be a
+// product and a select each.  With that, and the diagonal super-blocks at full weight on
+// one side instead of at half weight on both: quaternions 128 -> 96, 3000 k-points, 2.55
+// -> 2.26 ms in FP32, 961 in FP64 1.69 -> 1.53; complex64 160 -> 128, 4096, two chunks in
+// flight, 2.43 -> 2.35; real 181 -> 128 2.51 -> 2.44.  The three barriers of a step and
+// the chains between them bound the small elements, issue the quaternions.)
 // Blocks whose columns are all <= s are skipped (one wave-uniform test per
 // block column: a stored block's rows are live while its columns are).
 // Outputs match the LDS-blocked reduction: d, e (real), tau, reflectors below
@@ -146,7 +152,7 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
     // LOW variant still reads the column of step s in its update phase while a
     // wave ahead may write the column of step s + 1 (no barrier in between)
     __shared__ S Xbuf[2][NX];
-    __shared__ R XD[NX];      // diagonal entries of column s as stored (A(s, s) / 2 at row s)
+    __shared__ S XC[NX];      // column s as it is (rows of its diagonal super-block and below)
     __shared__ S RP[NX];      // row sums of the symmetric product
     __shared__ S CP[NW][NXC];  // column sums, one row per wave
     __shared__ S Y[NX];       // y = A v, zero at rows <= s and >= n
@@ -167,7 +173,7 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
     VT* tau_o = tauout + kk * de_kstride;
     const int s_stop = s_end < n - 1 ? s_end : n - 1;
 
-    // ---- load: below the diagonal super-blocks A(i, j), inside them A(i, j) / 2 ----
+    // ---- load ----
     S A[NR];
     // slot i of this lane (i is a compile-time constant wherever these are used)
     auto aget = [&](int i) -> S {
@@ -196,8 +202,7 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
                 const bool up = i < j;
                 const int p = up ? j : i, q = up ? i : j;
                 const THin h = H[IN == 0 ? p + (int64_t)q * ld : q + (int64_t)p * ld];
-                const R f = Lay::straddles(l, m) ? R(0.5) : R(1);
-                a = scale(conj_if(sc_load<S>(h), (IN == 1) != up), f);
+                a = conj_if(sc_load<S>(h), (IN == 1) != up);
             }
             aset(Lay::idx(l, m), a);
         }
@@ -219,9 +224,8 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
                         const int i = r + PR * l;
                         if (m <= Lay::mmax(l)) {
                             const S a = aget(Lay::idx(l, m));
-                            const R f = Lay::straddles(l, m) ? R(2) : R(1);
-                            X[i] = sel(i > s, scale(a, f), zero);
-                            XD[i] = a.x;
+                            X[i] = sel(i > s, a, zero);
+                            XC[i] = a;
                         } else {
                             X[i] = zero;  // block above the diagonal: rows < s
                         }
@@ -240,57 +244,64 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
             part += i < NX ? t : R(0);
         }
         const R xn2 = wave::sum(part);
-        // tau = (beta - alpha) / beta, sc = 1 / (alpha - beta)
-        const S al = X[s + 1];
+        // tau = (beta - alpha) / beta, sc = 1 / (alpha - beta); v = u sc with u the column
+        // and alpha - beta in front, which is what the rest of the step works with:
+        // tau v v^H = u ts u^H, ts = sc tau conj(sc), and ts takes tau's place throughout.
+        const S al = XC[s + 1];
         R beta = al.x;
-        S tau{}, sc = one;
-        if (!(xn2 == R(0) && is_real(al))) {
+        S tau{}, sc = one, ts{};
+        R iden = 0;  // |sc|^2
+        if (reflects(xn2, al)) {
             const R nrm = sqrt(dot_acc(al, al, xn2));
             beta = al.x >= R(0) ? -nrm : nrm;
             const R ib = rcp_full(beta);
             tau = scale(al, -ib);
             tau.x = (beta - al.x) * ib;
-            const R br = al.x - beta, iden = rcp_full(fma(br, br, imag2(al)));
+            const R br = al.x - beta;
+            iden = rcp_full(fma(br, br, imag2(al)));
             sc = scale(conj_if(al, true), iden);
             sc.x = br * iden;
+            ts = mul(mul(sc, tau), conj_if(sc, true));
         }
         if (tid == 0) {
-            d[s] = 2.0 * (double)XD[s];
+            d[s] = (double)XC[s].x;
             e[s] = (double)beta;
             tau_o[s] = sc_store<S>(tau);
         }
+        // every wave puts u's first element in place, for itself: the others write the
+        // same, and read X[s + 1] only after their own write
+        if (lane == 0) {
+            S u0 = al;
+            u0.x = al.x - beta;
+            X[s + 1] = u0;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
         for (int q = 0; q < NYT; ++q) {
             const int i = s + 2 + tid + q * BS;
             if (i < n) Vk[i + (int64_t)s * ldv] = sc_store<S>(mul(X[i], sc));
         }
-        // v at this lane's rows and columns (X is zero outside s+1..n-1; loads
+        // u at this lane's rows and columns (X is zero outside s+1..n-1; loads
         // unconditional so they issue together)
-        // LOW (fewer registers, for two workgroups per CU): the column values of v and
-        // w are formed from LDS where they are used instead of being kept, and each
+        // LOW (fewer registers, for two workgroups per CU): the column values of u and
+        // w are read from LDS where they are used instead of being kept, and each
         // pair of block columns is reduced as soon as its partial sums are complete
         // (the same operations in the same order)
-        auto vcol = [&](int m) -> S {
-            const int j = c + PC * m;
-            return sel(j == s + 1, one, mul(X[j], sc));
-        };
+        auto vcol = [&](int m) -> S { return X[c + PC * m]; };
         S vr[LR], vc[LOW ? 1 : LC];
 #pragma unroll
-        for (int l = 0; l < LR; ++l) {
-            const int i = r + PR * l;
-            const S v = mul(X[i], sc);
-            vr[l] = sel(i == s + 1, one, v);
-        }
+        for (int l = 0; l < LR; ++l) vr[l] = X[r + PR * l];
         if constexpr (!LOW) {
 #pragma unroll
             for (int m = 0; m < LC; ++m) vc[m] = vcol(m);
         }
-        // ---- c. y = A v on the live blocks; local share of v^H A v ----
+        // ---- c. y = A u on the live blocks; local share of u^H A u ----
         S rp[LR], cp[LOW ? GC : NXC / PC];
 #pragma unroll
         for (int l = 0; l < LR; ++l) rp[l] = zero;
 #pragma unroll
         for (int m = 0; m < (LOW ? GC : NXC / PC); ++m) cp[m] = zero;
+        R qv = 0;
         const int q4 = lane >> 4;
         R* cpw = &CP[wv][0].x;
         // column sums of GC block columns from m on: lane row q holds component
@@ -311,9 +322,12 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
                 for (int l = Lay::lmin(m); l < LR; ++l) {
                     const S a = aget(Lay::idx(l, m));
                     fma_ab(rp[l], a, vcm);
-                    fma_cab(cp[mc], a, vr[l]);
+                    if (!Lay::straddles(l, m)) fma_cab(cp[mc], a, vr[l]);
                 }
             }
+            // row block m / Q: its diagonal super-block, now complete, counts half in u^H A u
+            if (m % Lay::Q == 0 && m + Lay::Q - 1 >= m0)
+                qv = dot_acc(vr[Lay::lmin(m)], scale(rp[Lay::lmin(m)], R(-0.5)), qv);
             if constexpr (LOW) {
                 if (m % GC == 0) {
                     if (m + GC - 1 >= m0) col_sums(m, cp);
@@ -322,8 +336,8 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
                 }
             }
         }
-        // sum over stored elements of conj(v_i) A_ij v_j; v^H A v = 2 Re of its total
-        R qv = 0;
+        // half of u^H A u: the sum of conj(u_i) A_ij u_j over the blocks below the diagonal
+        // super-blocks and half of it over those
 #pragma unroll
         for (int l = 0; l < LR; ++l)
             if (l >= l0) qv = dot_acc(vr[l], rp[l], qv);
@@ -366,40 +380,32 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
             R vav = 0;
 #pragma unroll
             for (int w = 0; w < NW; ++w) vav += Q[w];
-            const R alpha = -dot_acc(tau, tau, R(0)) * vav;  // v^H A v = 2 vav
-            const S v = sel(i == s + 1, one, mul(X[i], sc));
-            Y[i] = axpy(alpha, v, mul(y, tau));
-            RP[i] = v;
+            const R alpha = -dot_acc(tau, tau, R(0)) * (iden * (iden * vav));  // -(1/2)|ts|^2 u^H A u
+            Y[i] = axpy(alpha, X[i], mul(y, ts));
         }
         __syncthreads();
-        // ---- e. rank-2 update A -= v w^H + w v^H, at half weight in the diagonal super-blocks ----
-        S wr[LR], vh[LR], wh[LR];
+        // ---- e. rank-2 update A -= u w^H + w u^H ----
+        S wr[LR];
 #pragma unroll
-        for (int l = 0; l < LR; ++l) {
-            wr[l] = Y[r + PR * l];
-            vh[l] = scale(vr[l], R(0.5));
-            wh[l] = scale(wr[l], R(0.5));
-        }
+        for (int l = 0; l < LR; ++l) wr[l] = Y[r + PR * l];
 #pragma unroll
         for (int m = LC - 1; m >= 0; --m) {
             if (m >= m0) {
-                const S vcm = LOW ? RP[c + PC * m] : vc[LOW ? 0 : m];
+                const S vcm = LOW ? vcol(m) : vc[LOW ? 0 : m];
                 const S wcm = Y[c + PC * m];
 #pragma unroll
                 for (int l = Lay::lmin(m); l < LR; ++l) {
-                    // a -= v_i conj(w_j) + w_i conj(v_j)
-                    const bool half = Lay::straddles(l, m);
-                    const S vi = half ? vh[l] : vr[l], wi = half ? wh[l] : wr[l];
+                    // a -= u_i conj(w_j) + w_i conj(u_j)
                     S a = aget(Lay::idx(l, m));
-                    fms_abc(a, vi, wcm);
-                    fms_abc(a, wi, vcm);
+                    fms_abc(a, vr[l], wcm);
+                    fms_abc(a, wr[l], vcm);
                     aset(Lay::idx(l, m), a);
                 }
             }
         }
     }
     if (s_stop < n - 1) {
-        // hand the trailing block A[s_stop:, s_stop:] over (diagonal stored halved)
+        // hand the trailing block A[s_stop:, s_stop:] over
         VT* B = Bout + kk * (int64_t)ldb * ldb;
 #pragma unroll
         for (int l = 0; l < LR; ++l)
@@ -407,8 +413,7 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
             for (int m = 0; m <= Lay::mmax(l); ++m) {
                 const int i = r + PR * l, j = c + PC * m;
                 if (i < n && j >= s_stop && i >= j) {
-                    const R f = Lay::straddles(l, m) ? R(2) : R(1);
-                    const S a = scale(aget(Lay::idx(l, m)), f);
+                    const S a = aget(Lay::idx(l, m));
                     B[(j - s_stop) + (int64_t)(i - s_stop) * ldb] = sc_store<S>(a);
                     if constexpr (FULL) B[(i - s_stop) + (int64_t)(j - s_stop) * ldb] = sc_store<S>(conj_if(a, true));
                 }
@@ -424,7 +429,7 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
             if (m == ms)
 #pragma unroll
                 for (int l = 0; l < LR; ++l)
-                    if (m <= Lay::mmax(l) && c == cs && r + PR * l == s) d[s] = 2.0 * (double)aget(Lay::idx(l, m)).x;
+                    if (m <= Lay::mmax(l) && c == cs && r + PR * l == s) d[s] = (double)aget(Lay::idx(l, m)).x;
         if (tid == 0) {
             e[s] = 0.0;
             tau_o[s] = sc_store<S>(zero);

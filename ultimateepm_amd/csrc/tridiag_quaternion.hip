@@ -48,7 +48,7 @@ void stage(const q4<double>* H0, const q4<R>* Hb, int64_t hk, int n, int64_t nk,
             }
         } else {
             switch (kSize[stage_of(n)]) {
-                case 160: UEPM_GRID(5, 2, 6); break;
+                case 160: UEPM_GRID(5, 2, 5); break;
                 case 128: UEPM_GRID(4, 2, 0); break;
                 case 96: UEPM_GRID(3, 2, 0); break;
                 default: UEPM_GRID(2, 4, 0); break;

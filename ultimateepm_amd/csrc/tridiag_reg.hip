@@ -76,7 +76,7 @@ __global__ __launch_bounds__(64, 2) void tridiag_wave64_kernel(const THin* __res
         const float aly = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x.y), s + 1));
         const float dss = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x.x), s));
         float beta = alx, tr = 0, ti = 0, sr = 1, si = 0;
-        if (!(xn2 == 0.f && aly == 0.f)) {
+        if (reflects(xn2, c2<float>{alx, aly})) {
             const float nrm = sqrtf(fmaf(alx, alx, fmaf(aly, aly, xn2)));
             beta = alx >= 0.f ? -nrm : nrm;
             const float ib = rcp_full(beta);

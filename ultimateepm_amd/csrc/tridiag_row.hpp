@@ -158,7 +158,7 @@ __global__ __launch_bounds__(64 * RW * CW, MINW) void tridiag_row_kernel(
         const R xn2 = wave::sum(part);
         R beta = al.x;
         S tau{}, sc = one;
-        if (!(xn2 == R(0) && is_real(al))) {
+        if (reflects(xn2, al)) {
             const R nrm = sqrt(dot_acc(al, al, xn2));
             beta = al.x >= R(0) ? -nrm : nrm;
             const R ib = rcp_full(beta);

@@ -168,7 +168,7 @@ __global__ __launch_bounds__(512, 2) void tridiag_strip_kernel(const THin* __res
         const S al = X[s + 1];
         float beta = al.x;
         S tau{}, sc = one;
-        if (!(xn2 == 0.f && is_real(al))) {
+        if (reflects(xn2, al)) {
             const float nrm = sqrt(dot_acc(al, al, xn2));
             beta = al.x >= 0.f ? -nrm : nrm;
             const float ib = rcp_full(beta);
