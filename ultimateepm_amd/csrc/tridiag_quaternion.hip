@@ -4,7 +4,10 @@
 // for a 2N x 2N complex one.  Half the multiply-adds, half the elements and half
 // the steps; the N x N tridiagonal T holds each Kramers pair of levels once.
 // The grids of tridiag_grid.hpp in quaternion arithmetic, shrinking as the
-// complex chain does (tridiag_reg.hip).
+// complex chain does (tridiag_reg.hip).  Shapes are the fastest of a sweep; 32 steps of
+// 2048 matrices, ms, 32 x 16 lanes against 16 x 16: FP32 160 1.98, 2.21; 128 1.50 (1.19 with
+// 6 of 20 blocks in LDS), 1.15; 96 0.74, 0.63; 64 (63 steps) 0.68, 0.49; FP64 128 2.48 (2.74
+// with no blocks in LDS), too large; 96 1.69, 1.33; 64 1.31, 1.05.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -36,22 +39,22 @@ void stage(const q4<double>* H0, const q4<R>* Hb, int64_t hk, int n, int64_t nk,
     using S = q4<R>;
     auto grid = [&](const auto* H) {
         using THin = std::remove_const_t<std::remove_pointer_t<decltype(H)>>;
-#define UEPM_GRID(lr, w, nl)                                                                                            \
-    reg_stage<S, 32, lr, w, IN, THin, true, nl>(H, hk, n, n, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s)
+#define UEPM_GRID(pr, lr, w, nl)                                                                                            \
+    reg_stage<S, pr, lr, w, IN, THin, true, nl>(H, hk, n, n, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s)
         if constexpr (sizeof(R) == sizeof(float)) {
             switch (kSize[stage_of(n)]) {
-                case 192: UEPM_GRID(6, 2, 0); break;
-                case 160: UEPM_GRID(5, 2, 0); break;
-                case 128: UEPM_GRID(4, 2, 0); break;
-                case 96: UEPM_GRID(3, 4, 0); break;
-                default: UEPM_GRID(2, 6, 0); break;
+                case 192: UEPM_GRID(32, 6, 2, 0); break;
+                case 160: UEPM_GRID(32, 5, 2, 0); break;
+                case 128: UEPM_GRID(16, 8, 2, 0); break;
+                case 96: UEPM_GRID(16, 6, 3, 3); break;
+                default: UEPM_GRID(16, 4, 4, 0); break;
             }
         } else {
             switch (kSize[stage_of(n)]) {
-                case 160: UEPM_GRID(5, 2, 5); break;
-                case 128: UEPM_GRID(4, 2, 0); break;
-                case 96: UEPM_GRID(3, 2, 0); break;
-                default: UEPM_GRID(2, 4, 0); break;
+                case 160: UEPM_GRID(32, 5, 2, 5); break;
+                case 128: UEPM_GRID(32, 4, 2, 4); break;
+                case 96: UEPM_GRID(16, 6, 2, 6); break;
+                default: UEPM_GRID(16, 4, 2, 0); break;
             }
         }
 #undef UEPM_GRID

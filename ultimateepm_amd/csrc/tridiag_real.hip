@@ -45,8 +45,9 @@ int next(int n) {
 // sweep that did not spill in the steps; 16 x 16 lanes where a grid fits their
 // registers (four waves meet at a barrier instead of eight), 32 x 16 above.
 // Measured, ms per 32 steps and 2048 matrices: FP32 448: 3.04, 384: 2.24, 320:
-// 1.73, 288: 1.09, 256: 0.77, 224: 0.66; FP64 320: 2.53, 288: 1.87, 256: 1.54,
-// 224: 1.35.  Per 4096: FP32 192 (53 steps): 1.36, 128 (64 steps): 0.55 (grid:
+// 1.73, 288: 1.09, 256: 0.77, 224: 0.62 (16 x 16 lanes: the same), 160: 0.31; FP64 320: 2.53, 288: 1.87, 256: 1.54,
+// 224: 1.35, 160: 0.52 (0.58 without blocks in LDS).  Per 4096: FP32 192 (53 steps):
+// 1.17 (1.43 at three waves per SIMD without), 128 (64 steps): 0.55 (grid:
 // 0.71), 64: 0.15; FP64 2.19, 1.01 (grid: 1.31), 0.19.
 template <typename THin>
 void stage(const THin* H, int64_t hk, int n, int ld, int64_t nk, float* V, int ldv, int64_t vk, double* dd, double* de,
@@ -64,7 +65,7 @@ void stage(const THin* H, int64_t hk, int n, int ld, int64_t nk, float* V, int l
         case 288: UEPM_GRID(32, 9, 4, 1, THin, true, 8, true); break;
         case 256: UEPM_GRID(32, 8, 4, 1, THin, true, 0, true); break;
         case 224: UEPM_GRID(32, 7, 4, 1, THin, false, 0, true); break;
-        case 192: UEPM_GRID(16, 12, 3, 1, THin, false, 0, true); break;
+        case 192: UEPM_GRID(16, 12, 4, 1, THin, true, 16, true); break;
         case 160:
             if constexpr (kFromH) UEPM_GRID(16, 10, 4, 1, THin, false, 0, true);
             break;
@@ -88,7 +89,7 @@ void stage(const double* H, int64_t hk, int n, int ld, int64_t nk, double* V, in
         case 256: UEPM_GRID(32, 8, 2, 1, double, true, 0, true); break;
         case 224: UEPM_GRID(32, 7, 2, 1, double, true, 0, true); break;
         case 192: UEPM_GRID(16, 12, 2, 1, double, true, 0, true); break;
-        case 160: UEPM_GRID(16, 10, 2, 1, double, true, 0, true); break;
+        case 160: UEPM_GRID(16, 10, 3, 1, double, true, 16, true); break;
         case 128: UEPM_ROWS(2, 2, 4, 2); break;
         case 96: UEPM_ROWS(2, 1, 6, 2); break;
         default: UEPM_ROWS(1, 1, 4, 3); break;

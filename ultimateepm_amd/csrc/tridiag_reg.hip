@@ -161,19 +161,19 @@ __global__ __launch_bounds__(64, 2) void tridiag_wave64_kernel(const THin* __res
     }
 }
 
-// n <= 64: 2 x 4 blocks; n <= 128: 4 x 8; n <= 192: 6 x 12; n <= 256: 8 x 16;
-// n <= 288: 9 x 18 (rows x columns of the 32 x 16 grid)
 int tridiag_reg_max_n() { return 288; }
 
 // Hand-over between grids.  The late steps of a large grid carry its full
 // per-step overhead for a small trailing matrix, so each grid stops where the
-// next smaller one can take the trailing block: 288-grid (9 x 18 blocks) ->
-// 256 (8 x 16) -> 224 (7 x 14) -> 192 (6 x 12) -> 160 (5 x 10) -> 128 (4 x 8)
-// -> 96 (3 x 6) -> 64 (2 x 4).  Register budgets (workgroups per CU): 288
-// low-register, 256 VGPRs with 16 of its 90 blocks in LDS (1); 256 and 224
-// low-register, 256 and 223 VGPRs (1); 192 low-register, 128 VGPRs with 14 of
-// its 42 blocks in LDS (2); 160 low-register, 128 VGPRs (2); 128 at 128 VGPRs
-// (2); 96 low-register, 80 (3); 64 low-register, 63 (4).
+// next smaller one can take the trailing block: 288 -> 256 -> 224 -> 192 -> 160 ->
+// 128 -> 96 -> 64 (one wave).  From 160 down the lanes are 16 x 16, not 32 x 16: four waves
+// meet at a step's barriers instead of eight and twice the workgroups share a CU, so
+// one's barriers and chains hide behind another's work.  Low-register form throughout
+// but for 96, blocks in LDS where that is what one more workgroup takes.  VGPRs and
+// workgroups per CU: 288: 256, 16 of 90 blocks in LDS (1); 256: 244 (1); 224: 204 (1); 192:
+// 128, 14 of 42 blocks in LDS (2); 160: 168, 12 of 55 (3); 128: 128, 10 of 36 (4); 96: 127
+// (4).  32 steps of 2048 matrices, 32 x 16 -> 16 x 16 lanes: 160 0.68 -> 0.63 ms, 128 0.51 ->
+// 0.41, 96 0.32 -> 0.26; at 192 (21 steps) 32 x 16 stays the faster, 0.65 against 0.74.
 namespace {
 constexpr int kNumGrids = 8;
 constexpr int kGrid[kNumGrids] = {288, 256, 224, 192, 160, 128, 96, 64};
@@ -207,7 +207,7 @@ void wave64_stage(const THin* H, int64_t h_kstride, int n, int ld, int64_t nk, f
                        v_kstride, dd, de, dtau, de_kstride);
 }
 
-constexpr int NL288 = 16, NL192 = 14;  // blocks held in LDS by the 288- and 192-wide grids
+constexpr int NL288 = 16, NL192 = 14, NL160 = 12, NL128 = 10;  // blocks held in LDS by these grids
 
 template <typename THin, int IN>
 void grid_stage(int g, const THin* H, int64_t hk, int m, int ld, int64_t nk, float2* V, int ldv, int64_t vk,
@@ -217,9 +217,9 @@ void grid_stage(int g, const THin* H, int64_t hk, int m, int ld, int64_t nk, flo
         case 1: reg_stage<c2<float>, 32, 8, 2, IN, THin, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         case 2: reg_stage<c2<float>, 32, 7, 2, IN, THin, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         case 3: reg_stage<c2<float>, 32, 6, 4, IN, THin, true, NL192>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 4: reg_stage<c2<float>, 32, 5, 4, IN, THin, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 5: reg_stage<c2<float>, 32, 4, 4, IN, THin>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 6: reg_stage<c2<float>, 32, 3, 6, IN, THin, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        case 4: reg_stage<c2<float>, 16, 10, 3, IN, THin, true, NL160>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        case 5: reg_stage<c2<float>, 16, 8, 4, IN, THin, true, NL128>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        case 6: reg_stage<c2<float>, 16, 6, 4, IN, THin>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         default: wave64_stage<IN, THin>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s); break;  // last: s_end >= m - 1
     }
 }
@@ -306,12 +306,13 @@ hipError_t launch_tridiag_reg_c64_block(const float2* H, int64_t hk, int m, int 
     return c64_chain<0>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, work, s);
 }
 
-// ---- FP64: grids 192 (6 x 12, low-register, 256 VGPRs with a small spill), 160
-// (5 x 10, low-register) and 128 (4 x 8), one workgroup per CU; 96 (3 x 6,
-// low-register, 128 VGPRs), two.  The last 64 steps run one row per lane in two
+// ---- FP64: grids 192 (10 of 42 blocks in LDS) and 160 of 32 x 16 lanes, 256 and 236
+// VGPRs, one workgroup per CU; 128 and 96 of 16 x 16 lanes, two and three (32 steps of
+// 2048 matrices, 32 x 16 -> 16 x 16 lanes: 128 1.15 -> 0.80 ms, 96 0.62 -> 0.49; 160 1.55
+// against 1.65; one matrix alone takes a tenth longer on half the lanes).  The last 64 steps run one row per lane in two
 // column waves, four workgroups per CU (tridiag_row.hpp; 4096 blocks of 64 take
 // 0.59 ms, a 2 x 4 grid 1.48; blocks of 27 in one wave 0.14; at 96 the grid is
-// the faster, 1.27 ms for 32 steps against 1.50).  A larger FP64 matrix runs the
+// the faster, 1.0 ms for 32 steps against 1.50).  A larger FP64 matrix runs the
 // blocked reduction first and hands over its trailing block at a panel boundary.
 namespace {
 constexpr int kNumGrids64 = 5;
@@ -325,16 +326,16 @@ int split64(int n) {
     const int g = grid64_of(n);
     return g < kNumGrids64 - 1 ? kGrid64[g + 1] : 0;
 }
-constexpr int NL64_192 = 10, NL64_96 = 2;  // blocks held in LDS by the 192- and 96-wide FP64 grids
+constexpr int NL64_192 = 10, NL64_128 = 2, NL64_96 = 4;  // blocks held in LDS by these FP64 grids
 template <int IN>
 void grid64_stage(int g, const double2* H, int64_t hk, int m, int ld, int64_t nk, double2* V, int ldv, int64_t vk,
                   double* dd, double* de, double2* dtau, int64_t dk, int s_end, double2* B, int ldb, hipStream_t s) {
     switch (g) {
         case 0: reg_stage<c2<double>, 32, 6, 1, IN, double2, true, NL64_192>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         case 1: reg_stage<c2<double>, 32, 5, 1, IN, double2, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 2: reg_stage<c2<double>, 32, 4, 1, IN, double2>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        case 2: reg_stage<c2<double>, 16, 8, 2, IN, double2, true, NL64_128>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         // hands both triangles to the row kernel
-        case 3: reg_stage<c2<double>, 32, 3, 4, IN, double2, true, NL64_96, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        case 3: reg_stage<c2<double>, 16, 6, 3, IN, double2, true, NL64_96, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         default:
             if constexpr (IN != 0) {
                 if (m <= 32) row_stage<c2<double>, 1, 1, 2, 2, IN>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
