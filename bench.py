@@ -31,6 +31,10 @@ FP32_MFMA_PEAK_TFLOPS = 157.3
 DATAPATH = {
     ("mixed", "tridiag_reg_kernel"): "VALU FP32 (157.3 TF/s, the FP32 MFMA rate too): no MFMA in the register-grid chain",
     ("fp64", "tridiag_reg_kernel"): "VALU FP64 (78.6 TF/s, equal to the FP64 MFMA rate)",
+    ("mixed", "tridiag_real"): "VALU FP32 (157.3 TF/s, the FP32 MFMA rate too): no MFMA in the reductions",
+    ("fp64", "tridiag_real"): "VALU FP64 (78.6 TF/s, equal to the FP64 MFMA rate)",
+    ("mixed", "tridiag_quaternion"): "VALU FP32 (157.3 TF/s, the FP32 MFMA rate too): no MFMA in the reductions",
+    ("fp64", "tridiag_quaternion"): "VALU FP64 (78.6 TF/s, equal to the FP64 MFMA rate)",
     ("mixed", "tridiag_blocked_kernel"): "VALU FP32 symmetric products, MFMA FP32 panel updates (157.3 TF/s either way)",
     ("mixed", "tridiag_blocked+reg_kernel"): "VALU FP32 symmetric products, MFMA FP32 panel updates, then the register grids",
     ("mixed", "tridiag_strip+reg_kernel"): "VALU FP32 (157.3 TF/s, the FP32 MFMA rate too): no MFMA in the register-grid chain",
@@ -46,9 +50,12 @@ def log(msg: str) -> None:
     print(f"[bench {time.strftime('%H:%M:%S')}] {msg}", file=sys.stderr, flush=True)
 
 
-def tridiag_flops(n: int) -> float:
-    """Algorithmic real flops of the Hermitian Householder reduction: (16/3) n^3."""
-    return 16.0 / 3.0 * n ** 3
+def tridiag_flops(n: int, kernel: str = "") -> float:
+    """Algorithmic real flops of the Householder reduction that `kernel` runs: (16/3) n^3
+    of a complex Hermitian matrix, (4/3) n^3 of a real one (an inversion centre, no
+    spin-orbit), (8/3) n^3 of the quaternions of a spinor one (an inversion centre)."""
+    third = 4.0 if kernel.startswith("tridiag_real") else 8.0 if kernel.startswith("tridiag_quaternion") else 16.0
+    return third / 3.0 * n ** 3
 
 
 def host_cpu() -> dict:
@@ -732,7 +739,7 @@ def main() -> int:
     dominant = max(stage_ms, key=lambda k: stage_ms[k][0])
     dom_ms, dom_launches = stage_ms[dominant]
     if dominant.startswith("tridiag"):
-        flops = tridiag_flops(r["dim"]) * args.nk * ts
+        flops = tridiag_flops(r["dim"], dominant) * args.nk * ts
         peak = FP32_MFMA_PEAK_TFLOPS if head == "mixed" else FP64_PEAK_TFLOPS
     else:
         flops = 0.0
@@ -741,7 +748,8 @@ def main() -> int:
     # the reduction's flops of a whole step over that step's wall time (timing off):
     # the chip-level rate with both lanes in flight and every other stage included
     step_s = r["elapsed"] / args.steps
-    chip = tridiag_flops(r["dim"]) * args.nk / step_s / 1e12
+    reduction = next((k for k in stage_ms if k.startswith("tridiag")), dominant)
+    chip = tridiag_flops(r["dim"], reduction) * args.nk / step_s / 1e12
     roofline = {
         "kernel": dominant,
         "bound": "mfma",
@@ -752,7 +760,7 @@ def main() -> int:
         "traffic": None,
         "avg_launch_ms": round(dom_ms / max(dom_launches, 1), 4),
         "k_per_launch": round(args.nk * ts / max(dom_launches, 1), 1),
-        "flop_per_k": tridiag_flops(r["dim"]),
+        "flop_per_k": tridiag_flops(r["dim"], reduction),
         "datapath": DATAPATH.get((head, dominant.split("<")[0]), "not listed for this kernel"),
         "stage_ms_per_step": {k: round(v[0] / ts, 3) for k, v in stage_ms.items()},
         "launches_in_flight": r["lanes"],
@@ -787,7 +795,7 @@ def main() -> int:
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "c64+f64" if head == "mixed" else "f64",
+        "dtype": ("f32+f64" if reduction.startswith("tridiag_real") else "c64+f64") if head == "mixed" else "f64",
         "data": "synthetic",
         "config": {
             "workload": f"Si non-local (materials.yaml), n={args.shells} shells (N={N}), {args.nk} seeded "
