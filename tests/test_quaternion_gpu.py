@@ -63,7 +63,8 @@ def test_which_plans_are_quaternion(gpu_ctx):
 # the first ones above the quaternion kernels' range; odd and even band counts
 @pytest.mark.parametrize("ng,nb,mixed", [(1, 2, False), (1, 1, True), (2, 3, False), (17, 7, True), (64, 9, False),
                                          (65, 8, False), (64, 24, True), (65, 23, True), (96, 4, False), (97, 35, False),
-                                         (128, 5, True), (129, 6, False), (160, 7, False), (161, 6, False),
+                                         (128, 5, True), (129, 6, False), (129, 6, True), (144, 6, False), (144, 5, True),
+                                         (145, 6, False), (145, 6, True), (160, 7, False), (161, 6, False),
                                          (161, 16, True), (192, 11, True), (193, 12, True)])
 def test_quaternion_matches_general(gpu_ctx, ng, nb, mixed):
     print(f"case: quaternion against general, Ge, {ng} vectors, {nb} bands, mixed {mixed}", flush=True)

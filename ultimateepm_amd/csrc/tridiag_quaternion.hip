@@ -5,7 +5,9 @@
 // the steps; the N x N tridiagonal T holds each Kramers pair of levels once.
 // The grids of tridiag_grid.hpp in quaternion arithmetic, shrinking as the
 // complex chain does (tridiag_reg.hip).  Shapes are the fastest of a sweep; 32 steps of
-// 2048 matrices, ms, 32 x 16 lanes against 16 x 16: FP32 160 1.98, 2.21; 128 1.50 (1.19 with
+// 2048 matrices, ms, 32 x 16 lanes against 16 x 16: FP32 160 1.98, 2.21; 137 -> 128 (9
+// steps, the 160 against the 144 grid) 0.80, 0.59, FP64 2.30, 1.35 (512 registers, AGPRs
+// among them, one wave per SIMD); FP32 128 1.50 (1.19 with
 // 6 of 20 blocks in LDS), 1.15; 96 0.74, 0.63; 64 (63 steps) 0.68, 0.49; FP64 128 2.48 (2.74
 // with no blocks in LDS), too large; 96 1.69, 1.33; 64 1.31, 1.05.
 #include <hip/hip_runtime.h>
@@ -19,7 +21,7 @@ namespace uepm {
 
 namespace {
 
-constexpr int kSize[] = {192, 160, 128, 96, 64};
+constexpr int kSize[] = {192, 160, 144, 128, 96, 64};
 constexpr int kNum = sizeof(kSize) / sizeof(kSize[0]);
 constexpr int kMax32 = 192, kMax64 = 160;
 
@@ -28,9 +30,10 @@ int stage_of(int n) {
     while (g < kNum - 1 && n <= kSize[g + 1]) ++g;
     return g;
 }
+// 144 takes first blocks only: 16 steps are not worth a hand-over
 int next(int n) {
     const int g = stage_of(n);
-    return g < kNum - 1 ? kSize[g + 1] : 0;
+    return n > 128 ? (n > 160 ? 160 : 128) : g < kNum - 1 ? kSize[g + 1] : 0;
 }
 
 template <int IN, typename R>
@@ -45,6 +48,9 @@ void stage(const q4<double>* H0, const q4<R>* Hb, int64_t hk, int n, int64_t nk,
             switch (kSize[stage_of(n)]) {
                 case 192: UEPM_GRID(32, 6, 2, 0); break;
                 case 160: UEPM_GRID(32, 5, 2, 0); break;
+                case 144:
+                    if constexpr (IN == 1) UEPM_GRID(16, 9, 2, 12);
+                    break;
                 case 128: UEPM_GRID(16, 8, 2, 0); break;
                 case 96: UEPM_GRID(16, 6, 3, 3); break;
                 default: UEPM_GRID(16, 4, 4, 0); break;
@@ -52,6 +58,9 @@ void stage(const q4<double>* H0, const q4<R>* Hb, int64_t hk, int n, int64_t nk,
         } else {
             switch (kSize[stage_of(n)]) {
                 case 160: UEPM_GRID(32, 5, 2, 5); break;
+                case 144:
+                    if constexpr (IN == 1) UEPM_GRID(16, 9, 1, 14);
+                    break;
                 case 128: UEPM_GRID(32, 4, 2, 4); break;
                 case 96: UEPM_GRID(16, 6, 2, 6); break;
                 default: UEPM_GRID(16, 4, 2, 0); break;

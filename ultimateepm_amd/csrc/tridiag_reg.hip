@@ -166,7 +166,8 @@ int tridiag_reg_max_n() { return 288; }
 // Hand-over between grids.  The late steps of a large grid carry its full
 // per-step overhead for a small trailing matrix, so each grid stops where the
 // next smaller one can take the trailing block: 288 -> 256 -> 224 -> 192 -> 160 ->
-// 128 -> 96 -> 64 (one wave).  From 160 down the lanes are 16 x 16, not 32 x 16: four waves
+// 128 -> 96 -> 64 (one wave); a first block of 129 .. 144 takes a grid of its own (16 steps
+// at 144: 0.34 ms, the 160 grid 0.44).  From 160 down the lanes are 16 x 16, not 32 x 16: four waves
 // meet at a step's barriers instead of eight and twice the workgroups share a CU, so
 // one's barriers and chains hide behind another's work.  Low-register form throughout
 // but for 96, blocks in LDS where that is what one more workgroup takes.  VGPRs and
@@ -175,8 +176,8 @@ int tridiag_reg_max_n() { return 288; }
 // (4).  32 steps of 2048 matrices, 32 x 16 -> 16 x 16 lanes: 160 0.68 -> 0.63 ms, 128 0.51 ->
 // 0.41, 96 0.32 -> 0.26; at 192 (21 steps) 32 x 16 stays the faster, 0.65 against 0.74.
 namespace {
-constexpr int kNumGrids = 8;
-constexpr int kGrid[kNumGrids] = {288, 256, 224, 192, 160, 128, 96, 64};
+constexpr int kNumGrids = 9;
+constexpr int kGrid[kNumGrids] = {288, 256, 224, 192, 160, 144, 128, 96, 64};
 // index of the smallest grid that holds n
 int grid_of(int n) {
     int g = 0;
@@ -187,6 +188,8 @@ int grid_of(int n) {
 
 int tridiag_reg_split(int n) {
     if (n > kGrid[0]) return kGrid[0];
+    if (n > 128 && n <= 160) return 128;  // 144 takes first blocks only
+    if (n > 160 && n <= 192) return 160;
     const int g = grid_of(n);
     return g < kNumGrids - 1 ? kGrid[g + 1] : 0;
 }
@@ -207,7 +210,7 @@ void wave64_stage(const THin* H, int64_t h_kstride, int n, int ld, int64_t nk, f
                        v_kstride, dd, de, dtau, de_kstride);
 }
 
-constexpr int NL288 = 16, NL192 = 14, NL160 = 12, NL128 = 10;  // blocks held in LDS by these grids
+constexpr int NL288 = 16, NL192 = 14, NL160 = 12, NL144 = 14, NL128 = 10;  // blocks held in LDS by these grids
 
 template <typename THin, int IN>
 void grid_stage(int g, const THin* H, int64_t hk, int m, int ld, int64_t nk, float2* V, int ldv, int64_t vk,
@@ -218,8 +221,11 @@ void grid_stage(int g, const THin* H, int64_t hk, int m, int ld, int64_t nk, flo
         case 2: reg_stage<c2<float>, 32, 7, 2, IN, THin, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         case 3: reg_stage<c2<float>, 32, 6, 4, IN, THin, true, NL192>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         case 4: reg_stage<c2<float>, 16, 10, 3, IN, THin, true, NL160>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 5: reg_stage<c2<float>, 16, 8, 4, IN, THin, true, NL128>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 6: reg_stage<c2<float>, 16, 6, 4, IN, THin>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        case 5:
+            if constexpr (IN != 2) reg_stage<c2<float>, 16, 9, 4, IN, THin, true, NL144>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
+            break;
+        case 6: reg_stage<c2<float>, 16, 8, 4, IN, THin, true, NL128>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        case 7: reg_stage<c2<float>, 16, 6, 4, IN, THin>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         default: wave64_stage<IN, THin>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s); break;  // last: s_end >= m - 1
     }
 }
@@ -308,34 +314,38 @@ hipError_t launch_tridiag_reg_c64_block(const float2* H, int64_t hk, int m, int 
 
 // ---- FP64: grids 192 (10 of 42 blocks in LDS) and 160 of 32 x 16 lanes, 256 and 236
 // VGPRs, one workgroup per CU; 128 and 96 of 16 x 16 lanes, two and three (32 steps of
-// 2048 matrices, 32 x 16 -> 16 x 16 lanes: 128 1.15 -> 0.80 ms, 96 0.62 -> 0.49; 160 1.55
+// 2048 matrices, 32 x 16 -> 16 x 16 lanes: 137 -> 128 0.58 -> 0.46, 128 1.15 -> 0.80 ms, 96 0.62 -> 0.49; 160 1.55
 // against 1.65; one matrix alone takes a tenth longer on half the lanes).  The last 64 steps run one row per lane in two
 // column waves, four workgroups per CU (tridiag_row.hpp; 4096 blocks of 64 take
 // 0.59 ms, a 2 x 4 grid 1.48; blocks of 27 in one wave 0.14; at 96 the grid is
 // the faster, 1.0 ms for 32 steps against 1.50).  A larger FP64 matrix runs the
 // blocked reduction first and hands over its trailing block at a panel boundary.
 namespace {
-constexpr int kNumGrids64 = 5;
-constexpr int kGrid64[kNumGrids64] = {192, 160, 128, 96, 64};
+constexpr int kNumGrids64 = 6;
+constexpr int kGrid64[kNumGrids64] = {192, 160, 144, 128, 96, 64};
 int grid64_of(int n) {
     int g = 0;
     while (g < kNumGrids64 - 1 && n <= kGrid64[g + 1]) ++g;
     return g;
 }
 int split64(int n) {
+    if (n > 128) return n > 160 ? 160 : 128;  // 144 takes first blocks only
     const int g = grid64_of(n);
     return g < kNumGrids64 - 1 ? kGrid64[g + 1] : 0;
 }
-constexpr int NL64_192 = 10, NL64_128 = 2, NL64_96 = 4;  // blocks held in LDS by these FP64 grids
+constexpr int NL64_192 = 10, NL64_144 = 12, NL64_128 = 2, NL64_96 = 4;  // blocks held in LDS by these FP64 grids
 template <int IN>
 void grid64_stage(int g, const double2* H, int64_t hk, int m, int ld, int64_t nk, double2* V, int ldv, int64_t vk,
                   double* dd, double* de, double2* dtau, int64_t dk, int s_end, double2* B, int ldb, hipStream_t s) {
     switch (g) {
         case 0: reg_stage<c2<double>, 32, 6, 1, IN, double2, true, NL64_192>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         case 1: reg_stage<c2<double>, 32, 5, 1, IN, double2, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 2: reg_stage<c2<double>, 16, 8, 2, IN, double2, true, NL64_128>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        case 2:
+            if constexpr (IN != 2) reg_stage<c2<double>, 16, 9, 2, IN, double2, true, NL64_144>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
+            break;
+        case 3: reg_stage<c2<double>, 16, 8, 2, IN, double2, true, NL64_128>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         // hands both triangles to the row kernel
-        case 3: reg_stage<c2<double>, 16, 6, 3, IN, double2, true, NL64_96, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        case 4: reg_stage<c2<double>, 16, 6, 3, IN, double2, true, NL64_96, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         default:
             if constexpr (IN != 0) {
                 if (m <= 32) row_stage<c2<double>, 1, 1, 2, 2, IN>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
