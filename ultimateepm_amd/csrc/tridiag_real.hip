@@ -3,12 +3,12 @@
 // and no spin-orbit, in FP32 for the precision form and FP64 for the FP64 form.
 // A chain of shrinking kernels as for complex matrices (tridiag_reg.hip): real
 // lower-triangle grids (tridiag_grid.hpp) down to a trailing block of 128, then
-// one-row-per-lane kernels (tridiag_row.hpp).
+// one-row-per-lane kernels (tridiag_row.hpp); FP32 blocks of 65 .. 96 start in a grid.
 //
 // A real element takes a quarter of a complex one's multiply-adds and half its
 // registers, so each grid reaches twice the dimension or twice the workgroups
-// per CU.  Measured (random matrices, 4096 per launch, alone on the chip): n = 181
-// FP32 2.1 ms against 4.7 ms for the complex64 chain, FP64 3.4 ms against 11.6 ms.
+// per CU.  Si, n = 181, 2048 k-points alone on the chip: FP32 1.08 ms, FP64 1.87; the
+// complex kernels took 2.5 and 5.8 on the same matrices.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -47,8 +47,9 @@ int next(int n) {
 // Measured, ms per 32 steps and 2048 matrices: FP32 448: 3.04, 384: 2.24, 320:
 // 1.73, 288: 1.09, 256: 0.77, 224: 0.62 (16 x 16 lanes: the same), 160: 0.31; FP64 320: 2.53, 288: 1.87, 256: 1.54,
 // 224: 1.35, 160: 0.52 (0.58 without blocks in LDS).  Per 4096: FP32 192 (53 steps):
-// 1.17 (1.43 at three waves per SIMD without), 128 (64 steps): 0.55 (grid:
-// 0.71), 64: 0.15; FP64 2.19, 1.01 (grid: 1.31), 0.19.
+// 1.17 (1.43 at three waves per SIMD without), 128 (64 steps): 0.55 (32 steps of a grid
+// alone: 0.47), 96 (32 steps): 0.28 (rows: 0.34), 64: 0.15; FP64 2.19, 128: 1.01 (32 steps
+// of a grid alone: 0.70), 96: 0.44 (grid: 0.49), 64: 0.19.
 template <typename THin>
 void stage(const THin* H, int64_t hk, int n, int ld, int64_t nk, float* V, int ldv, int64_t vk, double* dd, double* de,
            float* dtau, int64_t dk, int s_end, float* B, int ldb, hipStream_t s) {
@@ -71,7 +72,7 @@ void stage(const THin* H, int64_t hk, int n, int ld, int64_t nk, float* V, int l
             break;
         case 128: UEPM_ROWS(2, 2, 4, 5); break;
         case 96:
-            if constexpr (kFromH) UEPM_ROWS(2, 1, 6, 3);
+            if constexpr (kFromH) UEPM_GRID(16, 6, 8, 1, THin, true, 0, true);
             break;
         default: UEPM_ROWS(1, 1, 4, 5); break;
     }
