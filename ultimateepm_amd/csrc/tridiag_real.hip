@@ -8,7 +8,7 @@
 // A real element takes a quarter of a complex one's multiply-adds and half its
 // registers, so each grid reaches twice the dimension or twice the workgroups
 // per CU.  Si, n = 181, 2048 k-points alone on the chip: FP32 1.08 ms, FP64 1.87; the
-// complex kernels took 2.5 and 5.8 on the same matrices.
+// complex kernels took 2.4 and 5.8 on the same matrices.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
