@@ -53,8 +53,8 @@ __global__ __launch_bounds__(BS, 4) void assemble_kernel(DevParams P, const int3
     const double* k = kpts + 3 * (size_t)kk;
     const int N = P.N;
     const VecLayout L = vec_layout(P);
-    int32_t* Gp = reinterpret_cast<int32_t*>(S + L.count * N);
-    for (int i = threadIdx.x; i < N; i += BS) vector_init(P, L, k, G, i, S, Gp);
+    int32_t* Gs = reinterpret_cast<int32_t*>(S + L.count * N);
+    for (int i = threadIdx.x; i < N; i += BS) vector_init(P, L, k, G, i, S, Gs);
     for (int t = threadIdx.x; t < kVPhaseTab; t += BS) vtab[t] = local_phase(P, t / 49 - 3, (t / 7) % 7 - 3, t % 7 - 3);
     __syncthreads();
     T* A = H + (size_t)kk * ld * (F == HForm::kQuaternion ? N : P.dim);
@@ -82,9 +82,7 @@ __global__ __launch_bounds__(BS, 4) void assemble_kernel(DevParams P, const int3
             const bool in = i < N && j < N && i >= j;
             double re = 0.0, im = 0.0, so[6];
             if (in) {
-                const int gi = Gp[i], gj = Gp[j];
-                const int gx = (gi & 1023) - (gj & 1023), gy = (gi >> 10 & 1023) - (gj >> 10 & 1023);
-                const int gz = (gi >> 20) - (gj >> 20);
+                const int gx = Gs[i] - Gs[j], gy = Gs[N + i] - Gs[N + j], gz = Gs[2 * N + i] - Gs[2 * N + j];
                 local_V(P, gx, gy, gz, re, im, vtab);
                 if (i == j) {
                     const double kx = S[i], ky = S[N + i], kz = S[2 * N + i];
@@ -151,8 +149,9 @@ namespace {
 template <HForm F>
 hipError_t launch_assemble_form(const DevParams& P, const int32_t* dG, const double* dk, int64_t nk,
                                 typename HElem<F>::T* dH, int ld, hipStream_t s) {
-    // the per-vector arrays (at most 164 bytes a vector) beside the phase table and
-    // the transpose slots: 576 vectors take 118 of the 160 KB of a CU
+    // the per-vector arrays (at most 164 bytes a vector, 196 with spin-orbit) beside the
+    // phase table and the transpose slots: 576 vectors take 117 of the 160 KB of a CU, 288
+    // spinor ones 66
     const size_t shm = vec_bytes(P);
     const size_t fixed = sizeof(double2) * kVPhaseTab + (kAsmBS / 64) * (F == HForm::kSpinor || F == HForm::kQuaternion ? 4 : 16) * 17 * sizeof(typename HElem<F>::T);
     if (shm + fixed > 163840) return hipErrorInvalidValue;

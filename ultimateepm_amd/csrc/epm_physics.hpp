@@ -155,7 +155,7 @@ struct VecLayout {
     int32_t l0a = 0, l0c = 0, l2a = 0, l2c = 0;  // radial integrals (cation: the anion's when the radii are equal)
     int32_t B = 0;                    // spin-orbit radial factors of anion and cation
     int32_t q = 0;                    // cos, sin of the spin-orbit phase of G
-    int32_t count = 0;                // arrays in all (and one int32 per vector after them: G, packed)
+    int32_t count = 0;                // arrays in all (and three of int32 after them: the components of G)
 };
 __host__ __device__ inline VecLayout vec_layout(const DevParams& P) {
     VecLayout L;
@@ -179,11 +179,8 @@ __host__ __device__ inline VecLayout vec_layout(const DevParams& P) {
     return L;
 }
 __host__ __device__ inline size_t vec_bytes(const DevParams& P) {
-    return (sizeof(double) * (size_t)vec_layout(P).count + sizeof(int32_t)) * (size_t)P.N;
+    return (sizeof(double) * (size_t)vec_layout(P).count + 3 * sizeof(int32_t)) * (size_t)P.N;
 }
-
-// G of a basis vector in one word: three components biased by 512
-__device__ __forceinline__ int32_t pack_g(int x, int y, int z) { return (x + 512) | (y + 512) << 10 | (z + 512) << 20; }
 
 __device__ __forceinline__ void radial_init(int l, double nK, double R, double* S, int N, int i) {
     const double x = nK * R;
@@ -194,11 +191,13 @@ __device__ __forceinline__ void radial_init(int l, double nK, double R, double* 
 }
 
 __device__ __forceinline__ void vector_init(const DevParams& P, const VecLayout& L, const double* k, const int32_t* G,
-                                            int i, double* S, int32_t* Gp) {
+                                            int i, double* S, int32_t* Gs) {
     const int N = P.N;
     const int gx = G[3 * i], gy = G[3 * i + 1], gz = G[3 * i + 2];
     const double kx = k[0] + (double)gx, ky = k[1] + (double)gy, kz = k[2] + (double)gz;
-    Gp[i] = pack_g(gx, gy, gz);
+    Gs[i] = gx;
+    Gs[N + i] = gy;
+    Gs[2 * N + i] = gz;
     S[L.k * N + i] = kx;
     S[(L.k + 1) * N + i] = ky;
     S[(L.k + 2) * N + i] = kz;
@@ -226,7 +225,9 @@ __device__ __forceinline__ void vector_init(const DevParams& P, const VecLayout&
         S[L.B * N + i] = soc_radial(P.period_a, nK, P.bohr, P.xi_a);
         S[(L.B + 1) * N + i] = soc_radial(P.period_c, nK, P.bohr, P.xi_c);
         double s, c;
-        sincos(P.soc_kfac * (P.tau * (double)gx + P.tau * (double)gy + P.tau * (double)gz), &s, &c);
+        // soc_kfac tau is pi / 4: the phase has eight values, formed from the smallest
+        // argument (that of G itself grows with a basis far from the origin)
+        sincos(P.soc_kfac * (P.tau * (double)(((unsigned)gx + (unsigned)gy + (unsigned)gz) & 7u)), &s, &c);
         S[L.q * N + i] = c;
         S[(L.q + 1) * N + i] = s;
     }
