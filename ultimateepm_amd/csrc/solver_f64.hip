@@ -41,8 +41,9 @@ __device__ __forceinline__ double rcp_nr64(double x) {
 
 // number of eigenvalues of T below x: sign changes of the leading principal
 // minors p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2}, T scaled to norm 1..2 and e^2
-// held above 2^-120 (so that no two neighbours vanish and eight steps stay in
-// range; the pair is rescaled by a power of two every eight).  One multiply-add
+// held above 2^-160, so that no two neighbours vanish.  Of two neighbours the larger
+// falls by at most that (and a factor of eight) six times in eight steps, after which
+// the pair is rescaled by a power of two, so it stays in range.  One multiply-add
 // long per step, against a reciprocal and its Newton step for the quotients
 // p_i / p_{i-1}; the two have the same backward error.  n and the LDS arrays are
 // padded to whole pairs of blocks of eight (kSturmPad, rows that change no sign).
@@ -88,9 +89,8 @@ constexpr double kSturmPad = 16.0;
 
 // Eigenvalues of T by multisection, one wave per k-point and 64 / S bands (S probes
 // per band): a sweep narrows the bracket of every band S + 1-fold.  d and e^2,
-// scaled, sit in LDS, uniform reads across the wave.  abstol_rel: a bracket
-// narrower than abstol_rel ||T||_inf is final (0: the rounding level of the
-// eigenvalue, or a sixteenth of ||T||'s where that is more).  At N = 181,
+// scaled, sit in LDS, uniform reads across the wave.  A bracket is final at the
+// rounding level of its eigenvalue, or narrower than abstol_rel ||T||_inf.  At N = 181,
 // 16 bands, 4096 k-points (two chunks in flight) it takes 0.26 ms against 0.45 ms
 // with the ratio form of the count (a division a row) and unpadded rows; bound by
 // FP64 issue, and at one k-point by the chain of fmas (69 us for 11 sweeps).
@@ -150,14 +150,14 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
     for (int i = lane; i < np; i += 64) {
         const double ei = i > 0 && i < n ? scaled(e[i - 1]) : 0.0;
         sd[i] = i < n ? scaled(d[i]) : kSturmPad;
-        se2[i] = i < n ? fmax(ei * ei, 0x1p-120) : 0.0;
+        se2[i] = i < n ? fmax(ei * ei, 0x1p-160) : 0.0;
     }
     __syncthreads();
     const double eps = DBL_EPSILON;
     tnorm = scaled(tnorm);
     lo = scaled(lo) - 2.0 * eps * tnorm - 0x1p-58;  // and what the floor of e^2 may move
     hi = scaled(hi) + 2.0 * eps * tnorm + 0x1p-58;
-    const double abstol = fmax(abstol_rel, eps / 16.0) * tnorm;
+    const double abstol = abstol_rel * tnorm;
     // two shared sweeps first: the wave's 64 lanes probe one interval that holds
     // every band of the wave, and each band takes the probes around its index
     // (a count c at x puts eigenvalues 0..c-1 below x and c.. at or above it)
