@@ -142,9 +142,9 @@ struct Mfma<float> {
 };
 
 template <typename T, int BS, int NBP>
-__global__ __launch_bounds__(BS, 1) void tridiag_blocked_kernel(const double2* __restrict__ Hin, int n, int ld,
+__global__ __launch_bounds__(BS, 1) void tridiag_blocked_kernel(const double2* Hin, int n, int ld,
                                                                  int c0, cx<T>* __restrict__ scratch,
-                                                                 int64_t scratch_stride, cx<T>* __restrict__ Vout,
+                                                                 int64_t scratch_stride, cx<T>* Vout,
                                                                  double* __restrict__ dout, double* __restrict__ eout,
                                                                  cx<T>* __restrict__ tauout, int s_end) {
     constexpr int MOD = 128 / (int)sizeof(cx<T>);

@@ -122,12 +122,14 @@ struct RegLayout {
 // i + j ld); 1, as the conjugate of the upper triangle of a full Hermitian
 // matrix (element (j, i) at j + i ld); 2, row by row as a hand-over block.  Input (leading
 // dimension ld), reflectors (ldv) and d, e, tau of k-point kk start at
-// kk * h_kstride, kk * v_kstride and kk * de_kstride.
+// kk * h_kstride, kk * v_kstride and kk * de_kstride.  The reflectors may go over the
+// input (the FP64 form), so neither pointer is __restrict__: the input is read before
+// the first step, which writes the first of them.
 template <int PR, int PC, int LR, int LC, int MINWG, typename S, typename THin, bool LOW = false, int NL = 0, int IN = 0,
           bool FULL = false>
-__global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* __restrict__ Hin, int64_t h_kstride,
+__global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* Hin, int64_t h_kstride,
                                                                     int n, int ld,
-                                                                    typename ScMem<S>::T* __restrict__ Vout, int ldv,
+                                                                    typename ScMem<S>::T* Vout, int ldv,
                                                                     int64_t v_kstride, double* __restrict__ dout,
                                                                     double* __restrict__ eout,
                                                                     typename ScMem<S>::T* __restrict__ tauout,

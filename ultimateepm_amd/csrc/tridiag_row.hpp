@@ -63,7 +63,7 @@ struct RowGroup {
 // j + i ld.  The hand-over block written (s_end < n - 1) holds both triangles too.
 template <typename S, int RW, int CW, int NG, int MINW, int IN, typename THin>
 __global__ __launch_bounds__(64 * RW * CW, MINW) void tridiag_row_kernel(
-    const THin* __restrict__ Hin, int64_t h_kstride, int n, int ld, typename ScMem<S>::T* __restrict__ Vout, int ldv,
+    const THin* Hin, int64_t h_kstride, int n, int ld, typename ScMem<S>::T* Vout, int ldv,
     int64_t v_kstride, double* __restrict__ dout, double* __restrict__ eout, typename ScMem<S>::T* __restrict__ tauout,
     int64_t de_kstride, int s_end, typename ScMem<S>::T* __restrict__ Bout, int ldb) {
     using R = typename S::R;

@@ -56,8 +56,8 @@ struct StripOrder {
 // 15 the update, 5 the trailing product) and the strip's latency (4.5, six units of
 // 8 KB in flight; 4 and 8 units measure the same).
 template <int LR, int MG, int NL, int IN, typename THin>
-__global__ __launch_bounds__(512, 2) void tridiag_strip_kernel(const THin* __restrict__ Hin, int64_t h_kstride, int n, int ld,
-                                                               float2* __restrict__ Vout, int ldv, int64_t v_kstride,
+__global__ __launch_bounds__(512, 2) void tridiag_strip_kernel(const THin* Hin, int64_t h_kstride, int n, int ld,
+                                                               float2* Vout, int ldv, int64_t v_kstride,
                                                                double* __restrict__ dout, double* __restrict__ eout,
                                                                float2* __restrict__ tauout, int64_t de_kstride,
                                                                float2* __restrict__ Bout, int64_t b_kstride,
