@@ -6,6 +6,9 @@
 // v_fmac_f64 and v_fmac_f64_dpp 4.8: the DPP operand is free in FP64.
 // Plain VALU instructions; each block opens with the two wait states a DPP
 // operand needs after a VALU write.
+// The accumulators are early clobbers: several instructions write them while later
+// ones still read the factors, so none may share a register with a factor of the
+// same value (it may where the compiler sees the two equal, as in a first pass over zeros).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -21,7 +24,7 @@ namespace rowop {
                 UEPM_MV(T, "2", "15", "10") UEPM_MV(T, "3", "16", "11") UEPM_MV(T, "0", "17", "12")              \
                     UEPM_MV(T, "1", "18", "13") UEPM_MV(T, "2", "19", "14") UEPM_MV(T, "3", "20", "15")
 #define UEPM_MV_OPS                                                                                              \
-    : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])                                                     \
+    : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3])                                                 \
     : "v"(v), "v"(A[0]), "v"(A[1]), "v"(A[2]), "v"(A[3]), "v"(A[4]), "v"(A[5]), "v"(A[6]), "v"(A[7]), "v"(A[8]), \
       "v"(A[9]), "v"(A[10]), "v"(A[11]), "v"(A[12]), "v"(A[13]), "v"(A[14]), "v"(A[15])
 
@@ -38,8 +41,8 @@ __device__ __forceinline__ void dot16(double (&acc)[4], double v, const double (
     "s_nop 1\n\t" UEPM_AX(T, "0", r0) UEPM_AX(T, "1", r1) UEPM_AX(T, "2", r2) UEPM_AX(T, "3", r3)              \
         UEPM_AX(T, "4", r4) UEPM_AX(T, "5", r5) UEPM_AX(T, "6", r6) UEPM_AX(T, "7", r7)
 #define UEPM_AX_OPS(o)                                                                                           \
-    : "+v"(A[o]), "+v"(A[o + 1]), "+v"(A[o + 2]), "+v"(A[o + 3]), "+v"(A[o + 4]), "+v"(A[o + 5]), "+v"(A[o + 6]), \
-      "+v"(A[o + 7])                                                                                             \
+    : "+&v"(A[o]), "+&v"(A[o + 1]), "+&v"(A[o + 2]), "+&v"(A[o + 3]), "+&v"(A[o + 4]), "+&v"(A[o + 5]),         \
+      "+&v"(A[o + 6]), "+&v"(A[o + 7])                                                                           \
     : "v"(x), "v"(c)
 
 // A[r] += c * (x of lane r of the row), r = 0..15
