@@ -202,17 +202,23 @@ int uepm_plan_last_timing(const uepm_plan* plan, int stage, double* ms, int64_t*
 /* ---- configuration, tuning and workspace -----------------------------------
  * No counterpart in the reference (its solve has no tunables). */
 typedef struct uepm_config {
-    int32_t tridiag;   /* 0 automatic (UEPM_MIXED plans above dim 384: LDS-blocked
-                          leading steps, then the register grids); 1 LDS-blocked
-                          reduction only; 2 register-resident complex64 reduction
+    int32_t tridiag;   /* 0 automatic: real kernels for a crystal of equal atoms without
+                          spin-orbit (dim <= 448, FP64 320), quaternion kernels with it
+                          (basis <= 192, FP64 160), else complex ones (UEPM_MIXED plans
+                          above dim 384 and FP64 plans above 192: LDS-blocked leading
+                          steps, then the register grids); 1 the complex kernels for any
+                          crystal, and in UEPM_MIXED plans the LDS-blocked reduction
+                          alone; 2 automatic, register-resident for certain
                           (UEPM_MIXED plans, dim <= 288)                              */
-    int32_t tri_block; /* LDS-blocked reduction workgroup size: 256 or 512 (0 = 512)  */
+    int32_t tri_block; /* LDS-blocked reduction workgroup size: 256 or 512 (0 = 512);
+                          no effect where that reduction does not run                 */
     int32_t bt_bands;  /* back-transform: 0 automatic (above dim 192, and UEPM_MIXED
                           plans with nb + 4 > 16: the blocked MFMA kernel while X
                           fits the LDS -- complex64 while nb + 4 <= 32, FP64 in
                           passes of 16 bands up to dim 524 at 160 KB; otherwise
                           16); 4, 8 or 16 bands per workgroup of the
-                          reflector-by-reflector kernel                               */
+                          reflector-by-reflector kernel; no effect on plans that run
+                          real or quaternion kernels                                  */
     int32_t max_chunk; /* k-points per launch (0 = automatic: <= 4096, <= 4 GiB of H) */
     int32_t lanes;     /* chunks in flight: 0 automatic (2 when a solve spans two or
                           more chunks: alternate chunks on the caller's stream and on
@@ -224,7 +230,9 @@ int uepm_plan_get_config(const uepm_plan* plan, uepm_config* cfg);
 int uepm_plan_set_config(uepm_plan* plan, const uepm_config* cfg);
 /* Autotuner: times every candidate configuration on the device k-points
  * d_k[0..nk) (one warm-up and two timed solves each, on `stream`), keeps the
- * fastest in the plan and returns it in *chosen (may be NULL). */
+ * fastest in the plan and returns it in *chosen (may be NULL).  A plan that takes
+ * real or quaternion kernels has one candidate, the automatic one; a knob without
+ * effect on the plan stays at its default.  max_chunk and lanes are kept. */
 int uepm_plan_tune(uepm_plan* plan, const double* d_k, int64_t nk, void* stream, uepm_config* chosen);
 /* Device workspace that solves of up to nk k-points need, and its allocation
  * ahead of time: after uepm_plan_reserve(plan, nk) such solves allocate nothing

@@ -914,31 +914,47 @@ int uepm_plan_tune(uepm_plan* p, const double* dk, int64_t nk, void* stream_, ue
     if (p->pins > 0) return fail(UEPM_ERR_INVALID_ARG, "uepm_plan_tune: the plan is used by a batch graph");
     HIP_OK(hipSetDevice(p->ctx->device));
     hipStream_t s = (hipStream_t)stream_;
-    // candidates: reduction variant x workgroup size, back-transform band groups
+    // candidates: reduction variant x workgroup size, back-transform band groups; one
+    // value for a knob that the plan's kernels do not have, or its choice would be noise
     std::vector<uepm_config> cand;
+    const uepm_config saved = p->cfg;
+    auto add = [&](int tridiag, int tri_block, int bt) {
+        cand.push_back({tridiag, tri_block, bt, saved.max_chunk, saved.lanes});
+    };
     const bool mixed = p->flags & UEPM_MIXED;
+    const bool want_vec = p->flags & UEPM_VECTORS;
     const bool reg_ok = mixed && p->dim <= uepm::tridiag_reg_max_n();
-    // back-transform: the blocked MFMA kernel (0: automatic, which is the blocked
-    // kernel in the precision form and above dim 192 in FP64) or 8 / 16 bands per
-    // workgroup of the reflector-by-reflector one
-    std::vector<int> bts = {8, 16};
-    if (mixed || (p->dim > 192 && uepm::apply_q_wy_f64_fits(p->dim, p->ctx->lds_limit))) bts.insert(bts.begin(), 0);
-    for (int bt : bts) {
-        if (reg_ok) cand.push_back({2, 0, bt, p->cfg.max_chunk, p->cfg.lanes});
-        for (int tb : {256, 512}) {
-            cand.push_back({1, tb, bt, p->cfg.max_chunk, p->cfg.lanes});
-            // above the register grids: blocked leading steps, register-grid tail
-            if (mixed && !reg_ok) cand.push_back({0, tb, bt, p->cfg.max_chunk, p->cfg.lanes});
+    p->cfg.tridiag = 0;
+    plan_apply_config(p);
+    if (p->real || p->quat) {
+        // one route, whose back-transform has no band groups (the complex kernels, which
+        // tridiag = 1 would ask for, take two to five times its time)
+        add(reg_ok ? 2 : 0, reg_ok ? 0 : 512, 0);
+    } else {
+        // back-transform: the blocked MFMA kernel (0: automatic, which is the blocked
+        // kernel in the precision form and above dim 192 in FP64) or 8 / 16 bands per
+        // workgroup of the reflector-by-reflector one; FP64 eigenvalues alone run none
+        std::vector<int> bts = {8, 16};
+        if (!mixed && !want_vec) bts = {0};
+        else if (mixed || (p->dim > 192 && uepm::apply_q_wy_f64_fits(p->dim, p->ctx->lds_limit))) bts.insert(bts.begin(), 0);
+        // the automatic reduction has a blocked part above dim 192 in FP64; in the precision
+        // form above 384
+        const bool blocked = mixed ? uepm::tridiag_reg_c64_tail(p->dim) < p->dim : uepm::tridiag_reg_c128_tail(p->dim) < p->dim;
+        for (int bt : bts) {
+            if (reg_ok) add(2, 0, bt);
+            else if (!blocked) add(0, 512, bt);
+            for (int tb : {256, 512}) {
+                if (mixed) add(1, tb, bt);  // blocked alone (FP64 has no such variant)
+                if (!reg_ok && blocked) add(0, tb, bt);
+            }
         }
     }
-    const uepm_config saved = p->cfg;
     const int saved_timing = p->timing;
     p->timing = 0;
     DeviceBuffer ev, vec, gr;
     int rc = UEPM_OK;
     if (ev.ensure(sizeof(double) * (size_t)nk * p->nb) != hipSuccess)
         rc = fail(UEPM_ERR_NO_MEMORY, "uepm_plan_tune: out of device memory");
-    const bool want_vec = p->flags & UEPM_VECTORS;
     if (rc == UEPM_OK && want_vec &&
         vec.ensure(sizeof(double2) * (size_t)nk * p->nb * p->dim) != hipSuccess)
         rc = fail(UEPM_ERR_NO_MEMORY, "uepm_plan_tune: out of device memory");
