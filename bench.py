@@ -300,7 +300,8 @@ def batching_leg(ctx, nk_per_item: int, branches: int = 8, ws_cap_gib: float = 2
     (InP + SOC excluded: its anion period has no spin-orbit radial model), nk
     seeded first-BZ k-points each, all captured into one hipGraph (concurrent
     branches) and launched once; reduction variant and band grouping chosen per
-    dimension by the autotuner.  Run in the precision form and in FP64."""
+    dimension and kind of crystal (equal atoms run other kernels than III-V
+    compounds) by the autotuner.  Run in the precision form and in FP64."""
     from ultimateepm_amd import api
     from ultimateepm_amd.material import load
 
@@ -310,7 +311,7 @@ def batching_leg(ctx, nk_per_item: int, branches: int = 8, ws_cap_gib: float = 2
     out = {"items": len(combos), "nk_per_item": nk_per_item, "branches": branches}
     evals = {}
     for mode in ("mixed", "fp64"):
-        tuned = {}  # dimension bucket -> configuration chosen by the autotuner
+        tuned = {}  # (dimension, kind of crystal) -> configuration chosen by the autotuner
         plans, bufs, items = [], [], []
         t_tune = time.perf_counter()
         for i, (m, n, soc) in enumerate(combos):
@@ -319,7 +320,7 @@ def batching_leg(ctx, nk_per_item: int, branches: int = 8, ws_cap_gib: float = 2
             p = api.Plan(ctx, load(m), api.basis_vectors(n), flags, nb)
             per_k = max(1, p.workspace_bytes(1))
             cap = int(max(1, min(4096, ws_cap_gib * (1 << 30) // per_k)))
-            key = (p.dim, mode)
+            key = (p.dim, "" if m in ("Si", "Ge") else "_iii_v")
             if key not in tuned:
                 sample = api.bz_sample(seed + 7, min(1024, nk_per_item))
                 dsample = api.DeviceArray.from_host(ctx, sample)
@@ -364,7 +365,7 @@ def batching_leg(ctx, nk_per_item: int, branches: int = 8, ws_cap_gib: float = 2
                      "plans_alone_s": round(alone, 4), "graph_over_alone": round(dt / alone, 3),
                      "alone_s_by_dim": {f"dim{d}": round(t, 4) for d, t in sorted(by_dim.items())},
                      "tune_and_setup_s": round(t_tune, 2),
-                     "tuned": {f"dim{d}": c for (d, _), c in sorted(tuned.items())}}
+                     "tuned": {f"dim{d}{kind}": c for (d, kind), c in sorted(tuned.items())}}
         for p in plans:
             p.close()
         for dk, de in bufs:
