@@ -114,8 +114,8 @@ hipError_t launch_tridiag_reg_c128(const double2* H, int64_t hk, int m, int ld, 
 
 // The reduction of a real symmetric H (n x n doubles per k-point, both triangles)
 // in FP32 or FP64, n <= tridiag_real_max_n(f32): outputs as launch_tridiag_reg_c64,
-// reflectors and tau real (V column-major, leading dimension n); `work` provides
-// tridiag_real_work_bytes(n, f32) per k-point.
+// reflectors and tau real (V column-major, leading dimension n; FP64: V may be dH);
+// `work` provides tridiag_real_work_bytes(n, f32) per k-point.
 int tridiag_real_max_n(bool f32);
 size_t tridiag_real_work_bytes(int n, bool f32);
 hipError_t launch_tridiag_real_f32(const double* dH, int n, int64_t nk, float* V, double* dd, double* de, float* dtau,
@@ -123,8 +123,8 @@ hipError_t launch_tridiag_real_f32(const double* dH, int n, int64_t nk, float* V
 hipError_t launch_tridiag_real_f64(const double* dH, int n, int64_t nk, double* V, double* dd, double* de, double* dtau,
                                    double* work, hipStream_t s);
 
-// The same for a quaternion H (n x n per k-point, n <= tridiag_quaternion_max_n): T
-// is n x n and holds each Kramers pair's level once.
+// The same for a quaternion H (n x n per k-point, n <= tridiag_quaternion_max_n; FP64: V
+// may be dH): T is n x n and holds each Kramers pair's level once.
 int tridiag_quaternion_max_n(bool f32);
 size_t tridiag_quaternion_work_bytes(int n, bool f32);
 hipError_t launch_tridiag_quaternion_f32(const q4<double>* dH, int n, int64_t nk, q4<float>* V, double* dd, double* de,

@@ -72,10 +72,10 @@ Sizes plan_sizes(const uepm_plan* p, int64_t chunk) {
     Sizes z{};
     z.d = z.e = sizeof(double) * (size_t)n * chunk;
     if (p->real) {
-        // real elements; the reflectors have their own buffer in both forms
+        // real elements; FP64 reflectors go over H
         const size_t r = mixed ? sizeof(float) : sizeof(double);
         z.H = sizeof(double) * (size_t)n * n * chunk;
-        z.Vf = r * (size_t)n * n * chunk;
+        if (mixed) z.Vf = r * (size_t)n * n * chunk;
         z.tauf = r * (size_t)n * chunk;
         z.S32 = uepm::tridiag_real_work_bytes(n, mixed) * chunk;
         if (mixed) {
@@ -95,7 +95,7 @@ Sizes plan_sizes(const uepm_plan* p, int64_t chunk) {
         const size_t r = 4 * (mixed ? sizeof(float) : sizeof(double));
         z.d = z.e = sizeof(double) * (size_t)N * chunk;
         z.H = 4 * sizeof(double) * (size_t)N * N * chunk;
-        z.Vf = r * (size_t)N * N * chunk;
+        if (mixed) z.Vf = r * (size_t)N * N * chunk;
         z.tauf = r * (size_t)N * chunk;
         z.S32 = uepm::tridiag_quaternion_work_bytes(N, mixed) * chunk;
         z.Ev = sizeof(double) * (size_t)m * chunk;
@@ -340,8 +340,7 @@ int solve_chunks(uepm_plan* p, const double* dk, int64_t nk, double* devals, dou
                                                          reinterpret_cast<float*>(w.tauf),
                                                          reinterpret_cast<float*>(w.S32), cs));
                 else
-                    HIP_OK(uepm::launch_tridiag_real_f64(Hr, n, c, reinterpret_cast<double*>(w.Vf), w.d, w.e,
-                                                         reinterpret_cast<double*>(w.tauf),
+                    HIP_OK(uepm::launch_tridiag_real_f64(Hr, n, c, Hr, w.d, w.e, reinterpret_cast<double*>(w.tauf),
                                                          reinterpret_cast<double*>(w.S32), cs));
                 HIP_OK(rec(ci, kTridiag, 1));
                 HIP_OK(rec(ci, kTriEig, 0));
@@ -362,9 +361,8 @@ int solve_chunks(uepm_plan* p, const double* dk, int64_t nk, double* devals, dou
                                                          reinterpret_cast<float*>(w.tauf), w.Z, nbr,
                                                          reinterpret_cast<double*>(w.X0), c, cs));
                 else
-                    HIP_OK(uepm::launch_apply_q_real_f64(reinterpret_cast<double*>(w.Vf), n,
-                                                         reinterpret_cast<double*>(w.tauf), w.Z, nb, Xc, gc, p->P, kc,
-                                                         p->G.as<int32_t>(), c, ks, status, c0, cs));
+                    HIP_OK(uepm::launch_apply_q_real_f64(Hr, n, reinterpret_cast<double*>(w.tauf), w.Z, nb, Xc, gc, p->P,
+                                                         kc, p->G.as<int32_t>(), c, ks, status, c0, cs));
                 HIP_OK(rec(ci, kBack, 1));
                 if (!mixed) continue;
                 HIP_OK(rec(ci, kRefine, 0));
@@ -378,7 +376,6 @@ int solve_chunks(uepm_plan* p, const double* dk, int64_t nk, double* devals, dou
                 const int N = p->N, m = (nbr + 1) / 2;
                 auto* Hq = reinterpret_cast<uepm::q4<double>*>(w.H);
                 auto* Vq32 = reinterpret_cast<uepm::q4<float>*>(w.Vf);
-                auto* Vq64 = reinterpret_cast<uepm::q4<double>*>(w.Vf);
                 auto* tq32 = reinterpret_cast<uepm::q4<float>*>(w.tauf);
                 auto* tq64 = reinterpret_cast<uepm::q4<double>*>(w.tauf);
                 auto* Xq = reinterpret_cast<uepm::q4<double>*>(w.X0);
@@ -390,7 +387,7 @@ int solve_chunks(uepm_plan* p, const double* dk, int64_t nk, double* devals, dou
                     HIP_OK(uepm::launch_tridiag_quaternion_f32(Hq, N, c, Vq32, w.d, w.e, tq32,
                                                                reinterpret_cast<uepm::q4<float>*>(w.S32), cs));
                 else
-                    HIP_OK(uepm::launch_tridiag_quaternion_f64(Hq, N, c, Vq64, w.d, w.e, tq64,
+                    HIP_OK(uepm::launch_tridiag_quaternion_f64(Hq, N, c, Hq, w.d, w.e, tq64,
                                                                reinterpret_cast<uepm::q4<double>*>(w.S32), cs));
                 HIP_OK(rec(ci, kTridiag, 1));
                 HIP_OK(rec(ci, kTriEig, 0));
@@ -408,7 +405,7 @@ int solve_chunks(uepm_plan* p, const double* dk, int64_t nk, double* devals, dou
                 if (mixed)
                     HIP_OK(uepm::launch_apply_q_quaternion_f32(Vq32, N, tq32, w.Z, m, Xq, c, cs));
                 else
-                    HIP_OK(uepm::launch_apply_q_quaternion_f64(Vq64, N, tq64, w.Z, nb, Xc, gc, p->P, kc,
+                    HIP_OK(uepm::launch_apply_q_quaternion_f64(Hq, N, tq64, w.Z, nb, Xc, gc, p->P, kc,
                                                                p->G.as<int32_t>(), c, ks, status, c0, cs));
                 HIP_OK(rec(ci, kBack, 1));
                 if (!mixed) continue;

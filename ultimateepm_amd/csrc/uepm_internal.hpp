@@ -70,7 +70,7 @@ constexpr int kMixedInvSweeps = 2;
 // stream, each with its own workspace.
 struct Lane {
     DeviceBuffer H, d, e, tau, Z, W, X, S;
-    DeviceBuffer Vf, tauf, S32, Ev, X0;  // precision form
+    DeviceBuffer Vf, tauf, S32, Ev, X0;  // precision form, real and quaternion plans
     DeviceBuffer kstat;                  // per k-point failure flag of the chunk in flight
 };
 
