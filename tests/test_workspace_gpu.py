@@ -27,3 +27,20 @@ def test_symmetric_plans_take_no_more_than_complex_ones(gpu_ctx, sym, soc, top, 
             p.set_config(tridiag=1)
             assert auto <= p.workspace_bytes(1), (N, nb)
             p.close()
+
+
+@pytest.mark.parametrize("dim", [289, 320, 384, 385, 400, 450, 512, 576])
+@pytest.mark.parametrize("nb", [1, 12, 24])
+def test_hand_over_of_large_complex64_reductions(gpu_ctx, dim, nb):
+    """Above dim 288 the reduction's own workspace is the larger of two hand-over blocks
+    (256 and 224 rows) and the blocked kernel's columns, beside H, the reflectors and
+    what the later stages hold."""
+    print(f"case: workspace of a mixed GaAs plan, dim {dim}, {nb} bands", flush=True)
+    p = api.Plan(gpu_ctx, load("GaAs"), np.ascontiguousarray(api.basis_vectors(26)[:dim]), api.MIXED, nb)
+    auto = p.workspace_bytes(1)
+    p.set_config(tridiag=1)
+    blocked = p.workspace_bytes(1)
+    p.close()
+    nbr = nb + 4
+    held = 24 * dim * dim + 40 * dim + (8 + 56 * dim) * nbr + 4
+    assert auto - held <= max(8 * (256 * 256 + 224 * 224), blocked - held)

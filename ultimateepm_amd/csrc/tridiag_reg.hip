@@ -6,6 +6,7 @@
 // The grids' layout and steps are described in tridiag_grid.hpp.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <utility>
 #include <cstdlib>
@@ -195,8 +196,9 @@ int tridiag_reg_split(int n) {
 }
 
 size_t tridiag_reg_work_bytes(int n) {
-    // two ping-pong hand-over blocks: the first hand-over's size and the next one's
-    const int t1 = tridiag_reg_split(n);
+    // two ping-pong hand-over blocks: the first hand-over's size and the next one's (the
+    // strip kernel hands over in place, and its strip lies in the first of the next two)
+    const int t1 = tridiag_reg_split(std::min(n, kGrid[0]));
     if (!t1) return 0;
     const int t2 = tridiag_reg_split(t1);
     return sizeof(float2) * ((size_t)t1 * t1 + (size_t)t2 * t2);
@@ -253,7 +255,7 @@ hipError_t c64_blocks(int r, float2* cur, float2* next, int64_t nk, float2* V, i
 // as fast as the blocked reduction at 362; every column of a longer strip adds as much to
 // the first step's traffic, and at 96 columns that is what the blocked one streams).
 constexpr int kStripMax = 384, kStripCols = (kStripMax - kGrid[0]) / 16, NLStrip = 30;
-static_assert(strip_slots(kStripMax / 32, kStripCols) <= 256 * 256, "the strip fits the second hand-over block");
+static_assert(strip_slots(kStripMax / 32, kStripCols) <= kGrid[1] * kGrid[1], "the strip fits a hand-over block");
 
 // The complex64 chain on a block of size m whose element (0, 0) sits at H
 // (leading dimension ld, per-k stride hk; read as IN says, IN = 0 or 1);
@@ -264,18 +266,22 @@ hipError_t c64_chain(const THin* H, int64_t hk, int m, int ld, int64_t nk, float
                      double* de, float2* dtau, int64_t dk, float2* work, hipStream_t s) {
     const int t1 = tridiag_reg_split(m);
     if (m > kGrid[0]) {
-        // the strip first (its memory: the second hand-over block), then the chain from 288
+        // the strip first (its memory: the hand-over block of 256, written after it), which
+        // leaves the block of 288 in V; then the chain from there
         if (!work || m > kStripMax) return hipErrorInvalidValue;
-        constexpr int64_t bk = (int64_t)kGrid[0] * kGrid[0];
-        float2* strip = work + nk * bk;
         hipLaunchKernelGGL((tridiag_strip_kernel<kStripMax / 32, kStripCols, NLStrip, IN, THin>), dim3((unsigned)nk), dim3(512),
-                           0, s, H, hk, m, ld, V, ldv, vk, dd, de, dtau, dk, work, bk, strip,
+                           0, s, H, hk, m, ld, V, ldv, vk, dd, de, dtau, dk, work,
                            (int64_t)strip_slots(kStripMax / 32, kStripCols));
         const hipError_t err = hipGetLastError();
         if (err != hipSuccess) return err;
-        const int off = m - kGrid[0];
-        return c64_blocks(kGrid[0], work, strip, nk, V + off + (int64_t)off * ldv, ldv, vk, dd + off, de + off, dtau + off, dk,
-                          s);
+        const int t = tridiag_reg_split(kGrid[0]);
+        int off = m - kGrid[0];
+        float2* B = V + off + (int64_t)off * ldv;
+        grid_stage<float2, 2>(0, (const float2*)B, vk, kGrid[0], ldv, nk, B, ldv, vk, dd + off, de + off, dtau + off, dk,
+                              kGrid[0] - t, work, t, s);
+        off = m - t;
+        return c64_blocks(t, work, work + nk * (int64_t)t * t, nk, V + off + (int64_t)off * ldv, ldv, vk, dd + off, de + off,
+                          dtau + off, dk, s);
     }
     if (!t1) {
         grid_stage<THin, IN>(grid_of(m), H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, m, (float2*)nullptr, 0, s);
