@@ -268,7 +268,9 @@ __global__ __launch_bounds__(BS, 1) void tridiag_blocked_kernel(const double2* H
             const double djj = (double)ys[j].x;
             const double ar = (double)ys[j + 1].x, ai = (double)ys[j + 1].y;
             double beta = ar, tr = 0.0, ti = 0.0, sr = 1.0, si = 0.0;
-            if (!(xn2 == 0.0 && ai == 0.0)) {
+            // no reflector for a column of nothing but tiny elements, as in the other kernels
+            // (scalars.hpp, reflects): 1 / |x| has to stay in range (NaN goes on)
+            if (!(xn2 + ai * ai <= (sizeof(T) == 4 ? 1e-30 : 1e-290))) {
                 const double nrm = sqrt(ar * ar + ai * ai + xn2);
                 beta = ar >= 0 ? -nrm : nrm;
                 const double ib = rcp_nr(beta);
