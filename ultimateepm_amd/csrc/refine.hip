@@ -725,8 +725,8 @@ __device__ bool small_rayleigh_ritz_of(int nbr, S* __restrict__ Ss, S* __restric
     }
     // Wt = L^-1 M (lane = column of M), then U = L^-1 Wt^H (lane = row of Wt): M' = U^H.
     // A row's terms are subtracted in ascending order; a real column stays in registers.
-    auto lower = [&](auto get, auto put) {
-        if constexpr (S::NC == 1) {
+    if constexpr (S::NC == 1) {
+        auto lower = [&](auto get, auto put) {
             S v[LDM];
 #pragma unroll
             for (int r = 0; r < LDM; ++r)
@@ -737,9 +737,7 @@ __device__ bool small_rayleigh_ritz_of(int nbr, S* __restrict__ Ss, S* __restric
                     v[r] = scale(t, 1.0 / Ss[r * LDM + r].x);
                     put(r, v[r]);
                 }
-        }
-    };
-    if constexpr (S::NC == 1) {
+        };
         if (i < nbr) lower([&](int r) { return Mm[r * LDM + i]; }, [&](int r, S v) { Wt[r * LDM + i] = v; });
         wsync();
         if (i < nbr) lower([&](int r) { return Wt[i * LDM + r]; }, [&](int r, S v) { Mm[i * LDM + r] = v; });

@@ -174,12 +174,5 @@ __device__ __forceinline__ typename ScMem<S>::T sc_store(S a) {
     } else v = a;
     return v;
 }
-// component i of a scalar (i a compile-time constant once unrolled)
-template <typename S>
-__device__ __forceinline__ typename S::R sc_comp(const S& a, int i) {
-    if constexpr (S::NC == 1) return a.x;
-    else if constexpr (S::NC == 2) return i == 0 ? a.x : a.y;
-    else return i == 0 ? a.x : i == 1 ? a.y : i == 2 ? a.z : a.w;
-}
 
 }  // namespace uepm

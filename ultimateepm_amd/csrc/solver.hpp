@@ -90,20 +90,19 @@ hipError_t launch_tridiag_reg_c64(const double2* dH, int n, int ld, int64_t nk, 
 // Complex64 register grids for n > 288: the strip kernel takes the steps down to
 // 288 for blocks up to 384 (launch_tridiag_reg_c64 too), the blocked reduction what
 // is above.  The trailing size they take over (a panel boundary of the blocked
-// kernel; n itself for n <= 384) and the launch on a complex64
-// block left in place by the blocked kernel (arguments as for the FP64 form
-// below; the hand-over workspace is tridiag_reg_work_bytes(m)).
+// kernel, 377 .. 384; n itself for n <= 384) and the launch on such a complex64
+// block (289 .. 384) left in place by the blocked kernel (arguments as for the FP64
+// form below; the hand-over workspace is tridiag_reg_work_bytes(m)).
 int tridiag_reg_c64_tail(int n);
 hipError_t launch_tridiag_reg_c64_block(const float2* H, int64_t hk, int m, int ld, int64_t nk, float2* V, int ldv,
                                         int64_t vk, double* dd, double* de, float2* dtau, int64_t dk, float2* work,
                                         hipStream_t s);
 // The same register-resident reduction in FP64 (grids 192 .. 96 and the row
-// kernel, which takes a first block of up to 64 only hermitian_full): trailing
-// size it takes over for a matrix of size n (n itself when n <= 192), its
-// hand-over workspace per k-point (bytes), and the
+// kernel): trailing size it takes over for a matrix of size n (n itself when
+// n <= 192, else 189 .. 192), its hand-over workspace per k-point (bytes), and the
 // launch on a block of size m whose element (0, 0) sits at H (leading
 // dimension ld, per-k stride hk; hermitian_full: both triangles hold the
-// Hermitian block, else only its lower triangle); reflectors, d, e, tau at the
+// Hermitian block, else only its lower triangle, m > 160); reflectors, d, e, tau at the
 // block's offset of the full matrix's outputs (V may alias H: each stage loads
 // its block before it writes, and writes only below the sub-diagonal).
 int tridiag_reg_c128_tail(int n);

@@ -1,7 +1,7 @@
 // tridiag_grid.hpp — register-resident Householder reduction of a Hermitian
 // block on a grid of lanes, one workgroup per k-point (gfx950); real, complex
 // and quaternion elements (scalars.hpp) in FP32 or FP64.  The chains of
-// shrinking grids are in tridiag_reg.hip (complex) and tridiag_real.hip.
+// shrinking grids are in tridiag_reg.hip, tridiag_real.hip and tridiag_quaternion.hip.
 //
 // Layout.  The lanes form a PR x PC = 32 x 16 (or 16 x 16) grid: lane (r, c) with
 // c = tid % 16, r = tid / 16 (a wave holds four r values and all sixteen c).

@@ -1,9 +1,10 @@
-// tridiag_reg.hip — register-resident Householder reduction of a Hermitian
-// H(k) to real symmetric tridiagonal form, one 512-lane workgroup per
-// k-point (gfx950): complex64 arithmetic for the precision form (dim <= 288),
-// complex128 for the FP64 form (dim <= 192), and a chain of shrinking grids
-// (below).
-// The grids' layout and steps are described in tridiag_grid.hpp.
+// tridiag_reg.hip — Householder reduction of a complex Hermitian H(k) to real
+// symmetric tridiagonal form, one workgroup per k-point and kernel (gfx950): a
+// chain of shrinking register grids (256 or 512 lanes, tridiag_grid.hpp) that ends
+// in a wave (complex64) or the row kernel (complex128, tridiag_row.hpp).
+// Complex64 for the precision form: whole matrices to dim 288, to 384 after the
+// strip kernel (tridiag_strip.hpp); complex128 for the FP64 form: to dim 192.
+// Larger ones come from the blocked reduction (tridiag_blocked.hip).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -29,9 +30,8 @@ namespace uepm {
 // the workgroup.  Columns are processed in blocks of 8, skipped once they are
 // past the live part (those registers are never read again).  Same outputs
 // as the grid kernels (d, e, tau, reflectors below the sub-diagonal of column
-// s of Vout).  The block is read as the grids read it (IN: 0 lower triangle
-// by columns, 1 conjugate of the upper triangle of a full Hermitian matrix,
-// 2 lower triangle by rows).
+// s of Vout).  The block is read as the grids read it (IN: 1 conjugate of the
+// upper triangle of a full Hermitian matrix, 2 lower triangle by rows).
 template <int IN, typename THin>
 __global__ __launch_bounds__(64, 2) void tridiag_wave64_kernel(const THin* __restrict__ Hin, int64_t h_kstride, int n,
                                                                int ld, float2* __restrict__ Vout, int ldv,
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(64, 2) void tridiag_wave64_kernel(const THin* __res
         if (i < n && j < n) {
             // lower element A(r, c), r >= c, as the grids read it
             const int r = j <= i ? i : j, c = j <= i ? j : i;
-            const THin h = H[IN == 0 ? r + (int64_t)c * ld : c + (int64_t)r * ld];
+            const THin h = H[c + (int64_t)r * ld];
             const float hx = (float)h.x, hy = IN == 1 ? -(float)h.y : (float)h.y;
             a = j <= i ? f2{hx, hy} : f2{hx, -hy};  // A(i, j) = conj(A(j, i)) above the diagonal
         }
@@ -224,7 +224,7 @@ void grid_stage(int g, const THin* H, int64_t hk, int m, int ld, int64_t nk, flo
         case 3: reg_stage<c2<float>, 32, 6, 4, IN, THin, true, NL192>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         case 4: reg_stage<c2<float>, 16, 10, 3, IN, THin, true, NL160>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         case 5:
-            if constexpr (IN != 2) reg_stage<c2<float>, 16, 9, 4, IN, THin, true, NL144>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
+            if constexpr (IN == 1) reg_stage<c2<float>, 16, 9, 4, IN, THin, true, NL144>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
             break;
         case 6: reg_stage<c2<float>, 16, 8, 4, IN, THin, true, NL128>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
         case 7: reg_stage<c2<float>, 16, 6, 4, IN, THin>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
@@ -257,42 +257,28 @@ hipError_t c64_blocks(int r, float2* cur, float2* next, int64_t nk, float2* V, i
 constexpr int kStripMax = 384, kStripCols = (kStripMax - kGrid[0]) / 16, NLStrip = 30;
 static_assert(strip_slots(kStripMax / 32, kStripCols) <= kGrid[1] * kGrid[1], "the strip fits a hand-over block");
 
-// The complex64 chain on a block of size m whose element (0, 0) sits at H
-// (leading dimension ld, per-k stride hk; read as IN says, IN = 0 or 1);
-// outputs at the block's offset of the full matrix's V (ldv, stride vk) and
-// d, e, tau (stride dk).
+// The complex64 chain above 288 on a block of size m whose element (0, 0) sits at H
+// (leading dimension ld, per-k stride hk; read as IN says, IN = 0 or 1); outputs at the
+// block's offset of the full matrix's V (ldv, stride vk) and d, e, tau (stride dk).  The
+// strip first (its memory: the hand-over block of 256, written after it), which leaves
+// the block of 288 in V; then the chain from there.
 template <int IN, typename THin>
-hipError_t c64_chain(const THin* H, int64_t hk, int m, int ld, int64_t nk, float2* V, int ldv, int64_t vk, double* dd,
-                     double* de, float2* dtau, int64_t dk, float2* work, hipStream_t s) {
-    const int t1 = tridiag_reg_split(m);
-    if (m > kGrid[0]) {
-        // the strip first (its memory: the hand-over block of 256, written after it), which
-        // leaves the block of 288 in V; then the chain from there
-        if (!work || m > kStripMax) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((tridiag_strip_kernel<kStripMax / 32, kStripCols, NLStrip, IN, THin>), dim3((unsigned)nk), dim3(512),
-                           0, s, H, hk, m, ld, V, ldv, vk, dd, de, dtau, dk, work,
-                           (int64_t)strip_slots(kStripMax / 32, kStripCols));
-        const hipError_t err = hipGetLastError();
-        if (err != hipSuccess) return err;
-        const int t = tridiag_reg_split(kGrid[0]);
-        int off = m - kGrid[0];
-        float2* B = V + off + (int64_t)off * ldv;
-        grid_stage<float2, 2>(0, (const float2*)B, vk, kGrid[0], ldv, nk, B, ldv, vk, dd + off, de + off, dtau + off, dk,
-                              kGrid[0] - t, work, t, s);
-        off = m - t;
-        return c64_blocks(t, work, work + nk * (int64_t)t * t, nk, V + off + (int64_t)off * ldv, ldv, vk, dd + off, de + off,
-                          dtau + off, dk, s);
-    }
-    if (!t1) {
-        grid_stage<THin, IN>(grid_of(m), H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, m, (float2*)nullptr, 0, s);
-        return hipGetLastError();
-    }
-    if (!work) return hipErrorInvalidValue;
-    // first grid on the block, then each smaller grid on the trailing block of its size
-    float2* next = work + nk * (int64_t)t1 * t1;
-    grid_stage<THin, IN>(grid_of(m), H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, m - t1, work, t1, s);
-    const int off = m - t1;
-    return c64_blocks(t1, work, next, nk, V + off + (int64_t)off * ldv, ldv, vk, dd + off, de + off, dtau + off, dk, s);
+hipError_t strip_chain(const THin* H, int64_t hk, int m, int ld, int64_t nk, float2* V, int ldv, int64_t vk, double* dd,
+                       double* de, float2* dtau, int64_t dk, float2* work, hipStream_t s) {
+    if (!work || m <= kGrid[0] || m > kStripMax) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((tridiag_strip_kernel<kStripMax / 32, kStripCols, NLStrip, IN, THin>), dim3((unsigned)nk), dim3(512),
+                       0, s, H, hk, m, ld, V, ldv, vk, dd, de, dtau, dk, work,
+                       (int64_t)strip_slots(kStripMax / 32, kStripCols));
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    const int t = tridiag_reg_split(kGrid[0]);
+    int off = m - kGrid[0];
+    float2* B = V + off + (int64_t)off * ldv;
+    grid_stage<float2, 2>(0, (const float2*)B, vk, kGrid[0], ldv, nk, B, ldv, vk, dd + off, de + off, dtau + off, dk,
+                          kGrid[0] - t, work, t, s);
+    off = m - t;
+    return c64_blocks(t, work, work + nk * (int64_t)t * t, nk, V + off + (int64_t)off * ldv, ldv, vk, dd + off, de + off,
+                      dtau + off, dk, s);
 }
 }  // namespace
 
@@ -300,7 +286,16 @@ hipError_t launch_tridiag_reg_c64(const double2* dH, int n, int ld, int64_t nk, 
                                   float2* dtau, float2* work, hipStream_t s) {
     if (n < 1 || n > kStripMax || nk <= 0) return hipErrorInvalidValue;
     const int64_t hk = (int64_t)ld * n;
-    return c64_chain<1>(dH, hk, n, ld, nk, Vout, ld, hk, dd, de, dtau, n, work, s);
+    if (n > kGrid[0]) return strip_chain<1>(dH, hk, n, ld, nk, Vout, ld, hk, dd, de, dtau, n, work, s);
+    const int t = tridiag_reg_split(n);
+    if (t && !work) return hipErrorInvalidValue;
+    // first grid on the matrix, then each smaller grid on the trailing block of its size
+    grid_stage<double2, 1>(grid_of(n), dH, hk, n, ld, nk, Vout, ld, hk, dd, de, dtau, n, t ? n - t : n,
+                           t ? work : (float2*)nullptr, t, s);
+    if (!t) return hipGetLastError();
+    const int off = n - t;
+    return c64_blocks(t, work, work + nk * (int64_t)t * t, nk, Vout + off + (int64_t)off * ld, ld, hk, dd + off, de + off,
+                      dtau + off, n, s);
 }
 
 int tridiag_reg_c64_tail(int n) {
@@ -314,8 +309,8 @@ int tridiag_reg_c64_tail(int n) {
 hipError_t launch_tridiag_reg_c64_block(const float2* H, int64_t hk, int m, int ld, int64_t nk, float2* V, int ldv,
                                         int64_t vk, double* dd, double* de, float2* dtau, int64_t dk, float2* work,
                                         hipStream_t s) {
-    if (m < 1 || m > kStripMax || nk <= 0) return hipErrorInvalidValue;
-    return c64_chain<0>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, work, s);
+    if (nk <= 0) return hipErrorInvalidValue;
+    return strip_chain<0>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, work, s);
 }
 
 // ---- FP64: grids 192 (10 of 42 blocks in LDS) and 160 of 32 x 16 lanes, 256 and 236
@@ -343,21 +338,25 @@ constexpr int NL64_192 = 10, NL64_144 = 12, NL64_128 = 2, NL64_96 = 4;  // block
 template <int IN>
 void grid64_stage(int g, const double2* H, int64_t hk, int m, int ld, int64_t nk, double2* V, int ldv, int64_t vk,
                   double* dd, double* de, double2* dtau, int64_t dk, int s_end, double2* B, int ldb, hipStream_t s) {
-    switch (g) {
-        case 0: reg_stage<c2<double>, 32, 6, 1, IN, double2, true, NL64_192>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 1: reg_stage<c2<double>, 32, 5, 1, IN, double2, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 2:
-            if constexpr (IN != 2) reg_stage<c2<double>, 16, 9, 2, IN, double2, true, NL64_144>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
-            break;
-        case 3: reg_stage<c2<double>, 16, 8, 2, IN, double2, true, NL64_128>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        // hands both triangles to the row kernel
-        case 4: reg_stage<c2<double>, 16, 6, 3, IN, double2, true, NL64_96, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        default:
-            if constexpr (IN != 0) {
+    if constexpr (IN == 0) {  // what the blocked reduction leaves: 189 .. 192
+        reg_stage<c2<double>, 32, 6, 1, IN, double2, true, NL64_192>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
+    } else {
+        switch (g) {
+            case 0:
+                if constexpr (IN == 1) reg_stage<c2<double>, 32, 6, 1, IN, double2, true, NL64_192>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
+                break;
+            case 1: reg_stage<c2<double>, 32, 5, 1, IN, double2, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+            case 2:
+                if constexpr (IN == 1) reg_stage<c2<double>, 16, 9, 2, IN, double2, true, NL64_144>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
+                break;
+            case 3: reg_stage<c2<double>, 16, 8, 2, IN, double2, true, NL64_128>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+            // hands both triangles to the row kernel
+            case 4: reg_stage<c2<double>, 16, 6, 3, IN, double2, true, NL64_96, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+            default:
                 if (m <= 32) row_stage<c2<double>, 1, 1, 2, 2, IN>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
                 else row_stage<c2<double>, 1, 2, 2, 2, IN>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
-            }
-            break;
+                break;
+        }
     }
 }
 }  // namespace
@@ -382,7 +381,7 @@ hipError_t launch_tridiag_reg_c128(const double2* H, int64_t hk, int m, int ld, 
                                    double2* V, int ldv, int64_t vk, double* dd, double* de, double2* dtau, int64_t dk,
                                    double2* work, hipStream_t s) {
     if (m < 1 || m > kGrid64[0] || nk <= 0) return hipErrorInvalidValue;
-    if (!hermitian_full && grid64_of(m) == kNumGrids64 - 1) return hipErrorInvalidValue;  // the row kernel reads both triangles
+    if (!hermitian_full && grid64_of(m) != 0) return hipErrorInvalidValue;
     // the first grid reads the block's rows (the conjugate upper triangle) when
     // the whole Hermitian matrix is there, its lower columns otherwise
     auto first = [&](int s_end, double2* B, int ldb) {

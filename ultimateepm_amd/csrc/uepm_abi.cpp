@@ -53,8 +53,9 @@ int64_t plan_chunk(const uepm_plan* p, int64_t nk) {
 }
 
 namespace {
-// Trailing size that the register grids (with the strip kernel up to n = 384) take over
-// in the precision form above n = 288, after a blocked reduction if less than n; 0 when the configuration asks for the blocked kernel.
+// Trailing size that the register grids (with the strip kernel up to n = 384) take
+// over in the precision form above n = 288, after a blocked reduction if less than n;
+// 0 when the configuration asks for the blocked kernel.
 int mixed_c64_tail(const uepm_plan* p) {
     if (p->tri_reg || p->cfg.tridiag == 1 || p->dim <= uepm::tridiag_reg_max_n()) return 0;
     return uepm::tridiag_reg_c64_tail(p->dim);
@@ -126,7 +127,7 @@ Sizes plan_sizes(const uepm_plan* p, int64_t chunk) {
     }
     if (stage_vec) {
         z.Z = sizeof(double) * (size_t)n * nbr * chunk;
-        z.W = sizeof(double) * 4 * (size_t)n * nbr * chunk;  // U factor (3 rows) + iterate
+        z.W = sizeof(double) * 4 * (size_t)n * nbr * chunk;  // two iterates, elimination states, norms (launch_tri_eig)
         if (!mixed) z.X = sizeof(double2) * (size_t)n * nb * chunk;
     }
     z.kstat = sizeof(int) * (size_t)chunk;
