@@ -91,9 +91,12 @@ constexpr double kSturmPad = 16.0;
 // per band): a sweep narrows the bracket of every band S + 1-fold.  d and e^2,
 // scaled, sit in LDS, uniform reads across the wave.  A bracket is final at the
 // rounding level of its eigenvalue, or narrower than abstol_rel ||T||_inf.  At N = 181,
-// 16 bands, 4096 k-points (two chunks in flight) it takes 0.26 ms against 0.45 ms
-// with the ratio form of the count (a division a row) and unpadded rows; bound by
-// FP64 issue, and at one k-point by the chain of fmas (69 us for 11 sweeps).
+// 16 bands, 4096 k-points (two chunks in flight) the precision form's takes 0.26 ms
+// against 0.45 ms with the ratio form of the count (a division a row) and unpadded
+// rows.  Alone on the chip it is bound by those reads (LDS busy 80% of the cycles, FP64
+// issue 57%), at one k-point by the chain of fmas (72 us).
+// Held final at eps / 16 ||T|| the FP64 brackets would close one to three sweeps
+// earlier (3000 k-points in flight, 0.33 -> 0.30 ms), and levels near zero lose digits.
 template <int S>
 __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __restrict__ dall,
                                                           const double* __restrict__ eall, int n, int nb,

@@ -211,11 +211,11 @@ void plan_apply_config(uepm_plan* p) {
     // A crystal of equal atoms has an inversion centre: without spin-orbit every
     // imaginary part of H(k) is exactly zero (V_A = 0, and the antisymmetric half of
     // two equal non-local terms), so the real kernels take the plan.  Si N = 181, 12
-    // bands and vectors: precision form 29.1 -> 15.1 ms per 16,001 k-points, FP64
-    // 22.1 -> 7.9 ms per 6,000.
+    // bands and vectors: precision form 29.1 -> 13.1 ms per 16,001 k-points, FP64
+    // 22.1 -> 6.9 ms per 6,000.
     // With spin-orbit the same crystal's H(k) is a quaternion matrix of half the
     // dimension, and every level a Kramers pair found once: Ge, dim 274, 16 bands,
-    // precision form 19.7 -> 9.2 ms per 3,000 k-points, FP64 18.3 -> 5.0 ms per 961.
+    // precision form 19.7 -> 7.2 ms per 3,000 k-points, FP64 18.3 -> 3.5 ms per 961.
     p->quat = p->inversion && (p->flags & UEPM_SOC) && p->soc_symmetric && p->cfg.tridiag != 1 &&
               p->N <= uepm::tridiag_quaternion_max_n(mixed);
     p->real = p->inversion && !(p->flags & UEPM_SOC) && p->cfg.tridiag != 1 && p->dim <= uepm::tridiag_real_max_n(mixed);
