@@ -147,8 +147,12 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
         if (live && sub == 0) evals[kk * nb + b] = __builtin_nan("");
         return;
     }
+    if (tnorm == 0.0) {  // the floor of e^2 would split the levels
+        if (live && sub == 0) evals[kk * nb + b] = 0.0;
+        return;
+    }
     // scaled by a power of two (exact) to 1 <= ||T|| < 2
-    const int ex = tnorm > 0.0 ? 1 - __builtin_amdgcn_frexp_exp(tnorm) : 0;
+    const int ex = 1 - __builtin_amdgcn_frexp_exp(tnorm);
     auto scaled = [&](double v) { return __builtin_amdgcn_ldexp(v, ex); };
     for (int i = lane; i < np; i += 64) {
         const double ei = i > 0 && i < n ? scaled(e[i - 1]) : 0.0;
@@ -241,10 +245,14 @@ __global__ __launch_bounds__(64, 2) void tri_vec_kernel(const double* __restrict
     }
     const double* d = dall + kk * n;
     const double* e = eall + kk * n;
-    const double lam = evals[t];
+    // T scaled by a power of two (exact), or the last iterate of a tiny T would have no
+    // norm in range; a T of zeros counts as of norm 1
+    const double tnorm = tnorms[kk];
+    const double scl = tnorm > 0.0 ? __builtin_amdgcn_ldexp(1.0, min(1 - __builtin_amdgcn_frexp_exp(tnorm), 1000)) : 1.0;
+    const double lam = evals[t] * scl;
     // smallest pivot: under the rounding of T, and large enough that a run of equal
     // levels with next to no coupling cannot grow the iterate out of range
-    const double tiny = fmax(0x1p-10 * DBL_EPSILON * tnorms[kk], DBL_MIN);
+    const double tiny = 0x1p-10 * DBL_EPSILON * (tnorm > 0.0 ? tnorm * scl : 1.0);
     auto at_least_tiny = [&](double a) { return fabs(a) < tiny ? copysign(tiny, a) : a; };
     const int nblk = (n - 1 + kRows - 1) / kRows;  // blocks of eliminated rows 0 .. n - 2
     double* __restrict__ C = W + (size_t)2 * n * T;  // (a, c, y) at every block's first row
@@ -264,17 +272,17 @@ __global__ __launch_bounds__(64, 2) void tri_vec_kernel(const double* __restrict
 #pragma unroll
             for (int u = 0; u < kRows; ++u) {
                 const int k = k0 + u;
-                r.e[u] = e[min(k, n - 1)];
+                r.e[u] = e[min(k, n - 1)] * scl;
                 r.d[u] = d[min(k + 1, n - 1)];
                 if (!first) r.y[u] = Xin[(size_t)min(k + 1, n - 1) * T + t];
             }
-            r.e[kRows] = e[min(k0 + kRows, n - 1)];
+            r.e[kRows] = e[min(k0 + kRows, n - 1)] * scl;
         };
         // eliminates row k = k0 + u: multipliers and interchange applied to the state;
         // out: reciprocal pivot, first and second super-diagonal of U, forward result
         auto eliminate = [&](State& s, const Rows& r, int k, int u, double* out) {
             const double sub = r.e[u];
-            const double dn = r.d[u] - lam;
+            const double dn = fma(r.d[u], scl, -lam);
             const double en = k + 2 < n ? r.e[u + 1] : 0.0;
             const double y1 = first ? lane_rand((uint32_t)(k + 1), b) : r.y[u] * sc;
             const double a = at_least_tiny(s.a);
@@ -294,7 +302,7 @@ __global__ __launch_bounds__(64, 2) void tri_vec_kernel(const double* __restrict
                 out[3] = top;
             }
         };
-        State s{d[0] - lam, n > 1 ? e[0] : 0.0, first ? lane_rand(0u, b) : Xin[t] * sc};
+        State s{fma(d[0], scl, -lam), n > 1 ? e[0] * scl : 0.0, first ? lane_rand(0u, b) : Xin[t] * sc};
         for (int blk = 0; blk < nblk; ++blk) {
             C[(size_t)(3 * blk) * T + t] = s.a;
             C[(size_t)(3 * blk + 1) * T + t] = s.c;
