@@ -90,13 +90,15 @@ constexpr double kSturmPad = 16.0;
 // Eigenvalues of T by multisection, one wave per k-point and 64 / S bands (S probes
 // per band): a sweep narrows the bracket of every band S + 1-fold.  d and e^2,
 // scaled, sit in LDS, uniform reads across the wave.  A bracket is final at the
-// rounding level of its eigenvalue, or narrower than abstol_rel ||T||_inf.  At N = 181,
+// rounding level of its eigenvalue or narrower than abstol_rel ||T||_inf; where every
+// coupling is felt (e^2 >= eps ||T||^2) also at a sixteenth of the rounding of ||T||, of
+// which the reduction has put several into such a T: levels near zero then close one to
+// three sweeps earlier (240 k-points, N = 137: 72 us instead of 86).  A T that decouples
+// may hold levels of H(k) to their own digits, and keeps them.  At N = 181,
 // 16 bands, 4096 k-points (two chunks in flight) the precision form's takes 0.26 ms
 // against 0.45 ms with the ratio form of the count (a division a row) and unpadded
 // rows.  Alone on the chip it is bound by those reads (LDS busy 80% of the cycles, FP64
 // issue 57%), at one k-point by the chain of fmas (72 us).
-// Held final at eps / 16 ||T|| the FP64 brackets would close one to three sweeps
-// earlier (3000 k-points in flight, 0.33 -> 0.30 ms), and levels near zero lose digits.
 template <int S>
 __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __restrict__ dall,
                                                           const double* __restrict__ eall, int n, int nb,
@@ -115,7 +117,7 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
     double* const sd = tri_lds;
     double* const se2 = tri_lds + np;
     // Gershgorin interval and scale
-    double lo = DBL_MAX, hi = -DBL_MAX, tnorm = 0.0;
+    double lo = DBL_MAX, hi = -DBL_MAX, tnorm = 0.0, emin = DBL_MAX;
     bool finite = true;
     for (int i = lane; i < n; i += 64) {
         const double di = d[i], el = i > 0 ? fabs(e[i - 1]) : 0.0, er = i + 1 < n ? fabs(e[i]) : 0.0;
@@ -123,8 +125,10 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
         lo = fmin(lo, di - el - er);
         hi = fmax(hi, di + el + er);
         tnorm = fmax(tnorm, fabs(di) + el + er);
+        if (i + 1 < n || n == 1) emin = fmin(emin, er);
     }
     for (int o = 32; o > 0; o >>= 1) {
+        emin = fmin(emin, __shfl_xor(emin, o, 64));
         lo = fmin(lo, __shfl_xor(lo, o, 64));
         hi = fmax(hi, __shfl_xor(hi, o, 64));
         tnorm = fmax(tnorm, __shfl_xor(tnorm, o, 64));
@@ -164,7 +168,9 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
     tnorm = scaled(tnorm);
     lo = scaled(lo) - 2.0 * eps * tnorm - 0x1p-58;  // and what the floor of e^2 may move
     hi = scaled(hi) + 2.0 * eps * tnorm + 0x1p-58;
-    const double abstol = abstol_rel * tnorm;
+    emin = scaled(emin);
+    const bool coupled = emin * emin >= eps * tnorm * tnorm;
+    const double abstol = fmax(abstol_rel, coupled ? eps / 16.0 : 0.0) * tnorm;
     // two shared sweeps first: the wave's 64 lanes probe one interval that holds
     // every band of the wave, and each band takes the probes around its index
     // (a count c at x puts eigenvalues 0..c-1 below x and c.. at or above it)
