@@ -93,12 +93,12 @@ constexpr double kSturmPad = 16.0;
 // rounding level of its eigenvalue or narrower than abstol_rel ||T||_inf; where every
 // coupling is felt (e^2 >= eps ||T||^2) also at a sixteenth of the rounding of ||T||, of
 // which the reduction has put several into such a T: levels near zero then close one to
-// three sweeps earlier (240 k-points, N = 137: 72 us instead of 86).  A T that decouples
+// three sweeps earlier (240 k-points, N = 137: 71 us instead of 86).  A T that decouples
 // may hold levels of H(k) to their own digits, and keeps them.  At N = 181,
 // 16 bands, 4096 k-points (two chunks in flight) the precision form's takes 0.26 ms
 // against 0.45 ms with the ratio form of the count (a division a row) and unpadded
 // rows.  Alone on the chip it is bound by those reads (LDS busy 80% of the cycles, FP64
-// issue 57%), at one k-point by the chain of fmas (72 us).
+// issue 57%), at one k-point by the chain of fmas (69 us).
 template <int S>
 __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __restrict__ dall,
                                                           const double* __restrict__ eall, int n, int nb,
