@@ -48,9 +48,11 @@ hipError_t launch_status_reset(unsigned long long* status, hipStream_t s);
 // abstol_rel > 0 ends bisection at brackets narrower than abstol_rel ||T||_inf
 // (the precision form, whose T carries complex64 rounding); 0 bisects to the
 // rounding level of each eigenvalue.
-// inv_sweeps: inverse-iteration sweeps for the eigenvectors of T (0: eigenvalues only).
+// inv_sweeps: inverse-iteration sweeps for the eigenvectors of T (0: eigenvalues only);
+// dW then provides tri_eig_work_doubles(n, nb) per k-point.
 // A non-finite T gives NaN eigenvalues and vectors and is flagged in kstat
 // (when not null) or else added to status (when not null).
+size_t tri_eig_work_doubles(int n, int nb);
 hipError_t launch_tri_eig(const double* dd, const double* de, int n, int nb, int64_t nk, double* devals, double* dZ,
                           double* dW, int inv_sweeps, double abstol_rel, int* kstat, unsigned long long* status,
                           int64_t k0, hipStream_t s);

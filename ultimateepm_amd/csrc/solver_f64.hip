@@ -236,6 +236,7 @@ __global__ __launch_bounds__(64, 4) void tri_eig_wave_kernel(const double* __res
 // normalised: cluster_orth_kernel does that.  N = 181, 16 bands, 4096 k-points, two
 // chunks in flight: 0.33 ms against 0.58 ms with the factors in memory.
 constexpr int kRows = 8;
+size_t tri_eig_work_doubles(int n, int nb) { return (size_t)(2 * n + 3 * ((n - 1 + kRows - 1) / kRows)) * nb + 1; }
 __global__ __launch_bounds__(64, 2) void tri_vec_kernel(const double* __restrict__ dall, const double* __restrict__ eall,
                                                         int n, int nb, int64_t T, const double* __restrict__ evals,
                                                         const double* __restrict__ tnorms, const int* __restrict__ kstat,
@@ -357,7 +358,7 @@ hipError_t launch_tri_eig(const double* dd, const double* de, int n, int nb, int
     const size_t shm = sizeof(double) * 2 * (size_t)((n + 15) & ~15);  // d and e^2 of the k-point
     const int64_t T = nk * nb;
     // the work array holds two iterates, the elimination states and, last, the norms
-    double* tnorms = inv_sweeps > 0 ? dW + (size_t)4 * n * T - nk : nullptr;
+    double* tnorms = inv_sweeps > 0 ? dW + nk * (tri_eig_work_doubles(n, nb) - 1) : nullptr;
     auto eig = [&](auto kern, int bands) {
         hipLaunchKernelGGL(kern, dim3((unsigned)nk, (unsigned)((nb + bands - 1) / bands)), dim3(64), shm, s, dd, de, n, nb,
                            devals, tnorms, abstol_rel, kstat, status, k0);

@@ -116,15 +116,16 @@ struct RegLayout {
 // Stage arguments: steps s < s_end run here (s_end >= n - 1: the whole
 // reduction); when s_end < n - 1 the updated trailing block A[s_end:, s_end:]
 // (lower triangle, full diagonal) goes to Bout row by row (element (i, j) at
-// j + i ldb, ldb * ldb per k; FULL: and its conjugate above the diagonal) for a
+// j + i ldb, b_kstride per k; FULL: and its conjugate above the diagonal) for a
 // smaller grid to continue.  IN says how
 // the lower triangle of the input is read: 0, column-major (element (i, j) at
 // i + j ld); 1, as the conjugate of the upper triangle of a full Hermitian
 // matrix (element (j, i) at j + i ld); 2, row by row as a hand-over block.  Input (leading
 // dimension ld), reflectors (ldv) and d, e, tau of k-point kk start at
 // kk * h_kstride, kk * v_kstride and kk * de_kstride.  The reflectors may go over the
-// input (the FP64 form), so neither pointer is __restrict__: the input is read before
-// the first step, which writes the first of them.
+// input (the FP64 form) and so may the hand-over block (the complex64 chain), so none
+// of the three pointers is __restrict__: the input is read before the first step, which
+// writes the first reflector; the block is written after the last.
 template <int PR, int PC, int LR, int LC, int MINWG, typename S, typename THin, bool LOW = false, int NL = 0, int IN = 0,
           bool FULL = false>
 __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* Hin, int64_t h_kstride,
@@ -134,7 +135,7 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
                                                                     double* __restrict__ eout,
                                                                     typename ScMem<S>::T* __restrict__ tauout,
                                                                     int64_t de_kstride, int s_end,
-                                                                    typename ScMem<S>::T* __restrict__ Bout, int ldb) {
+                                                                    typename ScMem<S>::T* Bout, int ldb, int64_t b_kstride) {
     using R = typename S::R;
     using VT = typename ScMem<S>::T;
     constexpr int NC = S::NC;
@@ -408,7 +409,7 @@ __global__ __launch_bounds__(PR* PC, MINWG) void tridiag_reg_kernel(const THin* 
     }
     if (s_stop < n - 1) {
         // hand the trailing block A[s_stop:, s_stop:] over
-        VT* B = Bout + kk * (int64_t)ldb * ldb;
+        VT* B = Bout + kk * b_kstride;
 #pragma unroll
         for (int l = 0; l < LR; ++l)
 #pragma unroll
@@ -443,10 +444,10 @@ namespace {
 template <typename S, int PR, int LR, int MINWG, int IN, typename THin, bool LOW = false, int NL = 0, bool FULL = false>
 void reg_stage(const THin* H, int64_t h_kstride, int n, int ld, int64_t nk, typename ScMem<S>::T* V, int ldv,
                int64_t v_kstride, double* dd, double* de, typename ScMem<S>::T* dtau, int64_t de_kstride, int s_end,
-               typename ScMem<S>::T* B, int ldb, hipStream_t s) {
+               typename ScMem<S>::T* B, int ldb, hipStream_t s, int64_t b_kstride = 0) {
     hipLaunchKernelGGL((tridiag_reg_kernel<PR, 16, LR, LR * PR / 16, MINWG, S, THin, LOW, NL, IN, FULL>),
                        dim3((unsigned)nk), dim3(PR * 16), 0, s, H, h_kstride, n, ld, V, ldv, v_kstride, dd, de, dtau,
-                       de_kstride, s_end, B, ldb);
+                       de_kstride, s_end, B, ldb, b_kstride ? b_kstride : (int64_t)ldb * ldb);
 }
 }  // namespace
 

@@ -7,9 +7,7 @@
 // Larger ones come from the blocked reduction (tridiag_blocked.hip).
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cstdint>
-#include <utility>
 #include <cstdlib>
 
 #include "solver.hpp"
@@ -195,15 +193,6 @@ int tridiag_reg_split(int n) {
     return g < kNumGrids - 1 ? kGrid[g + 1] : 0;
 }
 
-size_t tridiag_reg_work_bytes(int n) {
-    // two ping-pong hand-over blocks: the first hand-over's size and the next one's (the
-    // strip kernel hands over in place, and its strip lies in the first of the next two)
-    const int t1 = tridiag_reg_split(std::min(n, kGrid[0]));
-    if (!t1) return 0;
-    const int t2 = tridiag_reg_split(t1);
-    return sizeof(float2) * ((size_t)t1 * t1 + (size_t)t2 * t2);
-}
-
 namespace {
 template <int IN, typename THin>
 void wave64_stage(const THin* H, int64_t h_kstride, int n, int ld, int64_t nk, float2* V, int ldv, int64_t v_kstride,
@@ -216,37 +205,36 @@ constexpr int NL288 = 16, NL192 = 14, NL160 = 12, NL144 = 14, NL128 = 10;  // bl
 
 template <typename THin, int IN>
 void grid_stage(int g, const THin* H, int64_t hk, int m, int ld, int64_t nk, float2* V, int ldv, int64_t vk,
-                double* dd, double* de, float2* dtau, int64_t dk, int s_end, float2* B, int ldb, hipStream_t s) {
+                double* dd, double* de, float2* dtau, int64_t dk, int s_end, float2* B, int ldb, int64_t bk, hipStream_t s) {
     switch (g) {
-        case 0: reg_stage<c2<float>, 32, 9, 2, IN, THin, true, NL288>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 1: reg_stage<c2<float>, 32, 8, 2, IN, THin, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 2: reg_stage<c2<float>, 32, 7, 2, IN, THin, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 3: reg_stage<c2<float>, 32, 6, 4, IN, THin, true, NL192>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 4: reg_stage<c2<float>, 16, 10, 3, IN, THin, true, NL160>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        case 0: reg_stage<c2<float>, 32, 9, 2, IN, THin, true, NL288>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s, bk); break;
+        case 1: reg_stage<c2<float>, 32, 8, 2, IN, THin, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s, bk); break;
+        case 2: reg_stage<c2<float>, 32, 7, 2, IN, THin, true>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s, bk); break;
+        case 3: reg_stage<c2<float>, 32, 6, 4, IN, THin, true, NL192>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s, bk); break;
+        case 4: reg_stage<c2<float>, 16, 10, 3, IN, THin, true, NL160>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s, bk); break;
         case 5:
-            if constexpr (IN == 1) reg_stage<c2<float>, 16, 9, 4, IN, THin, true, NL144>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s);
+            if constexpr (IN == 1) reg_stage<c2<float>, 16, 9, 4, IN, THin, true, NL144>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s, bk);
             break;
-        case 6: reg_stage<c2<float>, 16, 8, 4, IN, THin, true, NL128>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
-        case 7: reg_stage<c2<float>, 16, 6, 4, IN, THin>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s); break;
+        case 6: reg_stage<c2<float>, 16, 8, 4, IN, THin, true, NL128>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s, bk); break;
+        case 7: reg_stage<c2<float>, 16, 6, 4, IN, THin>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s_end, B, ldb, s, bk); break;
         default: wave64_stage<IN, THin>(H, hk, m, ld, nk, V, ldv, vk, dd, de, dtau, dk, s); break;  // last: s_end >= m - 1
     }
 }
 }  // namespace
 
 namespace {
-// The rest of a complex64 chain: a hand-over block of size r, then each smaller
-// grid's, in ping-pong blocks (the block of size t lives at k * t * t; a stage reads
-// all of its block before it writes the next); outputs at the block's own offset.
-hipError_t c64_blocks(int r, float2* cur, float2* next, int64_t nk, float2* V, int ldv, int64_t vk, double* dd, double* de,
+// The rest of a complex64 chain: the hand-over block of size r in work (bk per k), then
+// each smaller grid's over it (a stage reads its whole block before its first step and
+// writes the next after its last); outputs at the block's own offset.
+hipError_t c64_blocks(int r, float2* work, int64_t bk, int64_t nk, float2* V, int ldv, int64_t vk, double* dd, double* de,
                       float2* dtau, int64_t dk, hipStream_t s) {
     for (int off = 0;;) {
         const int t = tridiag_reg_split(r);
-        grid_stage<float2, 2>(grid_of(r), (const float2*)cur, (int64_t)r * r, r, r, nk, V + off + (int64_t)off * ldv, ldv, vk,
-                              dd + off, de + off, dtau + off, dk, t ? r - t : r, t ? next : (float2*)nullptr, t, s);
+        grid_stage<float2, 2>(grid_of(r), (const float2*)work, bk, r, r, nk, V + off + (int64_t)off * ldv, ldv, vk, dd + off,
+                              de + off, dtau + off, dk, t ? r - t : r, t ? work : (float2*)nullptr, t, bk, s);
         if (!t) break;
         off += r - t;
         r = t;
-        std::swap(cur, next);
     }
     return hipGetLastError();
 }
@@ -255,32 +243,31 @@ hipError_t c64_blocks(int r, float2* cur, float2* next, int64_t nk, float2* V, i
 // as fast as the blocked reduction at 362; every column of a longer strip adds as much to
 // the first step's traffic, and at 96 columns that is what the blocked one streams).
 constexpr int kStripMax = 384, kStripCols = (kStripMax - kGrid[0]) / 16, NLStrip = 30;
-static_assert(strip_slots(kStripMax / 32, kStripCols) <= kGrid[1] * kGrid[1], "the strip fits a hand-over block");
+constexpr int kStripSlots = strip_slots(kStripMax / 32, kStripCols);
 
 // The complex64 chain above 288 on a block of size m whose element (0, 0) sits at H
 // (leading dimension ld, per-k stride hk; read as IN says, IN = 0 or 1); outputs at the
-// block's offset of the full matrix's V (ldv, stride vk) and d, e, tau (stride dk).  The
-// strip first (its memory: the hand-over block of 256, written after it), which leaves
-// the block of 288 in V; then the chain from there.
+// block's offset of the full matrix's V (ldv, stride vk) and d, e, tau (stride dk).  work:
+// the hand-over blocks of the k-points, then their strips.
 template <int IN, typename THin>
 hipError_t strip_chain(const THin* H, int64_t hk, int m, int ld, int64_t nk, float2* V, int ldv, int64_t vk, double* dd,
                        double* de, float2* dtau, int64_t dk, float2* work, hipStream_t s) {
     if (!work || m <= kGrid[0] || m > kStripMax) return hipErrorInvalidValue;
+    constexpr int64_t bk = (int64_t)kGrid[0] * kGrid[0];
     hipLaunchKernelGGL((tridiag_strip_kernel<kStripMax / 32, kStripCols, NLStrip, IN, THin>), dim3((unsigned)nk), dim3(512),
-                       0, s, H, hk, m, ld, V, ldv, vk, dd, de, dtau, dk, work,
-                       (int64_t)strip_slots(kStripMax / 32, kStripCols));
+                       0, s, H, hk, m, ld, V, ldv, vk, dd, de, dtau, dk, work, bk, work + nk * bk, (int64_t)kStripSlots);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    const int t = tridiag_reg_split(kGrid[0]);
-    int off = m - kGrid[0];
-    float2* B = V + off + (int64_t)off * ldv;
-    grid_stage<float2, 2>(0, (const float2*)B, vk, kGrid[0], ldv, nk, B, ldv, vk, dd + off, de + off, dtau + off, dk,
-                          kGrid[0] - t, work, t, s);
-    off = m - t;
-    return c64_blocks(t, work, work + nk * (int64_t)t * t, nk, V + off + (int64_t)off * ldv, ldv, vk, dd + off, de + off,
-                      dtau + off, dk, s);
+    const int off = m - kGrid[0];
+    return c64_blocks(kGrid[0], work, bk, nk, V + off + (int64_t)off * ldv, ldv, vk, dd + off, de + off, dtau + off, dk, s);
 }
 }  // namespace
+
+size_t tridiag_reg_work_bytes(int n) {
+    // the first hand-over block (the later ones go over it) and, above 288, the strip
+    const int t = tridiag_reg_split(n);
+    return sizeof(float2) * ((size_t)t * t + (n > kGrid[0] ? kStripSlots : 0));
+}
 
 hipError_t launch_tridiag_reg_c64(const double2* dH, int n, int ld, int64_t nk, float2* Vout, double* dd, double* de,
                                   float2* dtau, float2* work, hipStream_t s) {
@@ -290,12 +277,12 @@ hipError_t launch_tridiag_reg_c64(const double2* dH, int n, int ld, int64_t nk, 
     const int t = tridiag_reg_split(n);
     if (t && !work) return hipErrorInvalidValue;
     // first grid on the matrix, then each smaller grid on the trailing block of its size
+    const int64_t bk = (int64_t)t * t;
     grid_stage<double2, 1>(grid_of(n), dH, hk, n, ld, nk, Vout, ld, hk, dd, de, dtau, n, t ? n - t : n,
-                           t ? work : (float2*)nullptr, t, s);
+                           t ? work : (float2*)nullptr, t, bk, s);
     if (!t) return hipGetLastError();
     const int off = n - t;
-    return c64_blocks(t, work, work + nk * (int64_t)t * t, nk, Vout + off + (int64_t)off * ld, ld, hk, dd + off, de + off,
-                      dtau + off, n, s);
+    return c64_blocks(t, work, bk, nk, Vout + off + (int64_t)off * ld, ld, hk, dd + off, de + off, dtau + off, n, s);
 }
 
 int tridiag_reg_c64_tail(int n) {

@@ -46,9 +46,7 @@ struct StripOrder {
 // the rank-2 update of the step before is applied on the way (to the column that the
 // next reflector needs, by itself).
 // Steps NX - n .. 16 MG - 1 run here (m < MG columns are dead at their end); the
-// updated trailing block of NX - 16 MG then goes to its place in Vout, row by row
-// (element (i, j), i >= j, at j + i ldv: above the diagonal, where no reflector is), for
-// the next grid to read there.
+// updated trailing block of NX - 16 MG then goes to Bout row by row.
 //
 // The blocked reduction streams the columns that its LDS cannot hold (0.44 MB of
 // the 0.53 at dim 362, FP32) for every step: 5 TB/s over the chip, so memory bounds
@@ -62,6 +60,7 @@ __global__ __launch_bounds__(512, 2) void tridiag_strip_kernel(const THin* Hin, 
                                                                float2* Vout, int ldv, int64_t v_kstride,
                                                                double* __restrict__ dout, double* __restrict__ eout,
                                                                float2* __restrict__ tauout, int64_t de_kstride,
+                                                               float2* __restrict__ Bout, int64_t b_kstride,
                                                                float2* __restrict__ Sout, int64_t s_kstride) {
     using S = c2<float>;
     constexpr int PR = 32, PC = 16, BS = 512, NW = BS / 64;
@@ -310,13 +309,13 @@ __global__ __launch_bounds__(512, 2) void tridiag_strip_kernel(const THin* Hin, 
         unrolled<0, MT>(trailing_update);
         __syncthreads();
     }
-    float2* B = Vk + (int64_t)(n - NT) * (ldv + 1);
+    float2* B = Bout + kk * b_kstride;
 #pragma unroll
     for (int l = 0; l < LT; ++l)
 #pragma unroll
         for (int m = 0; m <= Lay::mmax(l); ++m) {
             const int i = r + PR * l, j = c + PC * m;
-            if (i >= j) B[j + (int64_t)i * ldv] = sc_store<S>(scale(aget(Lay::idx(l, m)), Lay::straddles(l, m) ? 2.f : 1.f));
+            if (i >= j) B[j + (int64_t)i * NT] = sc_store<S>(scale(aget(Lay::idx(l, m)), Lay::straddles(l, m) ? 2.f : 1.f));
         }
 }
 

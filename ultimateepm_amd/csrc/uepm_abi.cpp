@@ -85,7 +85,7 @@ Sizes plan_sizes(const uepm_plan* p, int64_t chunk) {
         }
         if (stage_vec) {
             z.Z = sizeof(double) * (size_t)n * nbr * chunk;
-            z.W = sizeof(double) * 4 * (size_t)n * nbr * chunk;
+            z.W = sizeof(double) * uepm::tri_eig_work_doubles(n, nbr) * chunk;
         }
         z.kstat = sizeof(int) * (size_t)chunk;
         return z;
@@ -103,13 +103,12 @@ Sizes plan_sizes(const uepm_plan* p, int64_t chunk) {
         if (mixed) z.X0 = 4 * sizeof(double) * (size_t)N * m * chunk;
         if (stage_vec) {
             z.Z = sizeof(double) * (size_t)N * m * chunk;
-            z.W = sizeof(double) * 4 * (size_t)N * m * chunk;
+            z.W = sizeof(double) * uepm::tri_eig_work_doubles(N, m) * chunk;
         }
         z.kstat = sizeof(int) * (size_t)chunk;
         return z;
     }
     z.H = sizeof(double2) * (size_t)n * n * chunk;
-    z.tau = sizeof(double2) * (size_t)n * chunk;
     if (mixed) {
         z.Vf = sizeof(float2) * (size_t)n * n * chunk;
         z.tauf = sizeof(float2) * (size_t)n * chunk;
@@ -121,13 +120,14 @@ Sizes plan_sizes(const uepm_plan* p, int64_t chunk) {
         z.X0 = sizeof(double2) * (size_t)n * nbr * chunk;
     } else {
         // blocked-reduction scratch, then (after it) the FP64 register grids' hand-over blocks
+        z.tau = sizeof(double2) * (size_t)n * chunk;
         const int t = uepm::tridiag_reg_c128_tail(n);
         const size_t blocked = t < n ? sizeof(double2) * (size_t)p->tp.scratch_elems : 0;
         z.S = std::max(blocked, uepm::tridiag_reg_c128_work_bytes(t)) * chunk;
     }
     if (stage_vec) {
         z.Z = sizeof(double) * (size_t)n * nbr * chunk;
-        z.W = sizeof(double) * 4 * (size_t)n * nbr * chunk;  // two iterates, elimination states, norms (launch_tri_eig)
+        z.W = sizeof(double) * uepm::tri_eig_work_doubles(n, nbr) * chunk;
         if (!mixed) z.X = sizeof(double2) * (size_t)n * nb * chunk;
     }
     z.kstat = sizeof(int) * (size_t)chunk;
